@@ -351,6 +351,13 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 // ---------------------------------------------------------------------------------------------
 // GEMM, fast forms: exact digit planes (no reference counterpart; same bits as NearSum)
 // ---------------------------------------------------------------------------------------------
+// the empty statistics of two operands (the residue form reduces both in one block)
+static const ExpStatsSlot *stats_init() {
+	static const std::vector<ExpStatsSlot> init(
+	    2 * kStatSlots, ExpStatsSlot{ExpStatsH{0, INT32_MAX, INT32_MIN, 0, INT32_MIN, INT32_MIN, {0, 0}}});
+	return init.data();
+}
+
 struct DigitOperand {
 	void *planes = nullptr;
 	int64_t ldp = 0, pstride = 0;  // in elements
@@ -363,14 +370,13 @@ static int32_t digit_split(ozblasHandle_t *oh, int elem, int k, int cols, const 
                            int64_t ldi, DigitOperand &d) {
 	Backend *b = be(oh);
 	d.colE = (int *)walloc(oh, sizeof(int) * (size_t)cols * 2);
-	ExpStatsH *dst = (ExpStatsH *)walloc(oh, sizeof(ExpStatsH));
+	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, kStatBytes);
 	if (!d.colE || !dst) return OZBLAS_STATUS_WORKSPACE;
-	ExpStatsH init{0, INT32_MAX, INT32_MIN, 0, INT32_MIN, INT32_MIN, {0, 0}};
-	OZ_HIP(hipMemcpyAsync(dst, &init, sizeof(init), hipMemcpyHostToDevice, b->stream));
+	OZ_HIP(hipMemcpyAsync(dst, stats_init(), kStatBytes, hipMemcpyHostToDevice, b->stream));
 	launch_digit_stats(b->stream, k, cols, in, ldi, d.colE, d.colE + cols, dst);
-	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, sizeof(ExpStatsH), hipMemcpyDeviceToHost, b->stream));
+	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, kStatBytes, hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
-	std::memcpy(&d.st, b->hPinned, sizeof(ExpStatsH));
+	d.st = merge_stats((const ExpStatsSlot *)b->hPinned);
 	d.S = d.st.maxS;
 	if (elem == 1) {  // tiled INT8 layout: k padded to 128 bytes, columns to 256 (zero digits)
 		d.ldp = rup(k, 128);
@@ -586,22 +592,18 @@ static int32_t gemm_fast(ozblasHandle_t *oh, char transA, char transB, int m, in
 // ---------------------------------------------------------------------------------------------
 struct ResOperand {
 	int *colE = nullptr, *colLo = nullptr;
-	ExpStatsH *dst = nullptr;
 	ExpStatsH st{};
 	void *planes = nullptr;
 	int64_t ldp = 0, pstride = 0;
 };
 
+// dst: the operand's kStatSlots statistics slots, initialised by the caller
 static int32_t res_stats(ozblasHandle_t *oh, int k, int cols, const double *in, int64_t ldi,
-                         ResOperand &r) {
-	Backend *b = be(oh);
+                         ResOperand &r, ExpStatsSlot *dst) {
 	r.colE = (int *)walloc(oh, sizeof(int) * (size_t)cols * 3);
-	r.dst = (ExpStatsH *)walloc(oh, sizeof(ExpStatsH));
-	if (!r.colE || !r.dst) return OZBLAS_STATUS_WORKSPACE;
+	if (!r.colE) return OZBLAS_STATUS_WORKSPACE;
 	r.colLo = r.colE + 2 * (size_t)cols;
-	static const ExpStatsH init{0, INT32_MAX, INT32_MIN, 0, INT32_MIN, INT32_MIN, {0, 0}};
-	OZ_HIP(hipMemcpyAsync(r.dst, &init, sizeof(init), hipMemcpyHostToDevice, b->stream));
-	launch_digit_stats(b->stream, k, cols, in, ldi, r.colE, r.colE + cols, r.dst, r.colLo);
+	launch_digit_stats(be(oh)->stream, k, cols, in, ldi, r.colE, r.colE + cols, dst, r.colLo);
 	return OZBLAS_STATUS_SUCCESS;
 }
 
@@ -633,14 +635,15 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 		ldbi = ldk;
 	}
 	ResOperand ra, rb;
-	OZ_TRY(res_stats(oh, k, m, ain, ldai, ra));
-	OZ_TRY(res_stats(oh, k, n, bin, ldbi, rb));
-	OZ_HIP(hipMemcpyAsync(b->hPinned, ra.dst, sizeof(ExpStatsH), hipMemcpyDeviceToHost, st));
-	OZ_HIP(hipMemcpyAsync((char *)b->hPinned + sizeof(ExpStatsH), rb.dst, sizeof(ExpStatsH),
-	                      hipMemcpyDeviceToHost, st));
+	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, 2 * kStatBytes);
+	if (!dst) return OZBLAS_STATUS_WORKSPACE;
+	OZ_HIP(hipMemcpyAsync(dst, stats_init(), 2 * kStatBytes, hipMemcpyHostToDevice, st));
+	OZ_TRY(res_stats(oh, k, m, ain, ldai, ra, dst));
+	OZ_TRY(res_stats(oh, k, n, bin, ldbi, rb, dst + kStatSlots));
+	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, 2 * kStatBytes, hipMemcpyDeviceToHost, st));
 	OZ_TRY(sync(oh));  // the one host round trip: the statistics decide the number of moduli
-	std::memcpy(&ra.st, b->hPinned, sizeof(ExpStatsH));
-	std::memcpy(&rb.st, (char *)b->hPinned + sizeof(ExpStatsH), sizeof(ExpStatsH));
+	ra.st = merge_stats((const ExpStatsSlot *)b->hPinned);
+	rb.st = merge_stats((const ExpStatsSlot *)b->hPinned + kStatSlots);
 	auto give_up = [&]() {
 		wreset(oh, base);
 		return OZBLAS_STATUS_SUCCESS;

@@ -15,6 +15,12 @@
 
 namespace oz {
 
+// maximum of a level count over columns or rows into one counter: nearly all hold the value already,
+// and atomics on one address cost about 10 ns each, so only those that raise it are issued
+__device__ inline void count_max(int *zmax, int z) {
+	if (__hip_atomic_load(zmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < z) atomicMax(zmax, z);
+}
+
 // ---------------------------------------------------------------------------------------------
 // dense: one workgroup per column of a k-contiguous operand (column j = in + j*ldi, length m)
 // ---------------------------------------------------------------------------------------------
@@ -61,7 +67,7 @@ __global__ __launch_bounds__(BS) void k_split_cols(int m, int n, const TI *in, i
 		if (threadIdx.x == 0) {
 			const int z = zero ? s : cap;  // cap == "never reached zero"
 			zcol[j] = z;
-			atomicMax(zmax, z);
+			count_max(zmax, z);
 		}
 	}
 }
@@ -126,7 +132,7 @@ __global__ __launch_bounds__(BS) void k_split_cols_reg(int m, int n, const TI *i
 		if (threadIdx.x == 0) {
 			const int z = zero ? s : cap;
 			zcol[j] = z;
-			atomicMax(zmax, z);
+			count_max(zmax, z);
 		}
 	}
 }
@@ -251,7 +257,7 @@ __global__ void k_split_csr(int m, const TI *val, const int *rowptr, TI *work, d
 	for (int i = b; i < e; i++) split[(int64_t)(last + 1) * lds + i] = zero ? 0.0 : (double)work[i];
 	const int z = zero ? s : cap;
 	zrow[r] = z;
-	atomicMax(zmax, z);
+	count_max(zmax, z);
 }
 
 __global__ void k_zero_slots_csr(int m, const int *rowptr, double *split, int64_t lds,
@@ -279,7 +285,9 @@ __global__ __launch_bounds__(BS) void k_digit_stats(int m, int n, const double *
 	for (int j = blockIdx.x; j < n; j += gridDim.x)
 		digit_col_stats_acc<BS>(in + (int64_t)j * ldi, m, colE + j, colS + j, acc, red, redd,
 		                        colLo ? colLo + j : nullptr);
-	if (threadIdx.x == 0) col_acc_flush(acc, st);
+	// st: kStatSlots copies, 64 bytes apart
+	if (threadIdx.x == 0)
+		col_acc_flush(acc, (ExpStats *)((char *)st + (blockIdx.x % kStatSlots) * sizeof(ExpStatsSlot)));
 }
 
 // digit plane writer for 2-byte digits: plane s of column j at planes + s*pstride + j*ldp
