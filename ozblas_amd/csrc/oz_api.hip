@@ -162,6 +162,150 @@ static int32_t count_cols(ozblasHandle_t *oh, int k, int cols, const T *in, int6
 	return OZBLAS_STATUS_SUCCESS;
 }
 
+// slice pairs of a GEMM in the reference's level order (src/cpu/ozblas_gemm.cpp:163-164,237-264)
+static std::vector<int2> pair_list(int nA, int nB, int fastMode) {
+	int maxlevel = (nA - 1) + (nB - 1);
+	maxlevel = imax(maxlevel - fastMode, imin(nA - 1, nB - 1));
+	std::vector<int2> p;
+	for (int ik = 0; ik <= maxlevel; ik++)
+		for (int ia = 0; ia < nA; ia++)
+			if (ik - ia >= 0 && ik - ia < nB) p.push_back(make_int2(ia, ik - ia));
+	return p;
+}
+
+// ---------------------------------------------------------------------------------------------
+// GEMM, plain form with narrow slices (oz_narrow.hip): S and DS on the INT8 / FP16 matrix units, the
+// bits of gemm_plain.  *handled = false (and nothing written) when the slices are not narrow integers
+// of one unit per column and level, or when the workspace does not hold the planes: the caller goes on
+// with the FP64 products.
+//   - splitEpsMode 9 and splitShift change the units, and a reproMode = 0 remainder slot is no slice;
+//   - m = 1 or n = 1 take the DOT / GEMV orders of the sum;
+//   - infinities, NaN and sigmas beyond the type's range are reported by the split kernel, as is a
+//     |q| beyond its format;
+//   - unit exponents that would bring a product near the ends of the binary64 range (binary64 data
+//     only): there the FP64 products round, or overflow, term by term.
+// The line at k = 1024: up to there a slice has 7 bits or more and may be +128, beyond INT8.
+// ---------------------------------------------------------------------------------------------
+template <class T>
+static int32_t gemm_narrow(ozblasHandle_t *oh, int m, int n, int k, T alpha, const T *ain, int64_t ldai,
+                           const T *bin, int64_t ldbi, T beta, T *C, int ldc, int fastMode, bool *handled) {
+	Backend *b = be(oh);
+	hipStream_t st = b->stream;
+	*handled = false;
+	if ((sizeof(T) == 4) == (b->mixed != 0)) return OZBLAS_STATUS_SUCCESS;  // S and DS only
+	const int rho = Prec<T>::rho(oh, k), bits = SplitRule<T>::kPrec - rho;
+	if (oh->splitEpsMode != 0 || oh->splitShift != 1 || m < 2 || n < 2 || k > kNarrowMaxK || bits < 1 || bits > 11)
+		return OZBLAS_STATUS_SUCCESS;
+	const bool fsum = (oh->sumMode == 0);
+	const int cap = split_cap(oh);
+	if (cap < 2) return OZBLAS_STATUS_SUCCESS;
+	const int elem = bits <= 6 ? 1 : 2;
+	const uint64_t base = wmark(oh);
+	auto give_up = [&]() {
+		wreset(oh, base);
+		return OZBLAS_STATUS_SUCCESS;
+	};
+	struct Side {
+		int cols, count;
+		void *planes;
+		int64_t pstride;
+		int *ue, *z;
+	} s[2] = {{m, 0, nullptr, 0, nullptr, nullptr}, {n, 0, nullptr, 0, nullptr, nullptr}};
+	const int64_t ldp = elem == 1 ? rup(k, 128) : rup(k, 64);
+	constexpr int kStat = kNarrowSlotInts * kNarrowSlots;  // ints per operand
+	static_assert(2 * kStat * sizeof(int) <= kPinnedBytes);
+	int *stat = (int *)walloc(oh, 2 * kStat * sizeof(int));
+	if (!stat) return give_up();
+	OZ_HIP(hipMemsetAsync(stat, 0, 2 * kStat * sizeof(int), st));
+	for (int q = 0; q < 2; q++) {
+		// slots up to the cap (+ the zero slot of reproMode 0): the split stores in the pass that counts
+		s[q].pstride = ldp * (elem == 1 ? rup(s[q].cols, 256) : s[q].cols);
+		s[q].planes = walloc(oh, (uint64_t)elem * s[q].pstride * (cap + 1));
+		s[q].ue = (int *)walloc(oh, sizeof(int) * (uint64_t)s[q].cols * (cap + 1));
+		s[q].z = (int *)walloc(oh, sizeof(int) * (uint64_t)s[q].cols);
+		if (!s[q].planes || !s[q].ue || !s[q].z) return give_up();
+		launch_narrow_split(st, elem, k, s[q].cols, q ? bin : ain, q ? ldbi : ldai, s[q].planes, ldp, s[q].pstride,
+		                    rho, cap, Prec<T>::Jsplit(b), s[q].ue, s[q].z, stat + q * kStat);
+	}
+	OZ_HIP(hipMemcpyAsync(b->hPinned, stat, 2 * kStat * sizeof(int), hipMemcpyDeviceToHost, st));
+	OZ_TRY(sync(oh));
+	int lo = 0, hi = 0;
+	for (int q = 0; q < 2; q++) {
+		int st4[4] = {0, 0, 0, 0};
+		for (int c = 0; c < kNarrowSlots; c++)
+			for (int v = 0; v < 4; v++)
+				st4[v] = imax(st4[v], ((const int32_t *)b->hPinned)[q * kStat + c * kNarrowSlotInts + v]);
+		if (st4[1] || (repro_slot(oh) && st4[0] >= cap)) return give_up();
+		s[q].count = split_count(oh, st4[0]);
+		lo += kNarrowOff - st4[2];  // st4[2] = 0: an operand of zeros
+		hi += st4[3] ? st4[3] - kNarrowOff : 0;
+	}
+	if (lo < -1000 || hi > 990) return give_up();
+	const std::vector<int2> pairs = pair_list(s[0].count, s[1].count, fastMode);
+	const int np = (int)pairs.size();
+	// int32 product planes of as many pairs as fit (all of them for NearSum), at most kPlaneGroup so that
+	// a large product's planes do not take the whole workspace
+	const int64_t ldt = elem == 1 ? rup(m, 256) : rup(m, 64), tstride = ldt * (elem == 1 ? rup(n, 256) : n);
+	struct Tables {
+		LevelBin bin;
+		int2 pair;
+		int order;
+	};
+	char *tab = (char *)walloc(oh, (uint64_t)np * sizeof(Tables) + 64);
+	T *carry = (T *)walloc(oh, sizeof(T) * (uint64_t)m * n);
+	if (!tab || !carry) return give_up();
+	const uint64_t avail = b->cap - ((b->top + 255) & ~uint64_t(255));
+	int64_t group = b->cap > b->top + 256 ? (int64_t)(avail / (4ull * tstride)) : 0;
+	if (group < 1 || (!fsum && group < np)) return give_up();
+	group = std::min<int64_t>(group, np);
+	int32_t *P = (int32_t *)walloc(oh, 4ull * tstride * group);
+	if (!P) return give_up();
+	std::vector<char> host((size_t)np * sizeof(Tables) + 64);
+	LevelBin *hb = (LevelBin *)host.data();
+	int2 *hp = (int2 *)(hb + np + np % 2);
+	int *ho = (int *)(hp + np);
+	for (int p = 0; p < np; p++) {
+		hb[p] = LevelBin{0, 1, p, 0, (int)ldp};
+		hp[p] = pairs[p];
+		ho[p] = p;
+	}
+	OZ_HIP(hipMemcpyAsync(tab, host.data(), host.size(), hipMemcpyHostToDevice, st));
+	const LevelBin *dB = (const LevelBin *)tab;
+	const int2 *dP = (const int2 *)(tab + ((char *)hp - (char *)hb));
+	const int *dO = (const int *)(tab + ((char *)ho - (char *)hb));
+	for (int q = 0; q < 2; q++)
+		launch_narrow_zero(st, elem, s[q].cols, s[q].planes, ldp, s[q].pstride, s[q].ue, s[q].z, s[q].count);
+	OZ_HIP(hipEventRecord(b->ev[3], st));
+	for (int64_t p0 = 0; p0 < np; p0 += group) {
+		const int g = (int)std::min<int64_t>(group, np - p0);
+		// bin p of a group writes plane p: the group's bins and pairs start at p0, its planes at 0
+		launch_digit_gemm(st, elem, m, n, (int)ldp, s[0].planes, ldp, s[0].pstride, s[1].planes, ldp, s[1].pstride,
+		                  dP, dB + p0, g, dO, P, ldt, tstride);
+		if (p0 + g == np) OZ_HIP(hipEventRecord(b->ev[4], st));
+		if (fsum) {
+			launch_narrow_sum(st, m, n, P, ldt, tstride, dP + p0, g, s[0].ue, s[1].ue, carry, p0 == 0, p0 + g == np,
+			                  alpha, beta, C, ldc);
+		} else if constexpr (std::is_same<T, float>::value) {
+			launch_narrow_terms_f(st, m, n, P, ldt, tstride, dP, np, s[0].ue, s[1].ue);
+			launch_global_nearsum(st, m, n, np, (float *)P, tstride, ldt, C, ldc, alpha, beta, Prec<T>::Jsum(b));
+		}
+	}
+	OZ_HIP(hipEventRecord(b->ev[5], st));
+	OZ_HIP(hipGetLastError());
+	OZ_TRY(sync(oh));
+	*handled = true;
+	oh->mbk = m;
+	oh->nbk = n;
+	oh->nSplitA = (float)s[0].count;
+	oh->nSplitB = (float)s[1].count;
+	oh->nSplitC = (float)np;
+	oh->t_comp = ev_sec(b->ev[3], b->ev[4]);
+	oh->t_sum = ev_sec(b->ev[4], b->ev[5]);
+	oh->n_comp = (float)(2.0 * m * n * (double)k * oh->nSplitC);
+	wreset(oh, base);
+	return OZBLAS_STATUS_SUCCESS;
+}
+
 // ---------------------------------------------------------------------------------------------
 // GEMM, plain form (src/cpu/ozblas_gemm.cpp:3-315)
 // ---------------------------------------------------------------------------------------------
@@ -199,6 +343,13 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		ldbi = ldk;
 	}
 	const uint64_t base2 = wmark(oh);
+	bool narrow = false;
+	OZ_TRY(gemm_narrow(oh, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, fastMode, &narrow));
+	if (narrow) {
+		oh->t_total = tt.sec();
+		wreset(oh, base);
+		return OZBLAS_STATUS_SUCCESS;
+	}
 	// blocking: slice counts of the whole operands bound those of any block, so halving the
 	// larger side (as src/cpu/ozblas_gemm.cpp:91-96) until the exact need fits is safe
 	int nAf = 0, nBf = 0, zAf = -1, zBf = -1;
@@ -267,28 +418,20 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 			                   nbk == n ? zBf : -1));
 			const int nA = da.count, nB = db.count;
 			// ---- pairs (src/cpu/ozblas_gemm.cpp:163-164,237-264)
-			int maxlevel = (nA - 1) + (nB - 1);
-			maxlevel = imax(maxlevel - fastMode, imin(nA - 1, nB - 1));
+			const int maxlevel = imax((nA - 1) + (nB - 1) - fastMode, imin(nA - 1, nB - 1));
 			const bool gemvPath = !dotPath && (n == 1 && fastMode == 0);  // products at nB*ia+ib
 			const int sumorder = dotPath ? 2 : ((fastMode == 0 && nbk_ == 1) ? 3 : 1);
-			std::vector<int> pia, pib;
-			for (int ik = 0; ik <= maxlevel; ik++)
-				for (int ia = 0; ia < nA; ia++) {
-					const int ib = ik - ia;
-					if (ib < 0 || ib >= nB) continue;
-					pia.push_back(ia);
-					pib.push_back(ib);
-				}
-			const int ic = (int)pia.size();
+			const std::vector<int2> pairs = pair_list(nA, nB, fastMode);
+			const int ic = (int)pairs.size();
 			const int64_t ldcs = rup(mbk_, 8);
 			const int64_t llsc = ldcs * nbk_;
 			std::vector<int64_t> hoff(3 * (size_t)ic);
 			for (int p = 0; p < ic; p++) {
-				hoff[p] = (int64_t)pia[p] * da.sstride;
-				hoff[ic + p] = (int64_t)pib[p] * db.sstride;
+				hoff[p] = (int64_t)pairs[p].x * da.sstride;
+				hoff[ic + p] = (int64_t)pairs[p].y * db.sstride;
 				int64_t it = p;                                   // GEMM: level order (:243)
-				if (gemvPath) it = (int64_t)nB * pia[p] + pib[p];  // GEMV (:221)
-				if (dotPath) it = (int64_t)nA * pib[p] + pia[p];   // DOT: C[ia + ib*nA] (:214)
+				if (gemvPath) it = (int64_t)nB * pairs[p].x + pairs[p].y;  // GEMV (:221)
+				if (dotPath) it = (int64_t)nA * pairs[p].y + pairs[p].x;   // DOT: C[ia + ib*nA] (:214)
 				hoff[2 * ic + p] = it * llsc;
 			}
 			int64_t *dOff = (int64_t *)walloc(oh, sizeof(int64_t) * 3 * (size_t)ic);

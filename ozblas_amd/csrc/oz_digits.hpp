@@ -25,6 +25,22 @@ __device__ inline double block_max(double v, double *red) {
 	return r;
 }
 
+// the same for non-negative values (never NaN), for loops of reductions whose latency counts: the wave
+// part runs on the DPP network, and one barrier is enough because consecutive calls alternate between
+// the two halves of `red` (2 BS / 64 doubles; `par`, 0 at first, is the caller's)
+template <int BS>
+__device__ __forceinline__ double block_max_nonneg(double v, double *red, int &par) {
+	v = wave_max_nonneg_f64(v);
+	if (BS == 64) return v;
+	double *h = red + par * (BS / 64);
+	par ^= 1;
+	if (threadIdx.x % 64 == 0) h[threadIdx.x / 64] = v;
+	__syncthreads();
+	double r = h[0];
+#pragma unroll
+	for (int i = 1; i < BS / 64; i++) r = std_max(r, h[i]);
+	return r;
+}
 
 struct ExpStats {  // global reductions written by k_digit_stats
 	int maxS;        // max digit count over columns

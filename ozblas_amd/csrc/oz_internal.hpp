@@ -222,6 +222,10 @@ __host__ __device__ inline int rho_dev_f(int dim, int mode) {
 // std::max semantics (NaN never replaces the running maximum)
 __host__ __device__ inline double std_max(double a, double b) { return (a < b) ? b : a; }
 
+// running maximum of magnitudes, one instruction: a NaN x never replaces it either
+__device__ __forceinline__ double max_abs(double a, double x) { return fmax(a, fabs(x)); }
+__device__ __forceinline__ float max_abs(float a, float x) { return fmaxf(a, fabsf(x)); }
+
 __host__ __device__ inline double scalbn_clamped(double v, int64_t e) {
 	if (e > 4000) e = 4000;
 	if (e < -4000) e = -4000;

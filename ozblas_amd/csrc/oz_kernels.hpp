@@ -62,6 +62,31 @@ void launch_gemm_f64_fsum(hipStream_t st, int M, int N, int K, const double *A, 
                           const double *B, int64_t ldb, const int64_t *aOff, const int64_t *bOff,
                           int npairs, float alpha, float beta, float *C, int64_t ldc);
 
+// ---- narrow slices (oz_narrow.hip): the split into integer planes (elem 1: tiled INT8, 2: FP16, both
+// as the digit kernels read them) with the exponents of their units, the zero slices up to the operand's
+// count, and the ordered sum of the pairs' int32 products
+constexpr int kNarrowOff = 4096;   // offset that keeps the exponent maxima positive
+constexpr int kNarrowSlots = 16;   // copies of the four maxima (workgroup b reduces into b % 16),
+constexpr int kNarrowSlotInts = 16;  // a cache line each
+constexpr int kNarrowMaxK = 32768;
+void launch_narrow_split(hipStream_t st, int elem, int m, int n, const double *in, int64_t ldi, void *planes,
+                         int64_t ldp, int64_t pstride, int rho, int cap, const uint16_t *J, int *ue, int *zcol,
+                         int *stat);
+void launch_narrow_split(hipStream_t st, int elem, int m, int n, const float *in, int64_t ldi, void *planes,
+                         int64_t ldp, int64_t pstride, int rho, int cap, const uint16_t *JF, int *ue, int *zcol,
+                         int *stat);
+void launch_narrow_zero(hipStream_t st, int elem, int n, void *planes, int64_t ldp, int64_t pstride, int *ue,
+                        const int *zcol, int count);
+void launch_narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride, const int2 *pairs,
+                       int np, const int *ueA, const int *ueB, double *carry, int first, int last, double alpha,
+                       double beta, double *C, int64_t ldc);
+void launch_narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride, const int2 *pairs,
+                       int np, const int *ueA, const int *ueB, float *carry, int first, int last, float alpha,
+                       float beta, float *C, int64_t ldc);
+// the terms of every pair written over its int32 plane (the input of launch_global_nearsum)
+void launch_narrow_terms_f(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride,
+                           const int2 *pairs, int np, const int *ueA, const int *ueB);
+
 // ---- sums (oz_sum.hip)
 void launch_global_nearsum(hipStream_t st, int m, int n, int ic, double *Cs, int64_t llsc,
                            int64_t ldsc, double *C, int64_t ldc, double alpha, double beta,

@@ -31,30 +31,31 @@ __global__ __launch_bounds__(BS) void k_split_cols(int m, int n, const TI *in, i
                                                    TI *out, int64_t ldo, double *split,
                                                    int64_t lds, int64_t sstride, int rho, int shift,
                                                    int cap, const uint16_t *J, int *zcol, int *zmax) {
-	__shared__ double red[BS / 64];
+	__shared__ double red[2 * BS / 64];
+	int par = 0;
 	for (int j = blockIdx.x; j < n; j += gridDim.x) {
 		const TI *x = in + (int64_t)j * ldi;
 		TI *r = out + (int64_t)j * ldo;
 		double *sp = split + (int64_t)j * lds;
 		double mx = 0.0;  // ozblasFindMaxCKernel (src/cpu/ozblas_split.cpp:37-52)
 		for (int i = threadIdx.x; i < m; i += BS) mx = std_max(mx, fabs((double)x[i]));
-		mx = block_max<BS>(mx, red);
+		mx = block_max_nonneg<BS>(mx, red, par);
 		int s = 0;
 		bool zero = false;
 		for (s = 0; s < cap; s++) {
 			const int tau = SplitRule<TI>::tau(mx, J);
 			const TI sigma = SplitRule<TI>::sigma(rho, tau, shift);
 			const TI *src = (s == 0) ? x : r;
-			double lm = 0.0;
+			TI lm = 0;
 			for (int i = threadIdx.x; i < m; i += BS) {
 				const TI v = src[i];
 				const TI a = (v + sigma) - sigma;
 				const TI rr = v - a;
 				sp[(int64_t)s * sstride + i] = (double)a;
 				r[i] = rr;
-				lm = std_max(lm, fabs((double)rr));
+				lm = max_abs(lm, rr);
 			}
-			mx = block_max<BS>(lm, red);
+			mx = block_max_nonneg<BS>((double)lm, red, par);
 			if (mx == 0.0) {
 				zero = true;
 				break;
@@ -83,7 +84,8 @@ __global__ __launch_bounds__(BS) void k_split_cols_reg(int m, int n, const TI *i
                                                        int rho, int shift, int cap,
                                                        const uint16_t *J, int *zcol, int *zmax,
                                                        int store, int fill) {
-	__shared__ double red[BS / 64];
+	__shared__ double red[2 * BS / 64];
+	int par = 0;
 	for (int j = blockIdx.x; j < n; j += gridDim.x) {
 		const TI *x = in + (int64_t)j * ldi;
 		double *sp = split + (int64_t)j * lds;
@@ -95,13 +97,13 @@ __global__ __launch_bounds__(BS) void k_split_cols_reg(int m, int n, const TI *i
 			v[q] = (i < m) ? x[i] : (TI)0;
 			mx = std_max(mx, fabs((double)v[q]));
 		}
-		mx = block_max<BS>(mx, red);
+		mx = block_max_nonneg<BS>(mx, red, par);
 		int s = 0;
 		bool zero = false;
 		for (s = 0; s < cap; s++) {
 			const int tau = SplitRule<TI>::tau(mx, J);
 			const TI sigma = SplitRule<TI>::sigma(rho, tau, shift);
-			double lm = 0.0;
+			TI lm = 0;
 #pragma unroll
 			for (int q = 0; q < R; q++) {
 				const int i = threadIdx.x + BS * q;
@@ -110,10 +112,10 @@ __global__ __launch_bounds__(BS) void k_split_cols_reg(int m, int n, const TI *i
 					const TI rr = v[q] - a;
 					if (store) sp[(int64_t)s * sstride + i] = (double)a;
 					v[q] = rr;
-					lm = std_max(lm, fabs((double)rr));
+					lm = max_abs(lm, rr);
 				}
 			}
-			mx = block_max<BS>(lm, red);
+			mx = block_max_nonneg<BS>((double)lm, red, par);
 			if (mx == 0.0) {
 				zero = true;
 				break;
