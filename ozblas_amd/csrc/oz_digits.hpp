@@ -96,7 +96,7 @@ __device__ inline void col_acc_flush(const ColAcc &a, ExpStats *st) {
 // x = sum_{s<S} d_s 2^(E - 8(s+1)) with d_s in [-128, 127].
 template <int BS>
 __device__ inline double block_sum(double v, double *red) {
-	for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+	v = wave_sum_f64(v);
 	const int w = threadIdx.x / 64, l = threadIdx.x % 64;
 	__syncthreads();
 	if (l == 0) red[w] = v;
@@ -104,6 +104,18 @@ __device__ inline double block_sum(double v, double *red) {
 	double r = red[0];
 	for (int i = 1; i < BS / 64; i++) r += red[i];
 	return r;
+}
+
+// the maximum over the 64 lanes, in every lane (the DPP steps of wave_max_nonneg_f64; lanes a step
+// does not write keep their own value)
+__device__ __forceinline__ int wave_max_i32(int v) {
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+	return __builtin_amdgcn_readlane(v, 63);
 }
 
 // elementwise part of the column statistics: running max |x|, max of -(lowest set bit), non-finite
@@ -121,11 +133,9 @@ __device__ __forceinline__ void col_stat_elem(double v, double &mx, int &nlo, in
 // 2 BS / 64 ints, redd BS / 64 doubles); every thread gets the results
 template <int BS>
 __device__ inline void block_max3(double &mx, int &nlo, int &bad, int *red, double *redd) {
-	for (int o = 32; o > 0; o >>= 1) {
-		mx = std_max(mx, __shfl_xor(mx, o, 64));
-		nlo = max(nlo, __shfl_xor(nlo, o, 64));
-		bad = max(bad, __shfl_xor(bad, o, 64));
-	}
+	mx = wave_max_nonneg_f64(mx);
+	nlo = wave_max_i32(nlo);
+	bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0 ? 1 : 0;
 	const int w = threadIdx.x / 64, l = threadIdx.x % 64;
 	__syncthreads();
 	if (l == 0) {
@@ -226,10 +236,6 @@ __device__ inline void digit_col_stats_acc(const double *x, int m, int *colE, in
 // columns are at most a few thousand long): max, lowest set bit and the norm's sum of squares reduced
 // across the wave; lane 0 adds the column to `acc`.  The results are those of digit_col_stats_acc
 // (the sum of squares only in another order, inside the bound's rounding margin).
-__device__ inline int wave_max_i32(int v) {
-	for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-	return v;
-}
 __device__ inline void digit_col_stats_wave(const double *x, int m, int *colE, int *colS, ColAcc &acc,
                                             int *colLo) {
 	const int l = threadIdx.x % 64;
