@@ -815,6 +815,8 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 	if (nmod > kResMaxMod) return give_up();
 	const ResConst &rc = res_const_host(nmod);
 	ResConst *dRc = (ResConst *)walloc(oh, sizeof(ResConst));
+	ResTab *dTab = nullptr;
+	if (nmod <= kResTabMod && !(dTab = (ResTab *)walloc(oh, sizeof(ResTab)))) return give_up();
 	if (elem == 1) {
 		ra.ldp = rb.ldp = rup(k, 128);
 		ra.pstride = ra.ldp * rup(m, 256);
@@ -868,6 +870,7 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 	}
 	*handled = true;
 	OZ_HIP(hipMemcpyAsync(dRc, &rc, sizeof(ResConst), hipMemcpyHostToDevice, st));
+	if (dTab) OZ_HIP(hipMemcpyAsync(dTab, &res_tab_host(nmod), sizeof(ResTab), hipMemcpyHostToDevice, st));
 	OZ_HIP(hipMemcpyAsync(dPairs, pairs.data(), sizeof(int2) * pairs.size(), hipMemcpyHostToDevice, st));
 	OZ_HIP(hipMemcpyAsync(dBins, bins.data(), sizeof(LevelBin) * bins.size(), hipMemcpyHostToDevice, st));
 	OZ_HIP(hipMemcpyAsync(dOrder, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice, st));
@@ -879,7 +882,7 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 	launch_digit_gemm(st, elem, m, n, Kpad, ra.planes, ra.ldp, ra.pstride, rb.planes, rb.ldp,
 	                  rb.pstride, dPairs, dBins, nbins, dOrder, nullptr, ldt, tstride, nullptr, 0, dRc, Rp);
 	OZ_HIP(hipEventRecord(b->ev[4], st));
-	launch_res_recon(st, m, n, Rp, ldt, tstride, nchunk, dRc, nmod, rc.nl, ra.colLo, rb.colLo, alpha,
+	launch_res_recon(st, m, n, Rp, ldt, tstride, nchunk, dRc, dTab, nmod, rc.nl, ra.colLo, rb.colLo, alpha,
 	                 beta, C, ldc);
 	OZ_HIP(hipEventRecord(b->ev[5], st));
 	OZ_HIP(hipGetLastError());

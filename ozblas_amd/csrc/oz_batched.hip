@@ -74,6 +74,7 @@ struct GItem {
 struct GRec {  // Chinese-remainder reconstruction + epilogue of one problem
 	const uint8_t *R;
 	const ResConst *rc;  // constants of the problem's moduli count
+	const ResTab *tab;   // and its tables for the matrix units (null where they do not apply)
 	const int *rowLo, *colLo;
 	double *C;
 	int64_t ldt, tstride, ldc;
@@ -278,7 +279,33 @@ __global__ __launch_bounds__(256) void k_recon_grouped(const GRec *g, const int 
 	}
 }
 
+// the same on the matrix units: kRecWave (32 rows, 4 columns) items per wave
+constexpr int kRecWave = 8;
+template <int NL>
+__global__ __launch_bounds__(256) void k_recon_grouped_mfma(const GRec *g, const int *start, int n,
+                                                            const int *flag) {
+	if (*flag) return;  // C stays untouched when the plan check failed
+	__shared__ uint32_t km[kResTabMod + 1][8];
+	const int o = owner(start, n, blockIdx.x);
+	const GRec r = g[o];
+	for (int q = threadIdx.x; q < (kResTabMod + 1) * 8; q += 256) km[q / 8][q % 8] = r.tab->km[q / 8][q % 8];
+	__syncthreads();
+	ResWave ws;
+	ws.load(r.tab);
+	const double invM = r.tab->invM[NL];
+	const int rb = (r.M + 31) / 32, total = rb * ((r.N + 3) / 4);
+	const int e0 = ((int)blockIdx.x - start[o]) * 4 * kRecWave +
+	               __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+	for (int q = 0; q < kRecWave; q++) {
+		const int e = e0 + 4 * q;
+		if (e >= total) break;
+		res_recon_wave<NL>(ws, km, invM, r.M, r.N, r.R, r.ldt, r.tstride, r.nmod, r.rowLo, r.colLo, r.alpha, r.beta,
+		                   r.C, r.ldc, (e % rb) * 32, e / rb);
+	}
+}
+
 // ---- host plan -------------------------------------------------------------------------------
+constexpr int kRecClasses = 7;  // the reconstruction's kernels: NW 3, 4, 6, 9, then NL 4, 6, 8 on the matrix units
 struct BatchKey {
 	std::vector<int32_t> m, n, k, lda, ldb, ldc;
 	std::vector<char> ta, tb;
@@ -326,9 +353,9 @@ struct BatchPlan {
 	GRec *dRec = nullptr;
 	int *dRecStart = nullptr;
 	GCheck *dCheck = nullptr;
-	// the reconstruction by word count (NW 3, 4, 6, 9): the problems of class c are GRec entries
+	// the reconstruction by class: the problems of class c are GRec entries
 	// [recFirst[c], recFirst[c] + recN[c]), recBlocks[c] workgroups, block starts relative to the class
-	int recFirst[4] = {0, 0, 0, 0}, recN[4] = {0, 0, 0, 0}, recBlocks[4] = {0, 0, 0, 0};
+	int recFirst[kRecClasses] = {}, recN[kRecClasses] = {}, recBlocks[kRecClasses] = {};
 	int tcfg = 0;  // 0: 128 x 128 tiles, 1: 256 x 256 tiles
 	int grid[2] = {0, 0};
 	float tuneMs[2] = {0.f, 0.f};
@@ -388,7 +415,7 @@ static int32_t launch_execute(BatchPlan *p, hipStream_t st) {
 			                   p->dItems[1], p->nItems[1], p->dCounter, p->dFlag, p->dRcAll);
 	}
 	// one launch per word-count class: the registers of the widest class do not bound the others
-	for (int cl = 0; cl < 4; cl++) {
+	for (int cl = 0; cl < kRecClasses; cl++) {
 		if (p->recBlocks[cl] == 0) continue;
 		const GRec *g = p->dRec + p->recFirst[cl];
 		const int *gs = p->dRecStart + p->recFirst[cl];
@@ -399,8 +426,14 @@ static int32_t launch_execute(BatchPlan *p, hipStream_t st) {
 			hipLaunchKernelGGL(k_recon_grouped<4>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
 		else if (cl == 2)
 			hipLaunchKernelGGL(k_recon_grouped<6>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
-		else
+		else if (cl == 3)
 			hipLaunchKernelGGL(k_recon_grouped<9>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
+		else if (cl == 4)
+			hipLaunchKernelGGL(k_recon_grouped_mfma<4>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
+		else if (cl == 5)
+			hipLaunchKernelGGL(k_recon_grouped_mfma<6>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
+		else
+			hipLaunchKernelGGL(k_recon_grouped_mfma<8>, grid, dim3(256), 0, st, g, gs, p->recN[cl], p->dFlag);
 	}
 	OZ_HIP(hipGetLastError());
 	return OZBLAS_STATUS_SUCCESS;
@@ -640,7 +673,11 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	// constants: the full moduli table, then one per moduli count in use
 	const uint64_t rcAllOff = L2.take(sizeof(ResConst));
 	std::vector<uint64_t> rcOff(kResMaxMod + 1, 0);
-	for (int nm : usedNmod) rcOff[nm] = L2.take(sizeof(ResConst));
+	std::vector<uint64_t> tabOff(kResMaxMod + 1, 0);
+	for (int nm : usedNmod) {
+		rcOff[nm] = L2.take(sizeof(ResConst));
+		if (nm <= kResTabMod) tabOff[nm] = L2.take(sizeof(ResTab));
+	}
 	// tables
 	std::vector<GWrite> hWrite;
 	size_t writeLds = 0;
@@ -676,8 +713,11 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	const int2 *dPairs = (const int2 *)(M2 + pairsOff);
 	p->dRcAll = (const ResConst *)(M2 + rcAllOff);
 	OZ_HIP(hipMemcpyAsync(M2 + rcAllOff, &res_const_host(kResMaxMod), sizeof(ResConst), hipMemcpyHostToDevice, st));
-	for (int nm : usedNmod)
+	for (int nm : usedNmod) {
 		OZ_HIP(hipMemcpyAsync(M2 + rcOff[nm], &res_const_host(nm), sizeof(ResConst), hipMemcpyHostToDevice, st));
+		if (nm <= kResTabMod)
+			OZ_HIP(hipMemcpyAsync(M2 + tabOff[nm], &res_tab_host(nm), sizeof(ResTab), hipMemcpyHostToDevice, st));
+	}
 	int wb = 0, rb = 0;
 	for (const ProbH &h : probs) {
 		const int q = h.q;
@@ -746,8 +786,10 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 		r.N = n[q];
 		r.nmod = h.nmod;
 		r.nchunk = h.nchunk;
-		const int nw = (h.nmod > 0) ? (res_const_host(h.nmod).nl + 1) / 2 : 3;
-		recClass.push_back(nw <= 3 ? 0 : nw <= 4 ? 1 : nw <= 6 ? 2 : 3);
+		const int nl = (h.nmod > 0) ? res_const_host(h.nmod).nl : 6, nw = (nl + 1) / 2;
+		const bool tab = h.nmod > 0 && h.nmod <= kResTabMod && h.nchunk == 1;
+		r.tab = tab ? (const ResTab *)(M2 + tabOff[h.nmod]) : nullptr;
+		recClass.push_back(tab ? 2 + res_recon_words(nl) / 2 : nw <= 3 ? 0 : nw <= 4 ? 1 : nw <= 6 ? 2 : 3);
 		hRec.push_back(r);
 		GCheck ck;
 		ck.opA = 2 * q;
@@ -783,14 +825,15 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	p->dWriteStart = (int *)(M2 + writeStartOff);
 	{  // the reconstruction tables in class order, block starts relative to each class
 		std::vector<GRec> byClass;
-		for (int cl = 0; cl < 4; cl++) {
+		for (int cl = 0; cl < kRecClasses; cl++) {
 			p->recFirst[cl] = (int)byClass.size();
 			int blocks = 0;
 			for (size_t i = 0; i < hRec.size(); i++) {
 				if (recClass[i] != cl) continue;
 				recStart.push_back(blocks);
-				blocks += (int)(((int64_t)hRec[i].M * ((hRec[i].N + 3) / 4) + 256 * kRecGroups - 1) /
-				                (256 * kRecGroups));
+				const int64_t groups = (hRec[i].N + 3) / 4;
+				blocks += cl < 4 ? (int)((hRec[i].M * groups + 256 * kRecGroups - 1) / (256 * kRecGroups))
+				                 : (int)(((hRec[i].M + 31) / 32 * groups + 4 * kRecWave - 1) / (4 * kRecWave));
 				byClass.push_back(hRec[i]);
 			}
 			p->recN[cl] = (int)byClass.size() - p->recFirst[cl];

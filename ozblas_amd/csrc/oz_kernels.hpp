@@ -141,6 +141,16 @@ struct ResConst {
 	double Mpd[kResMaxMod][kResMaxChunk];
 	double Md[kResMaxChunk];
 };
+// Tables of the reconstruction on the matrix units (oz_residue.hpp res_recon_wave), for products of up
+// to kResTabMod moduli: M / p_t in balanced base-256 digits laid out as the MFMA's operand.
+constexpr int kResTabMod = 32;
+struct ResTab {
+	uint32_t w[64][4];      // lane l: digits of limb row l % 32 for the moduli 16 (l / 32) .. + 15
+	int32_t init[2][16];    // accumulator start of lane half h: the limbs of 128 sum_t M / p_t
+	uint32_t km[kResTabMod + 1][8];  // -K M modulo 2^256
+	double invM[9];         // 2^(32 (NL - 2)) / M for NL words
+};
+const ResTab &res_tab_host(int nmod);  // nmod <= kResTabMod
 // the moduli list and per-count constants (host, built once); log2 of the product of the first n
 const ResConst &res_const_host(int nmod);
 double res_log2_product(int nmod);
@@ -160,8 +170,9 @@ void launch_res_write(hipStream_t st, int elem, int m, int n, const double *in, 
                       int64_t ldp, int64_t pstride);
 // C = fma(alpha, RN(X 2^(rowLo[i] + colLo[j])), beta C), X from the residue planes (nchunk k-chunk
 // planes per modulus, summed modulo p)
+// (tab: the device copy of res_tab_host(nmod), for up to kResTabMod moduli)
 void launch_res_recon(hipStream_t st, int M, int N, const uint8_t *R, int64_t ldr, int64_t rstride,
-                      int nchunk, const ResConst *rc, int nmod, int nl, const int *rowLo,
+                      int nchunk, const ResConst *rc, const ResTab *tab, int nmod, int nl, const int *rowLo,
                       const int *colLo, double alpha, double beta, double *C, int64_t ldc);
 int digit_gemm_tile(int elem, int M, int N);
 int recon_words(int Lmax);

@@ -21,6 +21,7 @@
 // about (spanA / 8) (spanB / 8) / 2 digit-pair GEMMs of the radix-256 digit form.
 #include "oz_residue.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -156,6 +157,80 @@ static void build_res_consts() {
 	}
 }
 
+// 256-bit unsigned integers for the tables, 32-bit words, least significant first
+struct U256 {
+	uint32_t w[8] = {};
+	void add(const U256 &o) {
+		uint64_t c = 0;
+		for (int q = 0; q < 8; q++) {
+			c += (uint64_t)w[q] + o.w[q];
+			w[q] = (uint32_t)c;
+			c >>= 32;
+		}
+	}
+	void negate() {
+		uint64_t c = 1;
+		for (int q = 0; q < 8; q++) {
+			c += (uint32_t)~w[q];
+			w[q] = (uint32_t)c;
+			c >>= 32;
+		}
+	}
+	int byte(int b) const { return (int)((w[b / 4] >> (8 * (b % 4))) & 255u); }
+};
+
+static ResTab g_tab[kResTabMod + 1];
+static std::once_flag g_tab_once;
+
+// limb row rho of the digit operand holds limb 16 ((rho / 4) % 2) + 4 (rho / 8) + rho % 4, so that the
+// lane half h of the result holds the limbs 16 h .. 16 h + 15 in order (register r of lane l is row
+// 8 (r / 4) + 4 (l / 32) + r % 4)
+static void build_res_tabs() {
+	for (int nmod = 1; nmod <= kResTabMod; nmod++) {
+		const ResConst &c = res_const_host(nmod);
+		ResTab &t = g_tab[nmod];
+		std::memset(&t, 0, sizeof(t));
+		int8_t dig[kResTabMod][32] = {};
+		U256 K0;  // 128 sum_t M / p_t (below 2^5 M / 4 < 2^250)
+		for (int m = 0; m < nmod; m++) {
+			U256 W;
+			for (int q = 0; q < 8; q++) W.w[q] = c.Mp[m][q];
+			int carry = 0;
+			for (int b = 0; b < 32; b++) {  // balanced digits in [-128, 127]
+				int d = W.byte(b) + carry;
+				carry = d >= 128 ? 1 : 0;
+				dig[m][b] = (int8_t)(d - 256 * carry);
+			}
+			for (int r = 0; r < 128; r++) K0.add(W);
+		}
+		for (int l = 0; l < 64; l++) {
+			const int rho = l % 32, limb = 16 * ((rho / 4) % 2) + 4 * (rho / 8) + rho % 4;
+			for (int j = 0; j < 16; j++) {
+				const int m = 16 * (l / 32) + j;
+				const int d = m < nmod ? dig[m][limb] : 0;
+				t.w[l][j / 4] |= (uint32_t)(d & 255) << (8 * (j % 4));
+			}
+		}
+		for (int b = 0; b < 32; b++) t.init[b / 16][b % 16] = K0.byte(b);
+		U256 Mv, kM;
+		for (int q = 0; q < 8; q++) Mv.w[q] = c.M[q];
+		double Md = 0.0;
+		for (int q = 7; q >= 0; q--) Md = Md * 4294967296.0 + (double)Mv.w[q];
+		for (int K = 0; K <= kResTabMod; K++) {
+			U256 v = kM;
+			v.negate();
+			std::memcpy(t.km[K], v.w, sizeof(v.w));
+			kM.add(Mv);
+		}
+		for (int NL = 2; NL <= 8; NL++) t.invM[NL] = std::ldexp(1.0, 32 * (NL - 2)) / Md;
+	}
+}
+
+const ResTab &res_tab_host(int nmod) {
+	std::call_once(g_tab_once, build_res_tabs);
+	return g_tab[nmod < 1 ? 1 : (nmod > kResTabMod ? kResTabMod : nmod)];
+}
+
 const ResConst &res_const_host(int nmod) {
 	std::call_once(g_rc_once, build_res_consts);
 	return g_rc[nmod < 1 ? 1 : (nmod > kResMaxMod ? kResMaxMod : nmod)];
@@ -266,9 +341,47 @@ __global__ __launch_bounds__(256) void k_res_recon(int M, int N, const uint8_t *
 	}
 }
 
+// the form on the matrix units: one k chunk, up to kResTabMod moduli; a wave takes the (32 rows,
+// 4 columns) items wave, wave + waves, ..., the row blocks of a column group in turn
+template <int NL>
+__global__ __launch_bounds__(256) void k_res_recon_mfma(int M, int N, const uint8_t *__restrict__ R, int64_t ldr,
+                                                        int64_t rstride, const ResTab *__restrict__ tab, int nmod,
+                                                        const int *__restrict__ rowLo,
+                                                        const int *__restrict__ colLo, double alpha, double beta,
+                                                        double *__restrict__ C, int64_t ldc) {
+	__shared__ uint32_t km[kResTabMod + 1][8];
+	for (int q = threadIdx.x; q < (kResTabMod + 1) * 8; q += 256) km[q / 8][q % 8] = tab->km[q / 8][q % 8];
+	__syncthreads();
+	ResWave ws;
+	ws.load(tab);
+	const double invM = tab->invM[NL];
+	const int rb = (M + 31) / 32, total = rb * ((N + 3) / 4);
+	const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + threadIdx.x / 64));
+	for (int e = wave; e < total; e += (int)gridDim.x * 4)
+		res_recon_wave<NL>(ws, km, invM, M, N, R, ldr, rstride, nmod, rowLo, colLo, alpha, beta, C, ldc,
+		                   (e % rb) * 32, e / rb);
+}
+
 void launch_res_recon(hipStream_t st, int M, int N, const uint8_t *R, int64_t ldr, int64_t rstride,
-                      int nchunk, const ResConst *rc, int nmod, int nl, const int *rowLo,
+                      int nchunk, const ResConst *rc, const ResTab *tab, int nmod, int nl, const int *rowLo,
                       const int *colLo, double alpha, double beta, double *C, int64_t ldc) {
+	// (32-bit items: 2^31 of 128 outputs are beyond any memory)
+	if (tab && nchunk == 1 && nmod <= kResTabMod) {
+		const int64_t waves = ((int64_t)(M + 31) / 32) * ((N + 3) / 4);
+		const unsigned g = (unsigned)std::min<int64_t>((waves + 3) / 4, 2048);
+		const int words = res_recon_words(nl);
+#define OZ_RES_RECON(NL)                                                                               \
+	hipLaunchKernelGGL(k_res_recon_mfma<NL>, dim3(g), dim3(256), 0, st, M, N, R, ldr, rstride, tab, nmod, \
+	                   rowLo, colLo, alpha, beta, C, ldc)
+		if (words == 4)
+			OZ_RES_RECON(4);
+		else if (words == 6)
+			OZ_RES_RECON(6);
+		else
+			OZ_RES_RECON(8);
+#undef OZ_RES_RECON
+		return;
+	}
 	int64_t g = ((int64_t)M * ((N + 3) / 4) + 255) / 256;
 	if (g > 16384) g = 16384;
 	const int nw = (nl + 1) / 2;

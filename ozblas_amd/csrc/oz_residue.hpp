@@ -178,6 +178,11 @@ template <int NW>
 __device__ __forceinline__ void res_group_values(const uint8_t *Rw, int64_t rstride, int nchunk,
                                         const ResConst *rc, int nmod, const int *e0, double *t) {
 	constexpr int NC = (64 * NW + kResChunkBits - 1) / kResChunkBits;
+	if (nmod <= 0) {  // an all-zero operand: no planes
+#pragma unroll
+		for (int e = 0; e < 4; e++) t[e] = 0.0;
+		return;
+	}
 	double A[4][NC];
 	double S[4];
 #pragma unroll
@@ -303,6 +308,163 @@ __device__ __forceinline__ void res_recon_group(int M, int N, const uint8_t *R, 
 			double *c = C + (int64_t)j * ldc + i;
 			*c = fma(alpha, t[e], beta * *c);
 		}
+	}
+}
+
+// ---- the reconstruction on the matrix units ---------------------------------------------------
+// X' = sum_t c_t M/p_t is a product of the byte matrix (elements x moduli) with the digits of the
+// M/p_t, so up to 32 moduli of 32 elements are one v_mfma_i32_32x32x32_i8: limb b of element e is
+// sum_t (c_t - 128) w_tb, below 2^19, on accumulators that start at the limbs of 128 sum_t M/p_t.  A wave
+// takes 32 rows x 4 columns: lane l loads the words (row l % 32, 4 columns) of the moduli
+// 16 (l / 32) .. + 15, turns them into four MFMA operands by byte permutes, and after four MFMAs holds
+// 16 of the 32 limbs of four elements; neighbouring limbs are paired and a swap of the lane halves
+// leaves lane l with all limbs of two elements: row l % 32, columns (l / 32) * 2 and the next.
+// In scalar binary64 (res_group_values) the sums are 6 instructions per element and modulus and the
+// carry and rounding another 240: 407 VALU instructions an element at 23 moduli, which bound the kernel
+// (8192 x 8192: 0.89 ms).  Here it is memory: 0.61 ms, 4.3 TB/s of residues, C in and C out.
+
+// the instance (NL) for a product of nl words
+inline int res_recon_words(int nl) { return nl <= 4 ? 4 : nl <= 6 ? 6 : 8; }
+
+// RN(x 2^e0) for the two's-complement integer x (NL 32-bit words, least significant first).  The
+// result is never subnormal and never overflows: the fast forms are taken only when every product is a
+// multiple of 2^-1000 and below 2^1000 (fast_valid).
+template <int NL>
+__device__ __forceinline__ double res_round(uint32_t (&x)[NL], int e0) {
+	const bool neg = (int32_t)x[NL - 1] < 0;
+	const uint32_t sm = neg ? 0xffffffffu : 0u;
+	uint32_t carry = sm & 1u;
+#pragma unroll
+	for (int q = 0; q < NL; q++) {
+		const uint32_t v = x[q] ^ sm;
+		x[q] = v + carry;
+		carry = x[q] < carry ? 1u : 0u;
+	}
+	// zero words at the top move out, 4, 2 and 1 at a time
+	int sh = 0;
+#pragma unroll
+	for (int s = 4; s >= 1; s /= 2) {
+		if (s >= NL) continue;
+		uint32_t top = 0;
+#pragma unroll
+		for (int q = 0; q < s; q++) top |= x[NL - 1 - q];
+		const bool z = top == 0;
+#pragma unroll
+		for (int q = NL - 1; q >= 0; q--) x[q] = z ? (q >= s ? x[q - s] : 0u) : x[q];
+		sh += z ? 32 * s : 0;
+	}
+	// the 64 bits from the leading one, everything below folded into the last of them: the one
+	// rounding of the fma is then the rounding of x
+	const int lz = x[NL - 1] ? __builtin_clz(x[NL - 1]) : 0;
+	const uint64_t hi = (((uint64_t)x[NL - 1] << 32) | x[NL - 2]) << lz;
+	const uint64_t lo = (((uint64_t)x[NL - 2] << 32) | x[NL - 3]) << lz;
+	uint32_t rest = (uint32_t)lo;
+#pragma unroll
+	for (int q = 0; q < NL - 3; q++) rest |= x[q];
+	const uint32_t mid = (uint32_t)(lo >> 32) | (rest ? 1u : 0u);
+	const double r = fma((double)(uint32_t)(hi >> 32), 0x1p32, (double)mid);
+	const double t = ldexp(r, e0 + 32 * (NL - 2) - sh - lz);
+	return neg ? -t : t;
+}
+
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+
+// per-lane state of a wave's reconstruction: the digit operand and the accumulator start
+struct ResWave {
+	l2v w;
+	i16v init;
+	__device__ void load(const ResTab *tab) {
+		const int l = threadIdx.x % 64;
+		const u4v v = *(const u4v *)tab->w[l];
+		w = __builtin_bit_cast(l2v, v);
+#pragma unroll
+		for (int r = 0; r < 16; r++) init[r] = tab->init[l / 32][r];
+	}
+};
+
+// rows i0 .. i0 + 31 and columns 4g .. 4g + 3 of C by one wave; km: the table -K M in LDS
+template <int NL>
+__device__ __forceinline__ void res_recon_wave(const ResWave &ws, const uint32_t (*km)[8], double invM, int M,
+                                               int N, const uint8_t *R, int64_t ldr, int64_t rstride, int nmod,
+                                               const int *rowLo, const int *colLo, double alpha, double beta,
+                                               double *C, int64_t ldc, int i0, int g) {
+	const int l = threadIdx.x % 64, h = l / 32;
+	const int i = i0 + l % 32;
+	const bool row = i < M;
+	const int ic = row ? i : M - 1;
+	const uint8_t *Rw = R + res_word_offset(ic, 4 * g, ldr);
+	uint32_t w[16];
+#pragma unroll
+	for (int j = 0; j < 16; j++)  // (a word beyond the moduli meets zero digits)
+		w[j] = *(const uint32_t *)(Rw + (int64_t)min(16 * h + j, nmod - 1) * rstride);
+	double *cp[2], c0[2];
+	int e0[2];
+	bool in[2];
+	const int li = rowLo[ic];
+#pragma unroll
+	for (int c = 0; c < 2; c++) {
+		const int j = 4 * g + 2 * h + c;
+		in[c] = row && j < N;
+		const int jc = j < N ? j : N - 1;
+		cp[c] = C + (int64_t)jc * ldc + ic;
+		c0[c] = *cp[c];
+		e0[c] = li + colLo[jc];
+	}
+	u4v b[4];
+#pragma unroll
+	for (int a = 0; a < 4; a++) {
+		// 4 x 4 byte transpose of the words of moduli 4a .. 4a + 3, then c_t - 128 as int8
+		const uint32_t t0 = __builtin_amdgcn_perm(w[4 * a + 1], w[4 * a], 0x05010400);
+		const uint32_t t1 = __builtin_amdgcn_perm(w[4 * a + 1], w[4 * a], 0x07030602);
+		const uint32_t t2 = __builtin_amdgcn_perm(w[4 * a + 3], w[4 * a + 2], 0x05010400);
+		const uint32_t t3 = __builtin_amdgcn_perm(w[4 * a + 3], w[4 * a + 2], 0x07030602);
+		b[0][a] = __builtin_amdgcn_perm(t2, t0, 0x05040100) ^ 0x80808080u;
+		b[1][a] = __builtin_amdgcn_perm(t2, t0, 0x07060302) ^ 0x80808080u;
+		b[2][a] = __builtin_amdgcn_perm(t3, t1, 0x05040100) ^ 0x80808080u;
+		b[3][a] = __builtin_amdgcn_perm(t3, t1, 0x07060302) ^ 0x80808080u;
+	}
+	int32_t p[4][8];
+#pragma unroll
+	for (int c = 0; c < 4; c++) {
+		const i16v acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ws.w, __builtin_bit_cast(l2v, b[c]), ws.init, 0, 0, 0);
+#pragma unroll
+		for (int r = 0; r < 8; r++) p[c][r] = acc[2 * r] + (acc[2 * r + 1] << 8);  // below 2^28
+	}
+#pragma unroll
+	for (int c = 0; c < 2; c++) {
+		int32_t q[16];
+#pragma unroll
+		for (int r = 0; r < 8; r++) {
+			const auto s = __builtin_amdgcn_permlane32_swap((uint32_t)p[c][r], (uint32_t)p[c + 2][r], false, false);
+			q[r] = (int32_t)s[0];
+			q[8 + r] = (int32_t)s[1];
+		}
+		// carries in base 2^16, two digits a word; X' is non-negative
+		uint32_t x[NL];
+		int32_t carry = 0;
+#pragma unroll
+		for (int k = 0; k < NL; k++) {
+			const int32_t a = q[2 * k] + carry;
+			const int32_t d = q[2 * k + 1] + (a >> 16);
+			x[k] = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)a, 0x05040100);
+			carry = d >> 16;
+		}
+		// X = X' - K M, K = rint(X' / M), with X / M at most 1/4 in magnitude: the three top words give
+		// X' / M to 2^-24 for the word counts nl (ResConst) of the instance, NL - 1 and NL (M is above
+		// 2^(32 (nl - 1) - 7)); NL = 4 serves every smaller count too, with all four words
+		double f = fma((double)x[NL - 1], 0x1p32, (double)x[NL - 2]);
+		f = fma((double)x[NL - 3], 0x1p-32, f);
+		if (NL == 4) f = fma((double)x[0], 0x1p-64, f);
+		const int K = (int)rint(f * invM);
+		uint32_t cy = 0;
+#pragma unroll
+		for (int k = 0; k < NL; k++) {
+			const uint64_t v = (uint64_t)x[k] + km[K][k] + cy;
+			x[k] = (uint32_t)v;
+			cy = (uint32_t)(v >> 32);
+		}
+		const double t = res_round<NL>(x, e0[c]);
+		if (in[c]) *cp[c] = fma(alpha, t, beta * c0[c]);
 	}
 }
 
