@@ -106,18 +106,6 @@ __device__ inline double block_sum(double v, double *red) {
 	return r;
 }
 
-// the maximum over the 64 lanes, in every lane (the DPP steps of wave_max_nonneg_f64; lanes a step
-// does not write keep their own value)
-__device__ __forceinline__ int wave_max_i32(int v) {
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
-	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
-	return __builtin_amdgcn_readlane(v, 63);
-}
-
 // elementwise part of the column statistics: running max |x|, max of -(lowest set bit), non-finite
 __device__ __forceinline__ void col_stat_elem(double v, double &mx, int &nlo, int &bad) {
 	if (!isfinite(v)) {

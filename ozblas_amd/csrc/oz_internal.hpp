@@ -159,6 +159,18 @@ __device__ __forceinline__ double wave_max_nonneg_f64(double v) {
 	return lane_f64(v, 63);
 }
 
+// the maximum over the 64 lanes, in every lane (the DPP steps of wave_max_nonneg_f64; lanes a step
+// does not write keep their own value)
+__device__ __forceinline__ int wave_max_i32(int v) {
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+	v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+	return __builtin_amdgcn_readlane(v, 63);
+}
+
 // (short)ceil(log2(fabs(max))): 0 for zero, NaN and Inf (x86-64 conversion of +-inf/NaN -> 0)
 __host__ __device__ inline int tau_of(double max, const uint16_t *J) {
 	const double x = fabs(max);

@@ -514,25 +514,32 @@ __device__ inline void vs_pre_sum(const VsPre *pre, unsigned long long &maxBits,
 	}
 }
 
+// (the three counters are raised by three lanes at once: an atomic costs about a microsecond here, and
+// one thread raising them in turn was most of this function's 4 us)
 template <int BS>
 __device__ inline void vs_stats_flush(double mx, int lo, int bad, VsPre *pre) {
-	__shared__ double redd[BS / 64];
-	__shared__ int redi[BS / 64];
-	mx = block_max_d<BS>(mx, redd);
-	for (int o = 32; o > 0; o >>= 1) {
-		lo = max(lo, __shfl_xor(lo, o, 64));
-		bad = max(bad, __shfl_xor(bad, o, 64));
+	constexpr int NW = BS / 64;
+	__shared__ double redd[NW];
+	__shared__ int redi[NW], redb[NW];
+	mx = wave_max_nonneg_f64(mx);
+	lo = wave_max_i32(lo);
+	bad = __any(bad);
+	if (threadIdx.x % 64 == 0) {
+		redd[threadIdx.x / 64] = mx;
+		redi[threadIdx.x / 64] = lo;
+		redb[threadIdx.x / 64] = bad;
 	}
-	if (threadIdx.x % 64 == 0) redi[threadIdx.x / 64] = lo | (bad << 30);
 	__syncthreads();
+	VsSlot &sl = pre->slot[blockIdx.x % kVsSpread];
 	if (threadIdx.x == 0) {
-		int l = 0, bd = 0;
-		for (int w = 0; w < BS / 64; w++) {
-			l = max(l, redi[w] & ((1 << 30) - 1));
-			bd |= redi[w] >> 30;
-		}
-		VsSlot &sl = pre->slot[blockIdx.x % kVsSpread];
+		for (int w = 1; w < NW; w++) mx = std_max(mx, redd[w]);
 		if (mx > 0.0) atomic_max_lazy(&sl.maxBits, (unsigned long long)d2u(mx));
+	} else if (threadIdx.x == 64 % BS + (NW == 1 ? 1 : 0)) {
+		int l = redi[0], bd = redb[0];
+		for (int w = 1; w < NW; w++) {
+			l = max(l, redi[w]);
+			bd |= redb[w];
+		}
 		if (l > 0) atomic_max_lazy(&sl.loOff, l);
 		if (bd) atomicOr(&sl.bad, 1);
 	}
@@ -622,6 +629,18 @@ __device__ int vs_verify(unsigned long long mb, int lof, int bad, const unsigned
 	return 0;
 }
 
+// sigma = 1.5 * 2^(k + prec - 1) from its bits (integer work on the uniform k: scalar registers)
+template <class TI>
+__device__ inline TI vs_sigma(int k);
+template <>
+__device__ inline double vs_sigma<double>(int k) {
+	return __builtin_bit_cast(double, ((uint64_t)(k + 52 + 1023) << 52) | (uint64_t(1) << 51));
+}
+template <>
+__device__ inline float vs_sigma<float>(int k) {
+	return __builtin_bit_cast(float, ((uint32_t)(k + 23 + 127) << 23) | (uint32_t(1) << 22));
+}
+
 constexpr int kVsSlotWords = (int)(sizeof(VsSlot) / 8) * kVsSpread;
 
 // pre: this split's reductions; preNext: the other buffer of the pair, cleared here by workgroup 0
@@ -639,7 +658,7 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 	}
 	if (blockIdx.x == 0)
 		for (int q = threadIdx.x; q < kVsSlotWords; q += BS) ((unsigned long long *)preNext->slot)[q] = 0ull;
-	__shared__ double red[BS / 64];
+	__shared__ double red[BS / 64][kVsPred];
 	unsigned long long mb;
 	int lof, pbad;
 	vs_pre_sum<false>(pre, mb, lof, pbad);
@@ -647,32 +666,48 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 		const double M0 = __builtin_bit_cast(double, (uint64_t)mb);
 		int k0, d, L;
 		vs_predict<TI>(M0, kVsLoOff - lof, rho, cap, J, k0, d, L);
-		double Fm[kVsPred];
+		// The residues by the split's own recurrence over the predicted units (remainder after level q
+		// = cmod(x, 2^(k0 - d q)), as in VsGen): four instructions a level.  A sigma outside the normal
+		// range makes the levels from there on meaningless; the walk rejects the chain at that level.
+		TI sig[kVsPred], Fm[kVsPred];
 #pragma unroll
-		for (int q = 0; q < kVsPred; q++) Fm[q] = 0.0;
+		for (int q = 0; q < kVsPred; q++) {
+			sig[q] = vs_sigma<TI>(k0 - d * q);
+			Fm[q] = 0;
+		}
 		// four elements per thread and step, their loads in flight together
 		const int64_t stride = (int64_t)gridDim.x * BS;
 		for (int64_t i = blockIdx.x * (int64_t)BS + threadIdx.x; i < n; i += 4 * stride) {
-			double v[4];
+			TI v[4];
 #pragma unroll
 			for (int e = 0; e < 4; e++) {
 				const int64_t ie = i + e * stride;
-				const double xl = (double)x[ie < n ? ie : (int64_t)n - 1];
-				v[e] = ie < n ? xl : 0.0;
+				const TI xl = x[ie < n ? ie : (int64_t)n - 1];
+				v[e] = ie < n ? xl : (TI)0;
 			}
 #pragma unroll
-			for (int e = 0; e < 4; e++)
+			for (int q = 0; q < kVsPred; q++)
+				if (q < L) {
 #pragma unroll
-				for (int q = 0; q < kVsPred; q++)
-					if (q < L) Fm[q] = std_max(Fm[q], fabs(vs_cmod(v[e], k0 - d * q)));
+					for (int e = 0; e < 4; e++) {
+						v[e] = v[e] - ((v[e] + sig[q]) - sig[q]);
+						Fm[q] = max_abs(Fm[q], v[e]);
+					}
+				}
 		}
+		// one round for all levels: the waves' maxima through LDS, then a lane per level raises its counter
+		const int w = threadIdx.x / 64;
 #pragma unroll
-		for (int q = 0; q < kVsPred; q++) {
-			if (q < L) {  // L is uniform: every thread takes the reductions it needs
-				const double f = block_max_d<BS>(Fm[q], red);
-				if (threadIdx.x == 0 && f > 0.0)
-					atomic_max_lazy(&pre->slot[blockIdx.x % kVsSpread].F[q], (unsigned long long)d2u(f));
+		for (int q = 0; q < kVsPred; q++)
+			if (q < L) {  // L is uniform
+				const double f = wave_max_nonneg_f64((double)Fm[q]);
+				if (threadIdx.x % 64 == 0) red[w][q] = f;
 			}
+		__syncthreads();
+		if ((int)threadIdx.x < L) {
+			double f = red[0][threadIdx.x];
+			for (int u = 1; u < BS / 64; u++) f = std_max(f, red[u][threadIdx.x]);
+			if (f > 0.0) atomic_max_lazy(&pre->slot[blockIdx.x % kVsSpread].F[threadIdx.x], (unsigned long long)d2u(f));
 		}
 	}
 }
@@ -681,18 +716,6 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 // with the plan's units, sigma_s = 0.75 * 2^(rho + tau_s) = 1.5 * 2^(k_s + prec - 1), in the input's
 // precision.  Slot last + 1 holds the remainder (0 when the chain ended in zero) and later slots 0:
 // the slots k_vsplit_write stores.  Slots at or above the slice count are for the caller to mask.
-// sigma = 1.5 * 2^(k + prec - 1) from its bits (integer work on the uniform k: scalar registers)
-template <class TI>
-__device__ inline TI vs_sigma(int k);
-template <>
-__device__ inline double vs_sigma<double>(int k) {
-	return __builtin_bit_cast(double, ((uint64_t)(k + 52 + 1023) << 52) | (uint64_t(1) << 51));
-}
-template <>
-__device__ inline float vs_sigma<float>(int k) {
-	return __builtin_bit_cast(float, ((uint32_t)(k + 23 + 127) << 23) | (uint32_t(1) << 22));
-}
-
 template <class TI, int NS>
 struct VsGen {
 	TI sig[NS];
@@ -2140,6 +2163,43 @@ __device__ __forceinline__ void vs_gen_masked(const VsGen<TI, NS> &g, TI v, int 
 		if (q >= cnt) out[q] = 0.0;
 }
 
+// The sums over the 64 lanes of 64 values each (exact, so any order) to out[0, 64), by every lane of a
+// wave.  Two halving exchanges first: swapping the lane halves of values q and q + 32 and adding leaves
+// lane half h with value q + 32 h, swapping neighbouring rows of 16 lanes the same way with 16 values a
+// lane; those are summed over the rows on the DPP network.  336 instructions, against 1152 for 64 full
+// wave sums.
+__device__ __forceinline__ double swap_add32(double a, double b) {
+	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+	const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+	const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+	const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+	const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ void wave_reduce_pairs(double (&v)[64], double *out) {
+	double a[32], b[16];
+#pragma unroll
+	for (int q = 0; q < 32; q++) a[q] = swap_add32(v[q], v[q + 32]);
+#pragma unroll
+	for (int q = 0; q < 16; q++) b[q] = swap_add16(a[q], a[q + 16]);
+	const int l = threadIdx.x % 64, p0 = 16 * ((l / 16) % 2) + 32 * (l / 32);
+#pragma unroll
+	for (int q = 0; q < 16; q++) {
+		double t = b[q];
+		t += dpp_f64<0xB1>(t);   // quad_perm [1,0,3,2]
+		t += dpp_f64<0x4E>(t);   // quad_perm [2,3,0,1]
+		t += dpp_f64<0x141>(t);  // row_half_mirror
+		t += dpp_f64<0x140>(t);  // row_mirror: every lane holds its row's sum
+		if (l % 16 == 0) out[p0 + q] = t;
+	}
+}
+
 // DOT of two split vectors with device slice counts, slice counts up to NAM x NBM: each element is
 // read once (two elements per thread and step, their loads issued together), its slices generated
 // in registers from the plans, and all pair products accumulate in registers.  Each workgroup
@@ -2189,8 +2249,10 @@ __device__ __forceinline__ void dots_reg_acc(int n, const VsRef &X, const VsRef 
 			else vs_gen_masked<TI, NBM>(gy, ye[e], nB, yb);
 #pragma unroll
 			for (int a = 0; a < NAM; a++)
+				if (a < nA) {
 #pragma unroll
-				for (int b = 0; b < NBM; b++) acc[a * NBM + b] = fma(xa[a], yb[b], acc[a * NBM + b]);
+					for (int b = 0; b < NBM; b++) acc[a * NBM + b] = fma(xa[a], yb[b], acc[a * NBM + b]);
+				}
 		}
 	}
 }
@@ -2214,21 +2276,7 @@ __global__ __launch_bounds__(BS) void k_dots_reg(int n, VsRef X, VsRef Y, double
 	else if (!sx) dots_reg_acc<BS, NAM, NBM, TI, false, true>(n, X, Y, nA, nB, acc);
 	else if (!sy) dots_reg_acc<BS, NAM, NBM, TI, true, false>(n, X, Y, nA, nB, acc);
 	else dots_reg_acc<BS, NAM, NBM, TI, true, true>(n, X, Y, nA, nB, acc);
-	const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-	// wave sums on the DPP network, 16 pairs at a time (skipping the rows a >= nA; absent pairs hold
-	// zeros and are not read); lane 63 holds the sums
-	constexpr int QC = 16;
-	static_assert((NAM * NBM) % QC == 0, "pair chunks");
-#pragma unroll
-	for (int q0 = 0; q0 < NAM * NBM; q0 += QC) {
-		if (q0 / NBM >= nA) continue;
-#pragma unroll
-		for (int q = 0; q < QC; q++) acc[q0 + q] = wave_sum63_f64(acc[q0 + q]);
-		if (l == 63) {
-#pragma unroll
-			for (int q = 0; q < QC; q++) red[w][q0 + q] = acc[q0 + q];
-		}
-	}
+	wave_reduce_pairs(acc, red[threadIdx.x / 64]);
 	__syncthreads();
 	for (int q = threadIdx.x; q < NAM * NBM; q += BS) {
 		const int a = q / NBM, b = q % NBM;
