@@ -1283,8 +1283,20 @@ __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas
 				if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) t = t + term(v[ia * NBM + ib]);
 			}
 	} else {
-		// NearSum over the products (its result does not depend on the order of the terms):
-		// compact the valid ones to the front of a register array
+		// NearSum over the products (its result does not depend on the order of the terms): the
+		// clear-cut case first (binary64), largest levels first
+		if constexpr (sizeof(T) == 8) {
+			SumCert c;
+#pragma unroll
+			for (int ik = 0; ik < NAM + NBM - 1; ik++)
+#pragma unroll
+				for (int ia = 0; ia < NAM; ia++) {
+					const int ib = ik - ia;
+					if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) c.add(v[ia * NBM + ib]);
+				}
+			if (c.done(NAM * NBM, t)) return t;
+		}
+		// else compact the valid ones to the front of a register array
 		RegVec<NAM * NBM, T> u;
 		int cnt = 0;
 #pragma unroll
@@ -2412,3 +2424,10 @@ void launch_scal_axpy_dev(hipStream_t st, int n, CgDev *S, int it, const float *
 }
 
 }  // namespace oz
+
+// test hook: the clear-cut case of NearSum (1: *t is its result)
+extern "C" int32_t ozblas_internal_sum_cert(int32_t n, const double *v, double *t) {
+	oz::SumCert c;
+	for (int i = 0; i < n; i++) c.add(v[i]);
+	return c.done(n, *t) ? 1 : 0;
+}
