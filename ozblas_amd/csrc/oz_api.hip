@@ -918,26 +918,36 @@ struct VecSplit {
 	VsRef ref() const { return VsRef{x, plan, slices, lds, info}; }
 };
 
+// Opens a call's use of Backend::vz: cleared here only when the previous use did not complete.  The caller
+// flips the parities of the scratches it splits with and resets vzDirty after its last synchronisation.
+static int32_t vz_begin(ozblasHandle_t *oh) {
+	Backend *b = be(oh);
+	if (b->vzDirty) {
+		OZ_HIP(hipMemsetAsync(b->vz, 0, vz_bytes(), b->stream));
+		b->vzPar[0] = b->vzPar[1] = 0;
+	}
+	b->vzDirty = true;
+	return OZBLAS_STATUS_SUCCESS;
+}
+
 // Splits x; with readCount the slice count is read back to the host (one synchronisation),
 // otherwise it stays on the device in vs.info for kernels that read it there.  With planOnly the
 // slices are stored only for a plan outside the residue model: the consumer generates them from
 // (x, plan) (VsRef).
-// zScratch / zInfo: a zeroed scratch (vsplit_scratch_bytes()) and info (16 bytes) the caller
-// cleared together with its other buffers (one fill in place of several)
 template <class T>
 static int32_t vec_split(ozblasHandle_t *oh, int n, const T *x, VecSplit &vs, bool readCount = true,
-                         bool planOnly = false, void *zScratch = nullptr, int *zInfo = nullptr) {
+                         bool planOnly = false) {
 	Backend *b = be(oh);
 	const int cap = split_cap(oh);
 	const int rho = Prec<T>::rho(oh, n);
 	vs.x = x;
 	vs.lds = rup(n, 32);
 	vs.slices = (double *)walloc(oh, 8ull * vs.lds * (cap + 2));
-	vs.info = zInfo ? zInfo : (int *)walloc(oh, 16);
-	void *scratch = zScratch ? zScratch : walloc(oh, vsplit_scratch_bytes());
+	vs.info = (int *)walloc(oh, 16);
+	void *scratch = walloc(oh, vsplit_scratch_bytes());
 	vs.plan = (VsPlan *)walloc(oh, sizeof(VsPlan));
 	if (!vs.slices || !vs.info || !scratch || !vs.plan) return OZBLAS_STATUS_WORKSPACE;
-	if (!zScratch) OZ_HIP(hipMemsetAsync(scratch, 0, vsplit_scratch_bytes(), b->stream));
+	OZ_HIP(hipMemsetAsync(scratch, 0, vsplit_scratch_bytes(), b->stream));
 	if (planOnly)
 		OZ_HIP(launch_vsplit_plan(b->stream, n, x, vs.slices, vs.lds, rho, oh->splitShift, cap,
 		                          repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), vs.info, scratch, nullptr,
@@ -1008,48 +1018,67 @@ static int32_t dot_impl(ozblasHandle_t *oh, int n, const T *x, const T *y, T *re
 		OZ_TRY(sync(oh));
 		std::memcpy(ret, b->hPinned, sizeof(T));
 	} else {
-		// one zeroed block [scratch x | scratch y | pair sums | info x | info y | result] (one fill),
-		// the slice counts stay on the device, one launch for the pair dots and their sum, and the
-		// counts and the result come back in one copy
-		const int cap = split_cap(oh);
-		const size_t sb = (size_t)rup((int64_t)vsplit_scratch_bytes(), 256);
-		const size_t vb = (size_t)rup(8ll * (cap + 1) * (cap + 1), 256);
-		char *Z = (char *)walloc(oh, 2 * sb + vb + 48);
-		double *part = (double *)walloc(oh, dots_part_bytes());
-		if (!Z || !part) return OZBLAS_STATUS_WORKSPACE;
-		int *R = (int *)(Z + 2 * sb + vb);  // [info x (4 ints) | info y (4 ints) | result (8 bytes)]
-		T *dres = (T *)(R + 8);
-		OZ_HIP(hipMemsetAsync(Z, 0, 2 * sb + vb + 48, b->stream));
-		if (y == x) {
-			OZ_TRY(vec_split(oh, n, x, xs, false, true, Z, R));
-			ys = xs;
-		} else {  // both plans by the same three launches
+		const int cap = split_cap(oh), rho = Prec<T>::rho(oh, n), repro = repro_slot(oh) ? 0 : 1;
+		const int fsum = oh->sumMode == 0 ? 1 : 0;
+		int *out = (int *)b->hPinned;  // the kernels store the counts and the result in host memory
+		out[2] = 1;
+		if (n <= kDotSmallMax) {
+			launch_dot_small(b->stream, n, x, y, rho, oh->splitShift, cap, repro, Prec<T>::Jsplit(b),
+			                 Prec<T>::Jsum(b), fsum, out);
+			OZ_HIP(hipGetLastError());
+			OZ_TRY(sync(oh));
+		}
+		if (out[2]) {
+			// the slice counts stay on the device, one launch for the pair dots and one for their sum
+			double *part = (double *)walloc(oh, dots_part_bytes());
+			char *I = (char *)walloc(oh, 64);
+			double *vals = nullptr;
+			if (!part || !I) return OZBLAS_STATUS_WORKSPACE;
+			char *Z = b->vz;
+			if (cap < kVzSlots) {
+				vals = (double *)(Z + 2 * vz_scratch_bytes());
+			} else {  // more slices than the kept pair sums hold
+				vals = (double *)walloc(oh, 8ull * (cap + 1) * (cap + 1));
+				if (!vals) return OZBLAS_STATUS_WORKSPACE;
+				OZ_HIP(hipMemsetAsync(vals, 0, 8ull * (cap + 1) * (cap + 1), b->stream));
+			}
+			OZ_TRY(vz_begin(oh));
 			VecSplit *v[2] = {&xs, &ys};
 			const T *src[2] = {x, y};
 			double *sl[2];
 			int *inf[2];
 			void *scr[2];
 			VsPlan *pl[2];
-			for (int q = 0; q < 2; q++) {
+			const int nv = (y == x) ? 1 : 2;
+			for (int q = 0; q < nv; q++) {
 				v[q]->x = src[q];
 				v[q]->lds = rup(n, 32);
 				v[q]->slices = sl[q] = (double *)walloc(oh, 8ull * v[q]->lds * (cap + 2));
 				v[q]->plan = pl[q] = (VsPlan *)walloc(oh, sizeof(VsPlan));
-				v[q]->info = inf[q] = R + 4 * q;
-				scr[q] = Z + q * sb;
+				v[q]->info = inf[q] = (int *)(I + 32 * q);
+				scr[q] = Z + q * vz_scratch_bytes();
 				if (!sl[q] || !pl[q]) return OZBLAS_STATUS_WORKSPACE;
 			}
-			OZ_HIP(launch_vsplit_plan2(b->stream, n, x, y, Prec<T>::rho(oh, n), oh->splitShift, cap,
-			                           repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), sl, xs.lds, inf, scr, pl));
+			if (nv == 1) {
+				OZ_HIP(launch_vsplit_plan(b->stream, n, x, sl[0], xs.lds, rho, oh->splitShift, cap, repro,
+				                          Prec<T>::Jsplit(b), inf[0], scr[0], nullptr, pl[0], false, nullptr, 0, -1,
+				                          b->vzPar[0]));
+				ys = xs;
+			} else {  // both plans by the same three launches
+				OZ_HIP(launch_vsplit_plan2(b->stream, n, x, y, rho, oh->splitShift, cap, repro, Prec<T>::Jsplit(b), sl,
+				                           xs.lds, inf, scr, pl, b->vzPar));
+				b->vzPar[1] ^= 1;
+			}
+			b->vzPar[0] ^= 1;
+			launch_dots_dev(b->stream, n, xs.ref(), ys.ref(), vals, part, Prec<T>::Jsum(b), fsum, nullptr, 0, 0,
+			                out + 4, f32 ? 1 : 0, out);
+			OZ_HIP(hipGetLastError());
+			OZ_TRY(sync(oh));
+			b->vzDirty = false;
 		}
-		launch_dots_dev(b->stream, n, xs.ref(), ys.ref(), (double *)(Z + 2 * sb), part, Prec<T>::Jsum(b),
-		                oh->sumMode == 0 ? 1 : 0, nullptr, 0, 0, dres, f32 ? 1 : 0);
-		OZ_HIP(hipMemcpyAsync(b->hPinned, R, 48, hipMemcpyDeviceToHost, b->stream));
-		OZ_TRY(sync(oh));
-		const int32_t *hr = (const int32_t *)b->hPinned;
-		std::memcpy(ret, hr + 8, sizeof(T));
-		xs.count = hr[0];
-		ys.count = (y == x) ? hr[0] : hr[4];
+		std::memcpy(ret, out + 4, sizeof(T));
+		xs.count = out[0];
+		ys.count = out[1];
 	}
 	oh->nSplitA = (float)xs.count;
 	oh->nSplitB = (float)ys.count;
@@ -1289,7 +1318,8 @@ static uint64_t dot_workspace_bytes(const ozblasHandle_t *oh, int n, bool same) 
 		t = bump(t, dot2_partials_bytes(cap + 2, cap + 2));
 		return t;
 	}
-	// the zeroed block (two scratches, pair sums, counts and result), the partials, per vector
+	// counts, pair sums and the partials, then per vector (the zeroed scratch, once part of this, is the
+	// handle's own now; its bytes still count, so that the limit on n is the documented one)
 	const uint64_t sb = (uint64_t)rup((int64_t)vsplit_scratch_bytes(), 256);
 	const uint64_t vb = (uint64_t)rup(8ll * (cap + 1) * (cap + 1), 256);
 	t = bump(t, 2 * sb + vb + 48);
@@ -1428,6 +1458,38 @@ static int32_t csrmv_impl(ozblasHandle_t *oh, int m, int n, int nnz, T alpha, co
 	}
 	oh->splitShift = 1;  // the vector split always uses splitShift = 1 (counterInit)
 	VecSplit xs;
+	if constexpr (sizeof(T) == 8) {
+		// binary64: the product generates x's slices from its plan (k_csrmv_plan), no stored slices and
+		// no count read back before it; a vector of more slices than its registers hold goes on below
+		const bool fsum = oh->sumMode == 0;
+		if (oh->splitEpsMode != 2 && as.count <= 4 && !(fsum && oh->fastMode) && !(b->mixed && !fsum)) {
+			const int cap = split_cap(oh);
+			int *out = (int *)b->hPinned;
+			xs.x = x;
+			xs.lds = rup(n, 32);
+			xs.slices = (double *)walloc(oh, 8ull * xs.lds * (cap + 2));
+			xs.info = (int *)walloc(oh, 16);
+			xs.plan = (VsPlan *)walloc(oh, sizeof(VsPlan));
+			if (!xs.slices || !xs.info || !xs.plan) return OZBLAS_STATUS_WORKSPACE;
+			OZ_TRY(vz_begin(oh));
+			OZ_HIP(launch_vsplit_plan(b->stream, n, x, xs.slices, xs.lds, Prec<T>::rho(oh, n), oh->splitShift, cap,
+			                          repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), xs.info, b->vz, nullptr, xs.plan,
+			                          false, nullptr, 0, -1, b->vzPar[0]));
+			b->vzPar[0] ^= 1;
+			launch_csrmv_plan(b->stream, m, as.slices, as.lds, as.count, colind, rowptr, xs.ref(), oh->fastMode,
+			                  fsum ? 1 : 0, alpha, beta, y, Prec<T>::Jsum(b), out);
+			OZ_HIP(hipGetLastError());
+			OZ_TRY(sync(oh));
+			b->vzDirty = false;
+			if (!out[1]) {
+				oh->nSplitA = (float)as.count;
+				oh->nSplitB = (float)out[0];
+				wreset(oh, base);
+				return OZBLAS_STATUS_SUCCESS;
+			}
+			xs = VecSplit();
+		}
+	}
 	OZ_TRY(vec_split(oh, n, x, xs));
 	OZ_TRY(csrmv_core(oh, m, n, nnz, alpha, as, colind, rowptr, xs, beta, y));
 	OZ_HIP(hipGetLastError());

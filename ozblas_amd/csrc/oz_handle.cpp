@@ -10,7 +10,7 @@
 #include <mutex>
 
 #include "oz_digits.hpp"
-#include "oz_internal.hpp"
+#include "oz_kernels.hpp"
 
 namespace oz {
 
@@ -177,6 +177,7 @@ extern "C" int32_t ozblasCreate(ozblasHandle_t *oh, uint64_t workSizeBytes) {
 	                 hipMemcpyHostToDevice));
 	OZ_HIP(hipHostMalloc(&b->hPinned, kPinnedBytes, hipHostMallocDefault));
 	OZ_HIP(hipMalloc(&b->dCounters, 256 * sizeof(int32_t)));
+	OZ_HIP(hipMalloc((void **)&b->vz, vz_bytes()));
 	for (auto &e : b->ev) OZ_HIP(hipEventCreate(&e));
 	b->scratch = static_scratch(b->device);  // with the handle's device current
 	oh->backend = b;
@@ -213,6 +214,7 @@ extern "C" int32_t ozblasDestroy(ozblasHandle_t *oh) {
 	(void)hipFree(b->dTauF);
 	(void)hipFree(b->dTauF2);
 	(void)hipFree(b->dCounters);
+	(void)hipFree(b->vz);
 	(void)hipHostFree(b->hPinned);
 	delete b;
 	oh->backend = nullptr;

@@ -55,6 +55,12 @@ struct Backend {
 	uint16_t *dTauF = nullptr;   // device copies of the binary32 tables JF, JF2
 	uint16_t *dTauF2 = nullptr;
 	int mixed = 0;  // 1 while a mixed (DS: binary64 data, binary32 slices) routine runs
+	// Zeroed scratch of the vector splits and DOTs of one call: the kernels leave it zero again (the
+	// split's reductions alternate between two buffers, vzPar), so no call clears it; vzDirty while a call
+	// is under way, so that one that failed is cleared by the next.
+	char *vz = nullptr;
+	int vzPar[2] = {0, 0};
+	bool vzDirty = true;
 	char *scratch = nullptr;  // this device's copy of the static scratch array (ozblasDdotNoAlloc)
 };
 

@@ -260,6 +260,11 @@ struct VsPre {
 	VsSlot slot[kVsSpread];
 };
 size_t vsplit_scratch_bytes();
+// Backend::vz: the zeroed scratch of two vector splits, then the pair sums of a DOT with up to
+// kVzSlots slices a side
+constexpr int kVzSlots = kVsMaxLevels + 1;
+size_t vz_scratch_bytes();  // one split's part
+size_t vz_bytes();
 // Splits x into slices at stride lds (cap + 2 slots) and its plan; the count goes to info[0].
 hipError_t launch_vsplit(hipStream_t st, int n, const double *x, double *slices, int64_t lds,
                          int rho, int shift, int cap, int reproMode, const uint16_t *J, int *info,
@@ -285,13 +290,13 @@ hipError_t launch_vsplit_plan(hipStream_t st, int n, const float *x, double *sli
                               void *scratch, VsPre *pre, VsPlan *plan, bool statsDone,
                               CgDev *S = nullptr, int it = 0, int clkCat = -1, int parity = 0);
 // the plans of two vectors of one length (the DOT's x and y; each with its own slices, info,
-// zeroed scratch and plan), by the same three launches
+// zeroed scratch and plan), by the same three launches; parity as in launch_vsplit_plan, per scratch
 hipError_t launch_vsplit_plan2(hipStream_t st, int n, const double *x, const double *y, int rho, int shift,
                                int cap, int reproMode, const uint16_t *J, double *const slices[2], int64_t lds,
-                               int *const info[2], void *const scratch[2], VsPlan *const plan[2]);
+                               int *const info[2], void *const scratch[2], VsPlan *const plan[2], int parity[2]);
 hipError_t launch_vsplit_plan2(hipStream_t st, int n, const float *x, const float *y, int rho, int shift,
                                int cap, int reproMode, const uint16_t *JF, double *const slices[2], int64_t lds,
-                               int *const info[2], void *const scratch[2], VsPlan *const plan[2]);
+                               int *const info[2], void *const scratch[2], VsPlan *const plan[2], int parity[2]);
 void launch_axpy_host(hipStream_t st, int n, double alpha, const double *x, double *y, int fused);
 void launch_axpy_host(hipStream_t st, int n, float alpha, const float *x, float *y, int fused);
 // t = b - A x by the reference's plain CSRMV (the CG's true residual)
@@ -338,6 +343,12 @@ struct VsRef {
 void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA,
                           const int *colind, const int *rowptr, VsRef X, int fsum, double *y,
                           double *Cs, int64_t ldc, const uint16_t *J, CgDev *S, int it, VsPre *preY);
+// y = alpha A x + beta y with x's plan (binary64; slices of A pre-split, nA <= 4): more than
+// kCsrPlanSlices slices of x leave y untouched; out (host memory): x's count, then 1 in that case
+constexpr int kCsrPlanSlices = 8;
+void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
+                       const int *rowptr, VsRef X, int fastMode, int fsum, double alpha, double beta, double *y,
+                       const uint16_t *J, int *out);
 // binary32 p and q (JF2: the binary32 NearSum table); p's slices capped at 8 by maxVecSlices;
 // mixed = 1: binary64 pair chains (<float,double>)
 void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA,
@@ -346,9 +357,19 @@ void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas,
                           int mixed = 0);
 // part: dots_part_bytes() of scratch for the per-workgroup pair partials (no initial value)
 size_t dots_part_bytes();
-// DOT of two split vectors (binary32 inputs with f32), completed by `mode` (0: C[0] = the DOT)
+// DOT of two split vectors (binary32 inputs with f32), completed by `mode` (0: C[0] = the DOT, and the
+// slice counts to counts[0] and counts[1]; both may be host memory)
 void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, double *part,
-                     const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32 = 0);
+                     const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32 = 0,
+                     int *counts = nullptr);
+// The whole DOT of two vectors of n <= kDotSmallMax elements in one workgroup.  out (host memory): the slice
+// counts of x and y in out[0] and out[1], out[2] = 1 when the general path has to run instead (a
+// non-finite value or more than 8 slices), the DOT at out + 4.
+constexpr int kDotSmallMax = 8192;
+void launch_dot_small(hipStream_t st, int n, const double *x, const double *y, int rho, int shift, int cap,
+                      int reproMode, const uint16_t *Js, const uint16_t *Jn, int fsum, int *out);
+void launch_dot_small(hipStream_t st, int n, const float *x, const float *y, int rho, int shift, int cap,
+                      int reproMode, const uint16_t *JF, const uint16_t *JF2, int fsum, int *out);
 // x += alpha p, r -= alpha q (reductions of r's split into preR); p = r + beta p (into preP)
 void launch_axpy2_dev(hipStream_t st, int n, CgDev *S, int it, const double *P, double *X,
                       const double *Q, double *R, VsPre *preR);

@@ -833,19 +833,23 @@ __global__ __launch_bounds__(256) void k_vsplit_write(int n, const TI *x, double
 
 size_t vsplit_scratch_bytes() { return 8ull * kVsK + 8ull * kVsBlocks + 64 + 2 * sizeof(VsPre) + 64; }
 
+size_t vz_scratch_bytes() { return (vsplit_scratch_bytes() + 255) & ~size_t(255); }
+size_t vz_bytes() { return 2 * vz_scratch_bytes() + 8ull * kVzSlots * kVzSlots; }
+
 // The plan of x (length n): the predicted chain, then the table scan and walk only when it does not
 // hold; with fallback the walk's workgroup also stores the slices of a plan marked bad (the
 // reference loop).  scratch: vsplit_scratch_bytes(), zeroed once (the kernels leave it zero again).
 // the pointers of a vector's split in its scratch (Fg, range, the done counter, the VsPre pair)
 template <class TI>
-static VsSecond<TI> vs_second(const TI *x, void *scratch, VsPlan *plan, int *info, double *slices) {
+static VsSecond<TI> vs_second(const TI *x, void *scratch, VsPlan *plan, int *info, double *slices, int parity) {
 	VsSecond<TI> v{};
 	v.x = x;
 	v.Fg = (unsigned long long *)scratch;
 	v.range = (int2 *)(v.Fg + kVsK);
 	v.done = (unsigned int *)(v.range + kVsBlocks);
-	v.pre = (VsPre *)((char *)scratch + 8ull * kVsK + 8ull * kVsBlocks + 64);
-	v.preNext = v.pre + 1;
+	VsPre *pre = (VsPre *)((char *)scratch + 8ull * kVsK + 8ull * kVsBlocks + 64);
+	v.pre = pre + (parity & 1);
+	v.preNext = pre + ((parity & 1) ^ 1);
 	v.plan = plan;
 	v.info = info;
 	v.slices = slices;
@@ -917,22 +921,22 @@ hipError_t launch_vsplit(hipStream_t st, int n, const float *x, double *slices, 
 template <class TI>
 static hipError_t vsplit_plan2(hipStream_t st, int n, const TI *x, const TI *y, int rho, int shift, int cap,
                                int reproMode, const uint16_t *J, double *const slices[2], int64_t lds,
-                               int *const info[2], void *const scratch[2], VsPlan *const plan[2]) {
-	const VsSecond<TI> v2 = vs_second<TI>(y, scratch[1], plan[1], info[1], slices[1]);
+                               int *const info[2], void *const scratch[2], VsPlan *const plan[2], int parity[2]) {
+	const VsSecond<TI> v2 = vs_second<TI>(y, scratch[1], plan[1], info[1], slices[1], parity[1]);
 	return vsplit_plan(st, n, x, slices[0], lds, rho, shift, cap, reproMode, J, info[0], scratch[0], nullptr,
-	                   plan[0], false, nullptr, 0, kClkNone, 1, 0, &v2);
+	                   plan[0], false, nullptr, 0, kClkNone, 1, parity[0], &v2);
 }
 
 hipError_t launch_vsplit_plan2(hipStream_t st, int n, const double *x, const double *y, int rho, int shift,
                                int cap, int reproMode, const uint16_t *J, double *const slices[2], int64_t lds,
-                               int *const info[2], void *const scratch[2], VsPlan *const plan[2]) {
-	return vsplit_plan2(st, n, x, y, rho, shift, cap, reproMode, J, slices, lds, info, scratch, plan);
+                               int *const info[2], void *const scratch[2], VsPlan *const plan[2], int parity[2]) {
+	return vsplit_plan2(st, n, x, y, rho, shift, cap, reproMode, J, slices, lds, info, scratch, plan, parity);
 }
 
 hipError_t launch_vsplit_plan2(hipStream_t st, int n, const float *x, const float *y, int rho, int shift,
                                int cap, int reproMode, const uint16_t *JF, double *const slices[2], int64_t lds,
-                               int *const info[2], void *const scratch[2], VsPlan *const plan[2]) {
-	return vsplit_plan2(st, n, x, y, rho, shift, cap, reproMode, JF, slices, lds, info, scratch, plan);
+                               int *const info[2], void *const scratch[2], VsPlan *const plan[2], int parity[2]) {
+	return vsplit_plan2(st, n, x, y, rho, shift, cap, reproMode, JF, slices, lds, info, scratch, plan, parity);
 }
 
 hipError_t launch_vsplit_plan(hipStream_t st, int n, const double *x, double *slices, int64_t lds,
@@ -1190,6 +1194,67 @@ void launch_nearsum_small(hipStream_t st, int nvals, double *vals, double alpha,
 	                   maxlevel, fsum, J);
 }
 
+// the sum over a row's pair products (NearSum, or Fsum in level order) with ia + ib <= maxlevel
+template <int NAM, int NBM, class T, class V>
+__device__ __forceinline__ T csr_pairs_sum(RegVec<NAM * NBM, V> &v, int nA, int nB, int maxlevel, int fsum,
+                                           const uint16_t *J) {
+	// a pair sum as a term of the sum in T (the binary64 chain of <float,double> rounds as the
+	// reference's (float) of the scaled product)
+	auto term = [](V p) -> T {
+		if constexpr (sizeof(V) == sizeof(T))
+			return p;
+		else
+			return sum_term<T>(p);
+	};
+	T t;
+	if (fsum) {
+		t = (T)0;
+#pragma unroll
+		for (int ik = 0; ik < NAM + NBM - 1; ik++)
+#pragma unroll
+			for (int ia = 0; ia < NAM; ia++) {
+				const int ib = ik - ia;
+				if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) t = t + term(v[ia * NBM + ib]);
+			}
+	} else {
+		// NearSum over the products (its result does not depend on the order of the terms): the
+		// clear-cut case first (binary64), largest levels first
+		if constexpr (sizeof(T) == 8) {
+			SumCert c;
+#pragma unroll
+			for (int ik = 0; ik < NAM + NBM - 1; ik++)
+#pragma unroll
+				for (int ia = 0; ia < NAM; ia++) {
+					const int ib = ik - ia;
+					if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) c.add(v[ia * NBM + ib]);
+				}
+			if (c.done(NAM * NBM, t)) return t;
+		}
+		// else compact the valid ones to the front of a register array
+		RegVec<NAM * NBM, T> u;
+		int cnt = 0;
+#pragma unroll
+		for (int ia = 0; ia < NAM; ia++)
+#pragma unroll
+			for (int ib = 0; ib < NBM; ib++) u[ia * NBM + ib] = (T)0;
+#pragma unroll
+		for (int ia = 0; ia < NAM; ia++)
+#pragma unroll
+			for (int ib = 0; ib < NBM; ib++) {
+				const bool ok = ia < nA && ib < nB && ia + ib <= maxlevel;
+#pragma unroll
+				for (int q = 0; q < NAM * NBM; q++)
+					if (ok && q == cnt) u[q] = term(v[ia * NBM + ib]);
+				cnt += ok ? 1 : 0;
+			}
+		if constexpr (sizeof(T) == 4)
+			t = nearsum_f(cnt, u, J);
+		else
+			t = nearsum(cnt, u, J);
+	}
+	return t;
+}
+
 // ---------------------------------------------------------------------------------------------
 // CSR slice products + global sum fused per row (ozblasRcsrmv, src/cpu/ozblas_csrmv.cpp:113-166):
 // v[ia][ib] = sum_j As_ia[j] * Xs_ib[col_j] (fma in row order as csrmm_n, exact), then NearSum
@@ -1264,61 +1329,140 @@ __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas
 					v[ia * NBM + ib] = (V)fma(a[q][ia], x[q][ib], (double)v[ia * NBM + ib]);
 		}
 	}
-	// a pair sum as a term of the sum in T (the binary64 chain of <float,double> rounds as the
-	// reference's (float) of the scaled product)
-	auto term = [](V p) -> T {
-		if constexpr (sizeof(V) == sizeof(T))
-			return p;
-		else
-			return sum_term<T>(p);
-	};
-	T t;
-	if (fsum) {
-		t = (T)0;
+	return csr_pairs_sum<NAM, NBM, T, V>(v, nA, nB, maxlevel, fsum, J);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The binary64 product with a row block staged in LDS: 256 consecutive rows of one workgroup own one
+// contiguous range of nonzeros, which all threads load in order -- the slices of A, the column index, and
+// with it the element of x -- into LDS; a thread then walks its row there, generating the slices of x
+// from the plan.  Read row by row from memory, neighbouring lanes are a row apart (7 nonzeros of a
+// stencil), so every cache line was fetched by seven instructions, and each row's chain of column index
+// and gather was a memory latency of its own: 59 us for the 100^3 Laplacian with 2 slices of A and 4 of x
+// at 426 VALU instructions a wave.  A block with more nonzeros than the stage holds takes the row walk
+// in memory.  Workgroups of one XCD (consecutive ones go to the 8 XCDs in turn) take one contiguous
+// eighth of the rows, so that an L2 holds the part of x its rows gather.
+// ---------------------------------------------------------------------------------------------
+constexpr int kCsrRows = 256;
+template <int NAM>
+struct CsrStage {
+	static constexpr int kCap = NAM <= 2 ? 2048 : 1280;  // nonzeros: 48 KB and 50 KB, three workgroups a CU
+	double a[NAM][kCap];
+	double x[kCap];
+};
+
+__device__ inline int csr_block(int nb) {
+	const int chunk = (nb + 7) / 8;
+	return ((int)blockIdx.x % 8) * chunk + (int)blockIdx.x / 8;  // may be nb or more (grid 8 chunk)
+}
+
+// loads the block's nonzeros [base, base + cnt) when they fit; false (uniform) otherwise
+template <int NAM>
+__device__ __forceinline__ bool csr_stage_load(CsrStage<NAM> &st, int base, int cnt, const double *As,
+                                               int64_t ldas, int nA, const int *colind, const double *X) {
+	if (cnt > CsrStage<NAM>::kCap) return false;
+	constexpr int U = 4;
+	for (int i0 = threadIdx.x; i0 < cnt; i0 += U * kCsrRows) {
+		int c[U];
+		double a[U][NAM], x[U];
 #pragma unroll
-		for (int ik = 0; ik < NAM + NBM - 1; ik++)
+		for (int u = 0; u < U; u++) {  // unconditional loads at clamped indices, all in flight
+			const int i = base + min(i0 + u * kCsrRows, cnt - 1);
+			c[u] = colind[i];
 #pragma unroll
-			for (int ia = 0; ia < NAM; ia++) {
-				const int ib = ik - ia;
-				if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) t = t + term(v[ia * NBM + ib]);
-			}
-	} else {
-		// NearSum over the products (its result does not depend on the order of the terms): the
-		// clear-cut case first (binary64), largest levels first
-		if constexpr (sizeof(T) == 8) {
-			SumCert c;
-#pragma unroll
-			for (int ik = 0; ik < NAM + NBM - 1; ik++)
-#pragma unroll
-				for (int ia = 0; ia < NAM; ia++) {
-					const int ib = ik - ia;
-					if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) c.add(v[ia * NBM + ib]);
-				}
-			if (c.done(NAM * NBM, t)) return t;
+			for (int q = 0; q < NAM; q++) a[u][q] = As[(int64_t)min(q, nA - 1) * ldas + i];
 		}
-		// else compact the valid ones to the front of a register array
-		RegVec<NAM * NBM, T> u;
-		int cnt = 0;
 #pragma unroll
-		for (int ia = 0; ia < NAM; ia++)
+		for (int u = 0; u < U; u++) x[u] = X[c[u]];
 #pragma unroll
-			for (int ib = 0; ib < NBM; ib++) u[ia * NBM + ib] = (T)0;
+		for (int u = 0; u < U; u++) {
+			const int i = i0 + u * kCsrRows;
+			if (i < cnt) {
 #pragma unroll
-		for (int ia = 0; ia < NAM; ia++)
-#pragma unroll
-			for (int ib = 0; ib < NBM; ib++) {
-				const bool ok = ia < nA && ib < nB && ia + ib <= maxlevel;
-#pragma unroll
-				for (int q = 0; q < NAM * NBM; q++)
-					if (ok && q == cnt) u[q] = term(v[ia * NBM + ib]);
-				cnt += ok ? 1 : 0;
+				for (int q = 0; q < NAM; q++) st.a[q][i] = q < nA ? a[u][q] : 0.0;
+				st.x[i] = x[u];
 			}
-		if constexpr (sizeof(T) == 4)
-			t = nearsum_f(cnt, u, J);
-		else
-			t = nearsum(cnt, u, J);
+		}
 	}
-	return t;
+	__syncthreads();
+	return true;
+}
+
+// the row with staged nonzeros [b, e): nA x nB pair sums in row order, then their sum
+template <int NAM, int NBM>
+__device__ __forceinline__ double csr_stage_row(const CsrStage<NAM> &st, int b, int e, int nA, int nB, int maxlevel,
+                                                int fsum, const uint16_t *J, const VsPlan *plan) {
+	double sig[NBM];
+	const int last = plan->last;
+#pragma unroll
+	for (int q = 0; q < NBM; q++) sig[q] = (q <= last) ? vs_sigma<double>(plan->k[q]) : 0.0;
+	RegVec<NAM * NBM, double> v;
+#pragma unroll
+	for (int q = 0; q < NAM * NBM; q++) v[q] = 0.0;
+	for (int j = b; j < e; j++) {
+		double r = st.x[j], a[NAM];
+#pragma unroll
+		for (int ia = 0; ia < NAM; ia++) a[ia] = st.a[ia][j];
+#pragma unroll
+		for (int ib = 0; ib < NBM; ib++)
+			if (ib < nB) {  // uniform
+				const double x = (r + sig[ib]) - sig[ib];  // VsGen's step
+				r = r - x;
+#pragma unroll
+				for (int ia = 0; ia < NAM; ia++) v[ia * NBM + ib] = fma(a[ia], x, v[ia * NBM + ib]);
+			}
+	}
+	return csr_pairs_sum<NAM, NBM, double, double>(v, nA, nB, maxlevel, fsum, J);
+}
+
+// y = alpha A x + beta y from the slices of A and x's plan (ozblasRcsrmv).  out (host memory): x's slice
+// count, and 1 in out[1] when it exceeds the register bound NBM -- then y is untouched and the caller
+// takes the stored slices.
+template <int NAM, int NBM>
+__global__ __launch_bounds__(kCsrRows) void k_csrmv_plan(int m, const double *As, int64_t ldas, int nA,
+                                                        const int *colind, const int *rowptr, VsRef X,
+                                                        int fastMode, int fsum, double alpha, double beta,
+                                                        double *y, const uint16_t *J, int *out) {
+	const int nB = X.info[0];
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		out[0] = nB;
+		out[1] = nB > NBM ? 1 : 0;
+	}
+	if (nB > NBM) return;
+	__shared__ CsrStage<NAM> st;
+	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
+	if (r0 >= m) return;
+	const int rows = min(kCsrRows, m - r0);
+	const int base = rowptr[r0], cnt = rowptr[r0 + rows] - base;
+	const int maxlevel = max((nA - 1) + (nB - 1) - fastMode, min(nA - 1, nB - 1));
+	const bool staged = !X.plan->bad && csr_stage_load<NAM>(st, base, cnt, As, ldas, nA, colind, (const double *)X.x);
+	const int r = r0 + (int)threadIdx.x;
+	if (r >= m) return;
+	double t;
+	if (staged) {
+		t = csr_stage_row<NAM, NBM>(st, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J, X.plan);
+	} else if (X.plan->bad) {
+		t = csrmm_row_sum<NAM, NBM>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel, fsum, J);
+	} else {
+		VsGen<double, NBM> g;
+		g.init(X.plan);
+		t = csrmm_row_sum<NAM, NBM, double, double, true>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel,
+		                                                  fsum, J, (const double *)X.x, &g);
+	}
+	y[r] = fma(alpha, t, beta * y[r]);
+}
+
+void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
+                       const int *rowptr, VsRef X, int fastMode, int fsum, double alpha, double beta, double *y,
+                       const uint16_t *J, int *out) {
+	const int nb = (m + kCsrRows - 1) / kCsrRows;
+	const dim3 g(8 * ((nb + 7) / 8));
+	if (nA <= 2)
+		hipLaunchKernelGGL((k_csrmv_plan<2, kCsrPlanSlices>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr,
+		                   X, fastMode, fsum, alpha, beta, y, J, out);
+	else
+		hipLaunchKernelGGL((k_csrmv_plan<4, kCsrPlanSlices>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr,
+		                   X, fastMode, fsum, alpha, beta, y, J, out);
 }
 
 template <int NAM, int NBM, class T, class V = T>
@@ -1940,13 +2084,30 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 		}
 		return;
 	}
-	const int r = blockIdx.x * blockDim.x + threadIdx.x;
 	double mx = 0.0;
 	int lo = 0, bad = 0;
+	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
+	const int r = r0 + (int)threadIdx.x;
+	// binary64 with a plan: the staged rows (csr_stage_row); uniform over the workgroup
+	constexpr bool kStage = sizeof(T) == 8;
+	int base = 0;
+	bool staged = false;
+	__shared__ typename std::conditional<kStage, CsrStage<NAM>, int>::type stage;
+	if constexpr (kStage) {
+		if (r0 < m && nB <= NBM && !X.plan->bad) {
+			const int rows = min(kCsrRows, m - r0);
+			base = rowptr[r0];
+			staged = csr_stage_load<NAM>(stage, base, rowptr[r0 + rows] - base, As, ldas, nA, colind, (const double *)X.x);
+		}
+	}
 	if (r < m) {
 		const int maxlevel = (nA - 1) + (nB - 1);
 		T t = 0;
-		if (nB > NBM) {
+		if (staged) {
+			if constexpr (kStage)
+				t = csr_stage_row<NAM, NBM>(stage, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J,
+				                            X.plan);
+		} else if (nB > NBM) {
 			if constexpr (sizeof(T) == 8) t = csrmm_big_row(r, As, ldas, nA, colind, rowptr, X, nB, fsum, Cs, ldc, J);
 		} else if (X.plan->bad) {
 			t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB,
@@ -1966,7 +2127,7 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 
 // Completion of a device DOT in one workgroup, after the product kernel: sums the nA x nB pair
 // dots (sumOrder 2) and applies `mode`
-//   0: C[0] = fma(1, t, 0 * C[0])                        (ozblasRdot's GEMM epilogue)
+//   0: C[0] = fma(1, t, 0 * 0)                           (ozblasRdot's GEMM epilogue, C = +0 before)
 //   1: tmp = t, alpha = dold / tmp                       (src/cpu/ozblas_cg.cpp:83-84)
 //   2: dnew = t, resi = sqrt(dnew), beta = dnew / dold,  (src/cpu/ozblas_cg.cpp:91-94,100-112)
 //      dold = dnew, history and the residual test
@@ -1978,7 +2139,7 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 // the sums dots_general accumulated in vals.
 template <int BS>
 __device__ void dots_finish(int nA, int nB, double *vals, const double *part, int nwg, const uint16_t *J,
-                            int fsum, CgDev *S, int it, int mode, void *C, int f32) {
+                            int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
 	static_assert(kDotMaxWG <= 2 * BS, "two partials per thread and pair");
 	__shared__ double psum[kDotPairs];
 	__shared__ double red[BS / 64][16];
@@ -2054,12 +2215,15 @@ __device__ void dots_finish(int nA, int nB, double *vals, const double *part, in
 		}
 	}
 	if (threadIdx.x != 0) return;
+	if (counts) {
+		counts[0] = nA;
+		counts[1] = nB;
+	}
 	if (f32) {
 		float *fv = vals_to_float(npairs, src);
 		const float t = dot_pairs_sum_f(npairs, fv, nA, nB, maxlevel, fsum, J);
 		if (mode == 0) {
-			float *Cf = (float *)C;
-			Cf[0] = fma1_f(1.f, t, 0.f * Cf[0]);
+			*(float *)C = fma1_f(1.f, t, 0.f * 0.f);
 		} else {
 			// the <float,float> CG's recurrences in binary32 (the CgDev fields hold binary32 values)
 			const float r = fma1_f(1.f, t, 0.f * 0.f);
@@ -2090,8 +2254,7 @@ __device__ void dots_finish(int nA, int nB, double *vals, const double *part, in
 	const double t = waveDone ? tw : dot_pairs_sum(npairs, src, nA, nB, maxlevel, fsum, J);
 	const double r = fma(1.0, t, 0.0 * 0.0);
 	if (mode == 0) {
-		double *Cd = (double *)C;
-		Cd[0] = fma(1.0, t, 0.0 * Cd[0]);
+		*(double *)C = r;
 	} else if (mode == 1) {
 		S->tmp = r;
 		S->alpha = S->dold / r;
@@ -2305,11 +2468,12 @@ __global__ __launch_bounds__(BS) void k_dots_reg(int n, VsRef X, VsRef Y, double
 template <int BS, int NAM, int NBM>
 __global__ __launch_bounds__(BS) void k_dots_fin(int nwg, const int *infoX, const int *infoY,
                                                  double *vals, const double *part, const uint16_t *J,
-                                                 int fsum, CgDev *S, int it, int mode, void *C, int f32) {
+                                                 int fsum, CgDev *S, int it, int mode, void *C, int f32,
+                                                 int *counts) {
 	if (cg_skip(S, it)) return;
 	const int nA = infoX[0], nB = infoY[0];
 	const bool reg = nA <= NAM && nB <= NBM;
-	dots_finish<BS>(nA, nB, vals, reg ? part : nullptr, nwg, J, fsum, S, it, mode, C, f32);
+	dots_finish<BS>(nA, nB, vals, reg ? part : nullptr, nwg, J, fsum, S, it, mode, C, f32, counts);
 }
 
 // x = fma(alpha, p, x); r = fma(-alpha, q, r)   (src/cpu/ozblas_cg.cpp:87-88, ozblas_axpy.cpp),
@@ -2355,11 +2519,12 @@ static void csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas,
                           const int *rowptr, VsRef X, int fsum, T *y, double *Cs, int64_t ldc, const uint16_t *J,
                           CgDev *S, int it, VsPre *preY) {
 	constexpr int kNbReg = 8;
+	const dim3 g(8 * (((m + kCsrRows - 1) / kCsrRows + 7) / 8));  // csr_block
 	if (nA <= 2)  // the matrix's count is known here; p's count only on the device
-		hipLaunchKernelGGL((k_csrmm_sum_dev<2, kNbReg, T, V>), dim3((m + 255) / 256), dim3(256), 0, st, m, As,
+		hipLaunchKernelGGL((k_csrmm_sum_dev<2, kNbReg, T, V>), g, dim3(kCsrRows), 0, st, m, As,
 		                   ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, J, S, it, preY);
 	else
-		hipLaunchKernelGGL((k_csrmm_sum_dev<4, kNbReg, T, V>), dim3((m + 255) / 256), dim3(256), 0, st, m, As,
+		hipLaunchKernelGGL((k_csrmm_sum_dev<4, kNbReg, T, V>), g, dim3(kCsrRows), 0, st, m, As,
 		                   ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, J, S, it, preY);
 }
 
@@ -2382,7 +2547,7 @@ void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas,
 size_t dots_part_bytes() { return sizeof(double) * kDotPairs * kDotMaxWG; }
 
 void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, double *part,
-                     const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32) {
+                     const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
 	constexpr int kRA = 8, kRB = 8;
 	int gx = (n + 1023) / 1024;  // four elements per thread and step
 	if (gx > kDotMaxWG) gx = kDotMaxWG;
@@ -2394,7 +2559,167 @@ void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, doub
 		hipLaunchKernelGGL((k_dots_reg<256, kRA, kRB, double>), dim3(gx), dim3(256), 0, st, n, X, Y, vals,
 		                   part, (const CgDev *)S, it);
 	hipLaunchKernelGGL((k_dots_fin<256, kRA, kRB>), dim3(1), dim3(256), 0, st, gx, X.info, Y.info, vals,
-	                   (const double *)part, J, fsum, S, it, mode, C, f32);
+	                   (const double *)part, J, fsum, S, it, mode, C, f32, counts);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The DOT of short vectors in one workgroup: both vectors in registers, the reference's split of each
+// level by level (ozblasSplitVecKernel, src/cpu/ozblas_split.cpp:75-104; x and y in one reduction round
+// a level), the slices again from the sigmas, all pair products, and the sum of dots_finish.  What
+// bounds a short DOT is launches: the general path's seven (fill, statistics, levels, scan, products,
+// completion, copy back) took 47 us at n = 1003.  Beyond kDotSmallMax elements one workgroup's
+// arithmetic costs more than the launches do.
+// ---------------------------------------------------------------------------------------------
+template <int BS, int E, class TI>
+__global__ __launch_bounds__(BS) void k_dot_small(int n, const TI *x, const TI *y, int rho, int shift, int cap,
+                                                  int reproMode, const uint16_t *Js, const uint16_t *Jn, int fsum,
+                                                  int *out) {
+	constexpr int NW = BS / 64, NS = 8;
+	__shared__ double red[2][NW][2];
+	__shared__ double wsum[NW][NS * NS];
+	__shared__ double vals[NS * NS];
+	const int w = threadIdx.x / 64;
+	TI v[2][E], keep[2][E];
+	int bad = 0;
+	double mx[2] = {0.0, 0.0};
+#pragma unroll
+	for (int e = 0; e < E; e++) {
+		const int i = (int)threadIdx.x + e * BS, ic = i < n ? i : n - 1;
+		const TI xl = x[ic], yl = y[ic];
+		keep[0][e] = v[0][e] = i < n ? xl : (TI)0;
+		keep[1][e] = v[1][e] = i < n ? yl : (TI)0;
+	}
+#pragma unroll
+	for (int e = 0; e < E; e++)
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			if (!isfinite(v[q][e])) bad = 1;
+			mx[q] = max_abs(mx[q], (double)v[q][e]);
+		}
+	int par = 0;
+	auto reduce = [&]() {  // the maxima of both vectors over the workgroup (one barrier: two buffers)
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			mx[q] = wave_max_nonneg_f64(mx[q]);
+			if (threadIdx.x % 64 == 0) red[par][w][q] = mx[q];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			mx[q] = red[par][0][q];
+#pragma unroll
+			for (int u = 1; u < NW; u++) mx[q] = std_max(mx[q], red[par][u][q]);
+		}
+		par ^= 1;
+	};
+	reduce();
+	const int bads = __syncthreads_or(bad);
+	TI sig[2][NS];
+	int z[2] = {cap, cap}, levels[2] = {0, 0};
+#pragma unroll
+	for (int q = 0; q < 2; q++)
+#pragma unroll
+		for (int s = 0; s < NS; s++) sig[q][s] = 0;
+#pragma unroll
+	for (int s = 0; s < NS; s++) {
+		const bool go0 = s < cap && z[0] == cap, go1 = s < cap && z[1] == cap;  // uniform
+		if (go0 || go1) {
+#pragma unroll
+			for (int q = 0; q < 2; q++) {
+				const bool go = q ? go1 : go0;
+				TI lm = 0;
+				if (go) {
+					sig[q][s] = SplitRule<TI>::sigma(rho, SplitRule<TI>::tau(mx[q], Js), shift);
+					levels[q] = s + 1;
+#pragma unroll
+					for (int e = 0; e < E; e++) {
+						const TI a = (v[q][e] + sig[q][s]) - sig[q][s];
+						v[q][e] = v[q][e] - a;
+						lm = max_abs(lm, v[q][e]);
+					}
+				}
+				mx[q] = (double)lm;
+			}
+			reduce();
+			if (go0 && mx[0] == 0.0) z[0] = s;
+			if (go1 && mx[1] == 0.0) z[1] = s;
+		}
+	}
+	// counts as the split loop's (src/cpu/ozblas_split.cpp:275-287)
+	int cnt[2];
+	bool over = bads != 0;
+#pragma unroll
+	for (int q = 0; q < 2; q++) {
+		cnt[q] = cap <= 1 ? 1 : z[q] < cap ? max(z[q], 1) + 1 : cap;
+		if (reproMode == 0) cnt[q]++;
+		over = over || cnt[q] > NS || (z[q] == cap && cap > NS);
+	}
+	if (over) {
+		if (threadIdx.x == 0) out[2] = 1;
+		return;
+	}
+	// slot s of an element: the slice of level s; the remainder (0 after a zero level) in the slot
+	// after the last level, which sigma = 0 yields; 0 from there on, and from the count on
+	double acc[NS * NS];
+#pragma unroll
+	for (int q = 0; q < NS * NS; q++) acc[q] = 0.0;
+#pragma unroll
+	for (int e = 0; e < E; e++) {
+		double sx[NS], sy[NS];
+		TI rx = keep[0][e], ry = keep[1][e];
+#pragma unroll
+		for (int s = 0; s < NS; s++) {
+			const TI a = (rx + sig[0][s]) - sig[0][s], b = (ry + sig[1][s]) - sig[1][s];
+			sx[s] = s < cnt[0] ? (double)a : 0.0;
+			sy[s] = s < cnt[1] ? (double)b : 0.0;
+			rx = rx - a;
+			ry = ry - b;
+		}
+#pragma unroll
+		for (int a = 0; a < NS; a++)
+			if (a < cnt[0]) {
+#pragma unroll
+				for (int b = 0; b < NS; b++) acc[a * NS + b] = fma(sx[a], sy[b], acc[a * NS + b]);
+			}
+	}
+	wave_reduce_pairs(acc, wsum[w]);
+	__syncthreads();
+	if (threadIdx.x < NS * NS) {
+		const int a = threadIdx.x / NS, b = threadIdx.x % NS;
+		double t = wsum[0][threadIdx.x];
+#pragma unroll
+		for (int u = 1; u < NW; u++) t += wsum[u][threadIdx.x];
+		if (a < cnt[0] && b < cnt[1]) vals[a + cnt[0] * b] = t;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) out[2] = 0;
+	dots_finish<BS>(cnt[0], cnt[1], vals, nullptr, 0, Jn, fsum, nullptr, 0, 0, out + 4, sizeof(TI) == 4 ? 1 : 0, out);
+}
+
+template <class TI>
+static void dot_small(hipStream_t st, int n, const TI *x, const TI *y, int rho, int shift, int cap, int reproMode,
+                      const uint16_t *Js, const uint16_t *Jn, int fsum, int *out) {
+	static_assert(kDotSmallMax <= 512 * 16, "elements per thread");
+#define OZ_DOT_SMALL(BS, E)                                                                                  \
+	hipLaunchKernelGGL((k_dot_small<BS, E, TI>), dim3(1), dim3(BS), 0, st, n, x, y, rho, shift, cap, reproMode, \
+	                   Js, Jn, fsum, out)
+	if (n <= 256 * 4)
+		OZ_DOT_SMALL(256, 4);
+	else if (n <= 512 * 8)
+		OZ_DOT_SMALL(512, 8);
+	else
+		OZ_DOT_SMALL(512, 16);
+#undef OZ_DOT_SMALL
+}
+
+void launch_dot_small(hipStream_t st, int n, const double *x, const double *y, int rho, int shift, int cap,
+                      int reproMode, const uint16_t *Js, const uint16_t *Jn, int fsum, int *out) {
+	dot_small(st, n, x, y, rho, shift, cap, reproMode, Js, Jn, fsum, out);
+}
+
+void launch_dot_small(hipStream_t st, int n, const float *x, const float *y, int rho, int shift, int cap,
+                      int reproMode, const uint16_t *JF, const uint16_t *JF2, int fsum, int *out) {
+	dot_small(st, n, x, y, rho, shift, cap, reproMode, JF, JF2, fsum, out);
 }
 
 // the AXPYs that also reduce for the next split: fewer workgroups (each reduces once)

@@ -223,16 +223,18 @@ __global__ void k_copy(const double *src, double *dst, int64_t n) {
 // the binary32 split (slices stored as doubles).
 // ---------------------------------------------------------------------------------------------
 template <class TI>
-__global__ void k_split_csr(int m, const TI *val, const int *rowptr, TI *work, double *split,
-                            int64_t lds, int shift, int cap, const uint16_t *J, int *zrow,
-                            int *zmax, int epsMode, int mixed) {
-	const int r = blockIdx.x * blockDim.x + threadIdx.x;
-	if (r >= m) return;
-	const int b = rowptr[r], e = rowptr[r + 1];
+__device__ __forceinline__ int csr_rho(int len, int epsMode, int mixed) {
 	// the mixed splits (binary64 data into binary32 slices, binary32 data into binary64 slices)
 	// have their own rho, the rest is the same
-	const int rho = !mixed ? SplitRule<TI>::rho_row(e - b, epsMode)
-	                       : (sizeof(TI) == 8 ? rho_dev_ds(e - b, epsMode) : rho_dev_sd(e - b, epsMode));
+	return !mixed ? SplitRule<TI>::rho_row(len, epsMode)
+	              : (sizeof(TI) == 8 ? rho_dev_ds(len, epsMode) : rho_dev_sd(len, epsMode));
+}
+
+template <class TI>
+__device__ void split_csr_row(int r, const TI *val, const int *rowptr, TI *work, double *split, int64_t lds,
+                              int shift, int cap, const uint16_t *J, int *zrow, int *zmax, int epsMode, int mixed) {
+	const int b = rowptr[r], e = rowptr[r + 1];
+	const int rho = csr_rho<TI>(e - b, epsMode, mixed);
 	double mx = 0.0;
 	for (int i = b; i < e; i++) mx = std_max(mx, fabs((double)val[i]));
 	int s = 0;
@@ -260,6 +262,73 @@ __global__ void k_split_csr(int m, const TI *val, const int *rowptr, TI *work, d
 	const int z = zero ? s : cap;
 	zrow[r] = z;
 	count_max(zmax, z);
+}
+
+// The same with the rows of a workgroup (256, one contiguous range of nonzeros) in LDS: remainders and
+// the current slice are rows in LDS, each slice leaves as one contiguous store of the range, and the
+// remainders never touch memory (row by row in memory: 0.34 ms for the 100^3 Laplacian, 2 slices, most
+// of it partial cache lines).  A longer range takes split_csr_row.
+constexpr int kCsrSplitCap = 2048;
+template <class TI>
+__global__ __launch_bounds__(256) void k_split_csr_staged(int m, const TI *val, const int *rowptr, TI *work,
+                                                          double *split, int64_t lds, int shift, int cap,
+                                                          const uint16_t *J, int *zrow, int *zmax, int epsMode,
+                                                          int mixed) {
+	const int r0 = blockIdx.x * 256, rows = min(256, m - r0);
+	const int base = rowptr[r0], cnt = rowptr[r0 + rows] - base;
+	const int r = r0 + (int)threadIdx.x;
+	if (cnt > kCsrSplitCap) {
+		if (r < m) split_csr_row(r, val, rowptr, work, split, lds, shift, cap, J, zrow, zmax, epsMode, mixed);
+		return;
+	}
+	__shared__ TI rem[kCsrSplitCap];
+	__shared__ double sl[kCsrSplitCap];
+	for (int i = threadIdx.x; i < cnt; i += 256) rem[i] = val[base + i];
+	__syncthreads();
+	int b = 0, e = 0, rho = 0;
+	double mx = 0.0;
+	if (r < m) {
+		b = rowptr[r] - base;
+		e = rowptr[r + 1] - base;
+		rho = csr_rho<TI>(e - b, epsMode, mixed);
+		for (int i = b; i < e; i++) mx = std_max(mx, fabs((double)rem[i]));
+	}
+	// done: the row's remainders are zero; its slots from the next one on hold 0 (the slot after the last
+	// slice) or nothing, as the row loop leaves them
+	bool done = r >= m;
+	int z = cap;
+	for (int s = 0; s <= cap; s++) {
+		// slot s: the slice of level s, the remainder after the last level, or the zero after it
+		if (!done && s < cap) {
+			const int tau = SplitRule<TI>::tau(mx, J);
+			const TI sigma = SplitRule<TI>::sigma_div(rho, tau, shift);
+			double lm = 0.0;
+			for (int i = b; i < e; i++) {
+				const TI v = rem[i];
+				const TI a = (v + sigma) - sigma;
+				const TI rr = v - a;
+				sl[i] = (double)a;
+				rem[i] = rr;
+				lm = std_max(lm, fabs((double)rr));
+			}
+			mx = lm;
+			if (mx == 0.0) {
+				done = true;
+				z = s;
+			}
+		} else if (r < m) {
+			for (int i = b; i < e; i++) sl[i] = done ? 0.0 : (double)rem[i];
+		}
+		const bool more = __syncthreads_or(!done || (s <= z && z < cap));
+		for (int i = threadIdx.x; i < cnt; i += 256) split[(int64_t)s * lds + base + i] = sl[i];
+		__syncthreads();
+		if (!more) break;
+	}
+	// one counter update per workgroup
+	if (r < m) zrow[r] = z;
+	z = r < m ? z : 0;
+	z = wave_max_i32(z);
+	if (threadIdx.x % 64 == 0) count_max(zmax, z);
 }
 
 __global__ void k_zero_slots_csr(int m, const int *rowptr, double *split, int64_t lds,
@@ -429,14 +498,14 @@ void launch_copy(hipStream_t st, const double *src, double *dst, int64_t n) {
 void launch_split_csr(hipStream_t st, int m, const double *val, const int *rowptr, double *work,
                       double *split, int64_t lds, int shift, int cap, const uint16_t *J, int *zrow,
                       int *zmax, int epsMode, int mixed) {
-	hipLaunchKernelGGL(k_split_csr<double>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
+	hipLaunchKernelGGL(k_split_csr_staged<double>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
 	                   work, split, lds, shift, cap, J, zrow, zmax, epsMode, mixed);
 }
 
 void launch_split_csr(hipStream_t st, int m, const float *val, const int *rowptr, float *work,
                       double *split, int64_t lds, int shift, int cap, const uint16_t *JF, int *zrow,
                       int *zmax, int epsMode, int mixed) {
-	hipLaunchKernelGGL(k_split_csr<float>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
+	hipLaunchKernelGGL(k_split_csr_staged<float>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
 	                   work, split, lds, shift, cap, JF, zrow, zmax, epsMode, mixed);
 }
 
