@@ -1361,7 +1361,7 @@ template <int NAM>
 __device__ __forceinline__ bool csr_stage_load(CsrStage<NAM> &st, int base, int cnt, const double *As,
                                                int64_t ldas, int nA, const int *colind, const double *X) {
 	if (cnt > CsrStage<NAM>::kCap) return false;
-	constexpr int U = 4;
+	constexpr int U = CsrStage<NAM>::kCap / kCsrRows;  // the whole stage in one round of loads
 	for (int i0 = threadIdx.x; i0 < cnt; i0 += U * kCsrRows) {
 		int c[U];
 		double a[U][NAM], x[U];
@@ -2155,19 +2155,27 @@ __device__ void dots_finish(int nA, int nB, double *vals, const double *part, in
 			// memory, so a round is a full memory latency)
 			double v[kDotFinOne];
 #pragma unroll
-			for (int q = 0; q < kDotFinOne; q++) {
-				// unconditional loads inside the buffer (kDotPairs x kDotMaxWG); the rows q >= npairs
-				// are summed too and never read
-				const double *row = part + (int64_t)q * kDotMaxWG;
-				const double a = row[t], b = row[t + BS];
-				v[q] = (t < nwg ? a : 0.0) + (t + BS < nwg ? b : 0.0);
+			for (int q0 = 0; q0 < kDotFinOne; q0 += 4) {
+				if (q0 < npairs) {  // uniform; loads inside the buffer (kDotPairs x kDotMaxWG)
+#pragma unroll
+					for (int q = q0; q < q0 + 4; q++) {
+						const double *row = part + (int64_t)q * kDotMaxWG;
+						const double a = row[t], b = row[t + BS];
+						v[q] = (t < nwg ? a : 0.0) + (t + BS < nwg ? b : 0.0);
+					}
+				}
 			}
-#pragma unroll
-			for (int q = 0; q < kDotFinOne; q++) v[q] = wave_sum63_f64(v[q]);
 			__shared__ double redOne[BS / 64][kDotFinOne];
-			if (l == 63) {
 #pragma unroll
-				for (int q = 0; q < kDotFinOne; q++) redOne[w][q] = v[q];
+			for (int q0 = 0; q0 < kDotFinOne; q0 += 4) {
+				if (q0 < npairs) {
+#pragma unroll
+					for (int q = q0; q < q0 + 4; q++) v[q] = wave_sum63_f64(v[q]);
+					if (l == 63) {
+#pragma unroll
+						for (int q = q0; q < q0 + 4; q++) redOne[w][q] = v[q];
+					}
+				}
 			}
 			__syncthreads();
 			if (t < npairs) {
@@ -2210,7 +2218,10 @@ __device__ void dots_finish(int nA, int nB, double *vals, const double *part, in
 		const double pv = ((int)threadIdx.x < npairs) ? src[threadIdx.x] : 0.0;
 		const bool finite = __all(!(fabs(pv) > 1.7976931348623157e308) && pv == pv);
 		if (finite) {
-			tw = nearsum_wave(npairs, pv, J);
+			// the clear-cut case, the same in every lane; else across the wave
+			SumCert c;
+			for (int q = 0; q < npairs; q++) c.add(src[q]);
+			if (!c.done(npairs, tw)) tw = nearsum_wave(npairs, pv, J);
 			waveDone = true;
 		}
 	}
@@ -2330,12 +2341,19 @@ __device__ __forceinline__ void vs_ref_load(const VsRef &V, bool stored, const V
 	}
 }
 
+// the first cnt slots (uniform), 0 beyond
 template <class TI, int NS>
-__device__ __forceinline__ void vs_gen_masked(const VsGen<TI, NS> &g, TI v, int cnt, double (&out)[NS]) {
-	g.gen(v, out);
+__device__ __forceinline__ void vs_gen_count(const VsGen<TI, NS> &g, TI v, int cnt, double (&out)[NS]) {
+	TI r = v;
 #pragma unroll
-	for (int q = 0; q < NS; q++)
-		if (q >= cnt) out[q] = 0.0;
+	for (int q = 0; q < NS; q++) {
+		out[q] = 0.0;
+		if (q < cnt) {
+			const TI a = (r + g.sig[q]) - g.sig[q];
+			out[q] = (double)a;
+			r = r - a;
+		}
+	}
 }
 
 // The sums over the 64 lanes of 64 values each (exact, so any order) to out[0, 64), by every lane of a
@@ -2419,9 +2437,9 @@ __device__ __forceinline__ void dots_reg_acc(int n, const VsRef &X, const VsRef 
 			const bool in = ie < n;
 			double xa[NAM], yb[NBM];
 			if constexpr (SX) vs_ref_load<TI, NAM>(X, true, gx, nA, ie, in, xa);
-			else vs_gen_masked<TI, NAM>(gx, xe[e], nA, xa);
+			else vs_gen_count<TI, NAM>(gx, xe[e], nA, xa);
 			if constexpr (SY) vs_ref_load<TI, NBM>(Y, true, gy, nB, ie, in, yb);
-			else vs_gen_masked<TI, NBM>(gy, ye[e], nB, yb);
+			else vs_gen_count<TI, NBM>(gy, ye[e], nB, yb);
 #pragma unroll
 			for (int a = 0; a < NAM; a++)
 				if (a < nA) {
