@@ -963,7 +963,7 @@ hipError_t launch_vsplit_plan(hipStream_t st, int n, const float *x, double *sli
 constexpr int kDotChunk = 16;
 constexpr int kDotPairs = 64;    // pair slots per workgroup partial of k_dots_reg
 constexpr int kDotMaxWG = 512;  // workgroups of k_dots_reg at most (two waves per SIMD)
-constexpr int kDotFinOne = 36;  // pair counts (6 x 6 slices) whose partials k_dots_fin loads in one round
+constexpr int kDotFinBS = 1024;  // threads of the completion
 
 template <int BS>
 __global__ __launch_bounds__(BS) void k_slice_dots(int n, const double *xs, int64_t ldx, int nA,
@@ -2140,73 +2140,38 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 template <int BS>
 __device__ void dots_finish(int nA, int nB, double *vals, const double *part, int nwg, const uint16_t *J,
                             int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
-	static_assert(kDotMaxWG <= 2 * BS, "two partials per thread and pair");
 	__shared__ double psum[kDotPairs];
-	__shared__ double red[BS / 64][16];
 	const int npairs = nA * nB;
 	double *src = vals;
 	if (part) {
-		// pairs in chunks of 16: every thread loads its (at most two) partials of each pair of the
-		// chunk, all loads in flight together (pair p's partials are contiguous: pair-major), then a
-		// sum over each wave (DPP) and the waves' sums in LDS
-		const int t = threadIdx.x, w = t / 64, l = t % 64;
-		if (npairs <= kDotFinOne) {
-			// one round: every load of every pair in flight together (the partials come from
-			// memory, so a round is a full memory latency)
-			double v[kDotFinOne];
+		// wave w sums pair w, w + waves, ...: its partials are contiguous (pair-major), kDotMaxWG / 64 loads
+		// a lane and pair, all of a wave's pairs in flight together (the partials come from memory, so a
+		// round is a full memory latency), then one wave sum a pair
+		constexpr int NW = BS / 64, PW = (kDotPairs + NW - 1) / NW, L = kDotMaxWG / 64;
+		const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+		double v[PW];
 #pragma unroll
-			for (int q0 = 0; q0 < kDotFinOne; q0 += 4) {
-				if (q0 < npairs) {  // uniform; loads inside the buffer (kDotPairs x kDotMaxWG)
+		for (int q = 0; q < PW; q++) {
+			v[q] = 0.0;
+			const int p = w + q * NW;
+			if (p < npairs) {  // uniform over the wave
+				const double *row = part + (int64_t)p * kDotMaxWG + l;
 #pragma unroll
-					for (int q = q0; q < q0 + 4; q++) {
-						const double *row = part + (int64_t)q * kDotMaxWG;
-						const double a = row[t], b = row[t + BS];
-						v[q] = (t < nwg ? a : 0.0) + (t + BS < nwg ? b : 0.0);
-					}
+				for (int u = 0; u < L; u++) {
+					const double a = row[64 * u];  // inside the buffer; not written beyond nwg
+					v[q] += l + 64 * u < nwg ? a : 0.0;
 				}
 			}
-			__shared__ double redOne[BS / 64][kDotFinOne];
-#pragma unroll
-			for (int q0 = 0; q0 < kDotFinOne; q0 += 4) {
-				if (q0 < npairs) {
-#pragma unroll
-					for (int q = q0; q < q0 + 4; q++) v[q] = wave_sum63_f64(v[q]);
-					if (l == 63) {
-#pragma unroll
-						for (int q = q0; q < q0 + 4; q++) redOne[w][q] = v[q];
-					}
-				}
-			}
-			__syncthreads();
-			if (t < npairs) {
-				double r = redOne[0][t];
-				for (int k = 1; k < BS / 64; k++) r += redOne[k][t];
-				psum[t] = r;
-			}
-			__syncthreads();
 		}
-		for (int p0 = (npairs <= kDotFinOne) ? npairs : 0; p0 < npairs; p0 += 16) {
-			double v[16];
 #pragma unroll
-			for (int q = 0; q < 16; q++) {
-				const double *row = part + (int64_t)min(p0 + q, kDotPairs - 1) * kDotMaxWG;
-				const double a = row[t], b = row[t + BS];
-				v[q] = (t < nwg ? a : 0.0) + (t + BS < nwg ? b : 0.0);
+		for (int q = 0; q < PW; q++) {
+			const int p = w + q * NW;
+			if (p < npairs) {
+				const double t = wave_sum63_f64(v[q]);
+				if (l == 63) psum[p] = t;
 			}
-#pragma unroll
-			for (int q = 0; q < 16; q++) v[q] = wave_sum63_f64(v[q]);
-			if (l == 63) {
-#pragma unroll
-				for (int q = 0; q < 16; q++) red[w][q] = v[q];
-			}
-			__syncthreads();
-			if (t < 16 && p0 + t < npairs) {
-				double r = red[0][t];
-				for (int k = 1; k < BS / 64; k++) r += red[k][t];
-				psum[p0 + t] = r;
-			}
-			__syncthreads();
 		}
+		__syncthreads();
 		src = psum;
 	}
 	const int maxlevel = (nA - 1) + (nB - 1);  // DOT forces fastMode = 0 (src/cpu/ozblas_gemm.cpp:25-28)
@@ -2341,26 +2306,19 @@ __device__ __forceinline__ void vs_ref_load(const VsRef &V, bool stored, const V
 	}
 }
 
-// the first cnt slots (uniform), 0 beyond
 template <class TI, int NS>
-__device__ __forceinline__ void vs_gen_count(const VsGen<TI, NS> &g, TI v, int cnt, double (&out)[NS]) {
-	TI r = v;
+__device__ __forceinline__ void vs_gen_masked(const VsGen<TI, NS> &g, TI v, int cnt, double (&out)[NS]) {
+	g.gen(v, out);
 #pragma unroll
-	for (int q = 0; q < NS; q++) {
-		out[q] = 0.0;
-		if (q < cnt) {
-			const TI a = (r + g.sig[q]) - g.sig[q];
-			out[q] = (double)a;
-			r = r - a;
-		}
-	}
+	for (int q = 0; q < NS; q++)
+		if (q >= cnt) out[q] = 0.0;
 }
 
-// The sums over the 64 lanes of 64 values each (exact, so any order) to out[0, 64), by every lane of a
-// wave.  Two halving exchanges first: swapping the lane halves of values q and q + 32 and adding leaves
-// lane half h with value q + 32 h, swapping neighbouring rows of 16 lanes the same way with 16 values a
-// lane; those are summed over the rows on the DPP network.  336 instructions, against 1152 for 64 full
-// wave sums.
+// The sums over the 64 lanes of NV values each (exact, so any order) to out[0, NV), by every lane of a
+// wave.  Two halving exchanges first: swapping the lane halves of values q and q + NV / 2 and adding
+// leaves lane half h with value q + h NV / 2, swapping neighbouring rows of 16 lanes the same way with
+// NV / 4 values a lane; those are summed over the rows on the DPP network.  For 64 values 336
+// instructions, against 1152 for 64 full wave sums.
 __device__ __forceinline__ double swap_add32(double a, double b) {
 	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
 	const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
@@ -2375,15 +2333,17 @@ __device__ __forceinline__ double swap_add16(double a, double b) {
 	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
 	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
 }
-__device__ __forceinline__ void wave_reduce_pairs(double (&v)[64], double *out) {
-	double a[32], b[16];
+template <int NV>
+__device__ __forceinline__ void wave_reduce_pairs(double (&v)[NV], double *out) {
+	static_assert(NV % 4 == 0, "two halvings");
+	double a[NV / 2], b[NV / 4];
 #pragma unroll
-	for (int q = 0; q < 32; q++) a[q] = swap_add32(v[q], v[q + 32]);
+	for (int q = 0; q < NV / 2; q++) a[q] = swap_add32(v[q], v[q + NV / 2]);
 #pragma unroll
-	for (int q = 0; q < 16; q++) b[q] = swap_add16(a[q], a[q + 16]);
-	const int l = threadIdx.x % 64, p0 = 16 * ((l / 16) % 2) + 32 * (l / 32);
+	for (int q = 0; q < NV / 4; q++) b[q] = swap_add16(a[q], a[q + NV / 4]);
+	const int l = threadIdx.x % 64, p0 = (NV / 4) * ((l / 16) % 2) + (NV / 2) * (l / 32);
 #pragma unroll
-	for (int q = 0; q < 16; q++) {
+	for (int q = 0; q < NV / 4; q++) {
 		double t = b[q];
 		t += dpp_f64<0xB1>(t);   // quad_perm [1,0,3,2]
 		t += dpp_f64<0x4E>(t);   // quad_perm [2,3,0,1]
@@ -2399,6 +2359,55 @@ __device__ __forceinline__ void wave_reduce_pairs(double (&v)[64], double *out) 
 // stores its pair partials to part[p * kDotMaxWG + blockIdx.x] -- no atomics on a few shared
 // addresses -- and k_dots_fin sums them (integer multiples of the product unit below 2^53: any
 // order is exact).  Larger counts take dots_general.
+// The whole of k_dots_reg for two plans of at most N slices whose slots need no masking: the slots past
+// the count are zero by themselves, because the chain ended in zero or the remainder's slot is counted.
+// Without the masks and the per-row guards an element is 6 N + N^2 instructions; with them the compiler
+// spilled scalars into lanes (736 v_readlane) and two vectors of 10^6 took 11 us.
+constexpr int kDotStep = 8;  // elements per thread and step, their loads in flight together
+template <int BS, int N, class TI>
+__device__ __forceinline__ void dots_exact(int n, const VsRef &X, const VsRef &Y, int nA, int nB, double *red,
+                                           double *part) {
+	const TI *xv = (const TI *)X.x, *yv = (const TI *)Y.x;
+	const int64_t stride = (int64_t)gridDim.x * BS;
+	double acc[N * N];
+#pragma unroll
+	for (int q = 0; q < N * N; q++) acc[q] = 0.0;
+	VsGen<TI, N> gx, gy;
+	gx.init(X.plan);
+	gy.init(Y.plan);
+	for (int64_t i = blockIdx.x * (int64_t)BS + threadIdx.x; i < n; i += kDotStep * stride) {
+		TI xe[kDotStep], ye[kDotStep];
+#pragma unroll
+		for (int e = 0; e < kDotStep; e++) {  // clamped past the end, where x counts as zero
+			const int64_t ie = i + e * stride, ic = min(ie, (int64_t)n - 1);
+			const TI xl = xv[ic];
+			xe[e] = ie < n ? xl : (TI)0;
+			ye[e] = yv[ic];
+		}
+#pragma unroll
+		for (int e = 0; e < kDotStep; e++) {
+			double xa[N], yb[N];
+			gx.gen(xe[e], xa);
+			gy.gen(ye[e], yb);
+#pragma unroll
+			for (int a = 0; a < N; a++)
+#pragma unroll
+				for (int b = 0; b < N; b++) acc[a * N + b] = fma(xa[a], yb[b], acc[a * N + b]);
+		}
+	}
+	wave_reduce_pairs<N * N>(acc, red + (threadIdx.x / 64) * N * N);
+	__syncthreads();
+	for (int q = threadIdx.x; q < N * N; q += BS) {
+		const int a = q / N, b = q % N;
+		if (a < nA && b < nB) {
+			double v = red[q];
+#pragma unroll
+			for (int k = 1; k < BS / 64; k++) v += red[k * N * N + q];
+			part[(int64_t)(a + nA * b) * kDotMaxWG + blockIdx.x] = v;  // pair-major
+		}
+	}
+}
+
 // the pair accumulation over this thread's elements; SX / SY: the vector's slices are stored (its
 // plan is marked bad) rather than generated
 template <int BS, int NAM, int NBM, class TI, bool SX, bool SY>
@@ -2410,7 +2419,7 @@ __device__ __forceinline__ void dots_reg_acc(int n, const VsRef &X, const VsRef 
 	if constexpr (!SY) gy.init(Y.plan);
 	const TI *xv = (const TI *)X.x, *yv = (const TI *)Y.x;
 	const int64_t stride = (int64_t)gridDim.x * BS;
-	constexpr int E = (SX || SY || sizeof(TI) == 4) ? 2 : 4;  // elements per thread and step
+	constexpr int E = 2;  // elements per thread and step
 	for (int64_t i = blockIdx.x * (int64_t)BS + threadIdx.x; i < n; i += E * stride) {
 		// every element's loads in flight, then one element's slices at a time
 		TI xe[E], ye[E];
@@ -2437,9 +2446,9 @@ __device__ __forceinline__ void dots_reg_acc(int n, const VsRef &X, const VsRef 
 			const bool in = ie < n;
 			double xa[NAM], yb[NBM];
 			if constexpr (SX) vs_ref_load<TI, NAM>(X, true, gx, nA, ie, in, xa);
-			else vs_gen_count<TI, NAM>(gx, xe[e], nA, xa);
+			else vs_gen_masked<TI, NAM>(gx, xe[e], nA, xa);
 			if constexpr (SY) vs_ref_load<TI, NBM>(Y, true, gy, nB, ie, in, yb);
-			else vs_gen_count<TI, NBM>(gy, ye[e], nB, yb);
+			else vs_gen_masked<TI, NBM>(gy, ye[e], nB, yb);
 #pragma unroll
 			for (int a = 0; a < NAM; a++)
 				if (a < nA) {
@@ -2450,8 +2459,10 @@ __device__ __forceinline__ void dots_reg_acc(int n, const VsRef &X, const VsRef 
 	}
 }
 
+// (two waves per SIMD: the masked instance alone would take 264 registers and leave one workgroup a CU,
+// two rounds of the grid)
 template <int BS, int NAM, int NBM, class TI>
-__global__ __launch_bounds__(BS) void k_dots_reg(int n, VsRef X, VsRef Y, double *vals, double *part,
+__global__ __launch_bounds__(BS, 2) void k_dots_reg(int n, VsRef X, VsRef Y, double *vals, double *part,
                                                  const CgDev *S, int it) {
 	static_assert(NAM * NBM <= kDotPairs && BS % 64 == 0 && BS <= 256, "pair partial layout");
 	if (cg_skip(S, it)) return;
@@ -2460,14 +2471,22 @@ __global__ __launch_bounds__(BS) void k_dots_reg(int n, VsRef X, VsRef Y, double
 		dots_general<BS, TI>(n, nA, nB, X, Y, vals);
 		return;
 	}
-	const bool sx = X.plan->bad, sy = Y.plan->bad;
+	const bool storedX = X.plan->bad, storedY = Y.plan->bad;
 	__shared__ double red[BS / 64][NAM * NBM];
+	auto plain = [](const VsPlan *p, int cnt) { return !p->bad && (p->zero || cnt > p->last + 1); };
+	if (plain(X.plan, nA) && plain(Y.plan, nB)) {
+		const int m = max(nA, nB);
+		if (m <= 4) dots_exact<BS, 4, TI>(n, X, Y, nA, nB, red[0], part);
+		else if (m <= 6) dots_exact<BS, 6, TI>(n, X, Y, nA, nB, red[0], part);
+		else dots_exact<BS, 8, TI>(n, X, Y, nA, nB, red[0], part);
+		return;
+	}
 	double acc[NAM * NBM];
 #pragma unroll
 	for (int q = 0; q < NAM * NBM; q++) acc[q] = 0.0;
-	if (!sx && !sy) dots_reg_acc<BS, NAM, NBM, TI, false, false>(n, X, Y, nA, nB, acc);
-	else if (!sx) dots_reg_acc<BS, NAM, NBM, TI, false, true>(n, X, Y, nA, nB, acc);
-	else if (!sy) dots_reg_acc<BS, NAM, NBM, TI, true, false>(n, X, Y, nA, nB, acc);
+	if (!storedX && !storedY) dots_reg_acc<BS, NAM, NBM, TI, false, false>(n, X, Y, nA, nB, acc);
+	else if (!storedX) dots_reg_acc<BS, NAM, NBM, TI, false, true>(n, X, Y, nA, nB, acc);
+	else if (!storedY) dots_reg_acc<BS, NAM, NBM, TI, true, false>(n, X, Y, nA, nB, acc);
 	else dots_reg_acc<BS, NAM, NBM, TI, true, true>(n, X, Y, nA, nB, acc);
 	wave_reduce_pairs(acc, red[threadIdx.x / 64]);
 	__syncthreads();
@@ -2523,11 +2542,24 @@ __global__ __launch_bounds__(256) void k_scal_axpy_dev(int n, CgDev *S, int it, 
 	const T b = (T)S->beta;
 	double mx = 0.0;
 	int lo = 0, bad = 0;
-	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-	     i += (int64_t)gridDim.x * blockDim.x) {
-		const T p = fma1_t((T)1, R[i], b * P[i]);
-		P[i] = p;
-		vs_stats_acc((double)p, mx, lo, bad);
+	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += 4 * stride) {
+		T r[4], p[4];  // four elements' loads in flight (clamped past the end)
+#pragma unroll
+		for (int e = 0; e < 4; e++) {
+			const int64_t ie = min(i + e * stride, (int64_t)n - 1);
+			r[e] = R[ie];
+			p[e] = P[ie];
+		}
+#pragma unroll
+		for (int e = 0; e < 4; e++) {
+			const int64_t ie = i + e * stride;
+			if (ie < n) {
+				const T t = fma1_t((T)1, r[e], b * p[e]);
+				P[ie] = t;
+				vs_stats_acc((double)t, mx, lo, bad);
+			}
+		}
 	}
 	vs_stats_flush<256>(mx, lo, bad, preP);
 }
@@ -2567,7 +2599,7 @@ size_t dots_part_bytes() { return sizeof(double) * kDotPairs * kDotMaxWG; }
 void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, double *part,
                      const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
 	constexpr int kRA = 8, kRB = 8;
-	int gx = (n + 1023) / 1024;  // four elements per thread and step
+	int gx = (n + 256 * kDotStep - 1) / (256 * kDotStep);
 	if (gx > kDotMaxWG) gx = kDotMaxWG;
 	if (gx < 1) gx = 1;
 	if (f32)
@@ -2576,7 +2608,7 @@ void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, doub
 	else
 		hipLaunchKernelGGL((k_dots_reg<256, kRA, kRB, double>), dim3(gx), dim3(256), 0, st, n, X, Y, vals,
 		                   part, (const CgDev *)S, it);
-	hipLaunchKernelGGL((k_dots_fin<256, kRA, kRB>), dim3(1), dim3(256), 0, st, gx, X.info, Y.info, vals,
+	hipLaunchKernelGGL((k_dots_fin<kDotFinBS, kRA, kRB>), dim3(1), dim3(kDotFinBS), 0, st, gx, X.info, Y.info, vals,
 	                   (const double *)part, J, fsum, S, it, mode, C, f32, counts);
 }
 
@@ -2597,15 +2629,15 @@ __global__ __launch_bounds__(BS) void k_dot_small(int n, const TI *x, const TI *
 	__shared__ double wsum[NW][NS * NS];
 	__shared__ double vals[NS * NS];
 	const int w = threadIdx.x / 64;
-	TI v[2][E], keep[2][E];
+	TI v[2][E];
 	int bad = 0;
 	double mx[2] = {0.0, 0.0};
 #pragma unroll
 	for (int e = 0; e < E; e++) {
 		const int i = (int)threadIdx.x + e * BS, ic = i < n ? i : n - 1;
 		const TI xl = x[ic], yl = y[ic];
-		keep[0][e] = v[0][e] = i < n ? xl : (TI)0;
-		keep[1][e] = v[1][e] = i < n ? yl : (TI)0;
+		v[0][e] = i < n ? xl : (TI)0;
+		v[1][e] = i < n ? yl : (TI)0;
 	}
 #pragma unroll
 	for (int e = 0; e < E; e++)
@@ -2678,13 +2710,13 @@ __global__ __launch_bounds__(BS) void k_dot_small(int n, const TI *x, const TI *
 	}
 	// slot s of an element: the slice of level s; the remainder (0 after a zero level) in the slot
 	// after the last level, which sigma = 0 yields; 0 from there on, and from the count on
+	// (the elements are read again: held through the levels they would cost the registers of the sums)
 	double acc[NS * NS];
 #pragma unroll
 	for (int q = 0; q < NS * NS; q++) acc[q] = 0.0;
-#pragma unroll
-	for (int e = 0; e < E; e++) {
+	for (int i = threadIdx.x; i < n; i += BS) {
 		double sx[NS], sy[NS];
-		TI rx = keep[0][e], ry = keep[1][e];
+		TI rx = x[i], ry = y[i];
 #pragma unroll
 		for (int s = 0; s < NS; s++) {
 			const TI a = (rx + sig[0][s]) - sig[0][s], b = (ry + sig[1][s]) - sig[1][s];
