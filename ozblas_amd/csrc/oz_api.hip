@@ -71,6 +71,14 @@ struct Prec<float> {
 	static const uint16_t *Jsum(Backend *b) { return b->dTauF2; }
 };
 
+// Whether a binary32 vector of n elements is to be met with the kernels for up to kCsrWideSlices slices: a
+// slice holds 24 - rho bits, so full mantissas take 24 / (24 - rho) slices and a spread of exponents a few
+// more.  The kernels for up to 8 hold fewer registers; a vector that exceeds them is computed again.
+static bool wide_vector(const ozblasHandle_t *oh, int n) {
+	const int bits = 24 - Prec<float>::rho(oh, n);
+	return !be(oh)->mixed && bits >= 1 && 24 / bits + 2 > kCsrPlanSlices;
+}
+
 // reference slice count from the per-column first-zero index (max over columns)
 static inline int split_count(const ozblasHandle_t *oh, int zmax) {
 	const int cap = split_cap(oh);
@@ -930,13 +938,9 @@ static int32_t vz_begin(ozblasHandle_t *oh) {
 	return OZBLAS_STATUS_SUCCESS;
 }
 
-// Splits x; with readCount the slice count is read back to the host (one synchronisation),
-// otherwise it stays on the device in vs.info for kernels that read it there.  With planOnly the
-// slices are stored only for a plan outside the residue model: the consumer generates them from
-// (x, plan) (VsRef).
+// Splits x into stored slices and reads their count back (one synchronisation).
 template <class T>
-static int32_t vec_split(ozblasHandle_t *oh, int n, const T *x, VecSplit &vs, bool readCount = true,
-                         bool planOnly = false) {
+static int32_t vec_split(ozblasHandle_t *oh, int n, const T *x, VecSplit &vs) {
 	Backend *b = be(oh);
 	const int cap = split_cap(oh);
 	const int rho = Prec<T>::rho(oh, n);
@@ -944,20 +948,15 @@ static int32_t vec_split(ozblasHandle_t *oh, int n, const T *x, VecSplit &vs, bo
 	vs.lds = rup(n, 32);
 	vs.slices = (double *)walloc(oh, 8ull * vs.lds * (cap + 2));
 	vs.info = (int *)walloc(oh, 16);
-	void *scratch = walloc(oh, vsplit_scratch_bytes());
 	vs.plan = (VsPlan *)walloc(oh, sizeof(VsPlan));
-	if (!vs.slices || !vs.info || !scratch || !vs.plan) return OZBLAS_STATUS_WORKSPACE;
-	OZ_HIP(hipMemsetAsync(scratch, 0, vsplit_scratch_bytes(), b->stream));
-	if (planOnly)
-		OZ_HIP(launch_vsplit_plan(b->stream, n, x, vs.slices, vs.lds, rho, oh->splitShift, cap,
-		                          repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), vs.info, scratch, nullptr,
-		                          vs.plan, false));
-	else
-		OZ_HIP(launch_vsplit(b->stream, n, x, vs.slices, vs.lds, rho, oh->splitShift, cap,
-		                     repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), vs.info, scratch, vs.plan));
-	if (!readCount) return OZBLAS_STATUS_SUCCESS;
+	if (!vs.slices || !vs.info || !vs.plan) return OZBLAS_STATUS_WORKSPACE;
+	OZ_TRY(vz_begin(oh));
+	OZ_HIP(launch_vsplit(b->stream, n, x, vs.slices, vs.lds, rho, oh->splitShift, cap, repro_slot(oh) ? 0 : 1,
+	                     Prec<T>::Jsplit(b), vs.info, b->vz, vs.plan, b->vzPar[0]));
+	b->vzPar[0] ^= 1;
 	OZ_HIP(hipMemcpyAsync(b->hPinned, vs.info, sizeof(int), hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
+	b->vzDirty = false;
 	vs.count = ((int32_t *)b->hPinned)[0];
 	return OZBLAS_STATUS_SUCCESS;
 }
@@ -1005,11 +1004,11 @@ static int32_t dot_impl(ozblasHandle_t *oh, int n, const T *x, const T *y, T *re
 	const bool dot2 = (oh->splitEpsMode == 2);
 	VecSplit xs, ys;
 	if (dot2) {
-		OZ_TRY(vec_split(oh, n, x, xs, true, false));
+		OZ_TRY(vec_split(oh, n, x, xs));
 		if (y == x)
 			ys = xs;
 		else
-			OZ_TRY(vec_split(oh, n, y, ys, true, false));
+			OZ_TRY(vec_split(oh, n, y, ys));
 		T *dres = (T *)walloc(oh, 8);
 		if (!dres) return OZBLAS_STATUS_WORKSPACE;
 		OZ_HIP(hipMemsetAsync(dres, 0, 8, b->stream));
@@ -1301,6 +1300,8 @@ extern "C" int32_t ozblasDdot(ozblasHandle_t *oh, int32_t n, const double *x, in
 
 // Bytes the binary64 DOT takes from the workspace: the bump allocations of dot_impl / vec_split in
 // their order (256-byte aligned), with the Dot2 buffers at the largest slice counts.
+constexpr uint64_t kNoAllocScratch = 24064;  // a vector's zeroed scratch: the handle's own (Backend::vz), but
+                                             // counted, so that the limit on n is the documented one
 static uint64_t dot_workspace_bytes(const ozblasHandle_t *oh, int n, bool same) {
 	auto bump = [](uint64_t top, uint64_t bytes) { return ((top + 255) & ~uint64_t(255)) + bytes; };
 	const int cap = split_cap(oh);
@@ -1310,7 +1311,7 @@ static uint64_t dot_workspace_bytes(const ozblasHandle_t *oh, int n, bool same) 
 		for (int v = 0; v < (same ? 1 : 2); v++) {
 			t = bump(t, 8ull * lds * (cap + 2));  // slices
 			t = bump(t, 16);                      // count
-			t = bump(t, vsplit_scratch_bytes());
+			t = bump(t, kNoAllocScratch);
 			t = bump(t, sizeof(VsPlan));
 		}
 		t = bump(t, 8);  // result
@@ -1318,11 +1319,9 @@ static uint64_t dot_workspace_bytes(const ozblasHandle_t *oh, int n, bool same) 
 		t = bump(t, dot2_partials_bytes(cap + 2, cap + 2));
 		return t;
 	}
-	// counts, pair sums and the partials, then per vector (the zeroed scratch, once part of this, is the
-	// handle's own now; its bytes still count, so that the limit on n is the documented one)
-	const uint64_t sb = (uint64_t)rup((int64_t)vsplit_scratch_bytes(), 256);
+	// counts, pair sums and the partials, then per vector
 	const uint64_t vb = (uint64_t)rup(8ll * (cap + 1) * (cap + 1), 256);
-	t = bump(t, 2 * sb + vb + 48);
+	t = bump(t, 2 * kNoAllocScratch + vb + 48);
 	t = bump(t, dots_part_bytes());
 	for (int v = 0; v < (same ? 1 : 2); v++) {
 		t = bump(t, 8ull * lds * (cap + 2));  // slices (stored for a plan outside the model)
@@ -1458,37 +1457,45 @@ static int32_t csrmv_impl(ozblasHandle_t *oh, int m, int n, int nnz, T alpha, co
 	}
 	oh->splitShift = 1;  // the vector split always uses splitShift = 1 (counterInit)
 	VecSplit xs;
-	if constexpr (sizeof(T) == 8) {
-		// binary64: the product generates x's slices from its plan (k_csrmv_plan), no stored slices and
-		// no count read back before it; a vector of more slices than its registers hold goes on below
-		const bool fsum = oh->sumMode == 0;
-		if (oh->splitEpsMode != 2 && as.count <= 4 && !(fsum && oh->fastMode) && !(b->mixed && !fsum)) {
-			const int cap = split_cap(oh);
-			int *out = (int *)b->hPinned;
-			xs.x = x;
-			xs.lds = rup(n, 32);
-			xs.slices = (double *)walloc(oh, 8ull * xs.lds * (cap + 2));
-			xs.info = (int *)walloc(oh, 16);
-			xs.plan = (VsPlan *)walloc(oh, sizeof(VsPlan));
-			if (!xs.slices || !xs.info || !xs.plan) return OZBLAS_STATUS_WORKSPACE;
-			OZ_TRY(vz_begin(oh));
-			OZ_HIP(launch_vsplit_plan(b->stream, n, x, xs.slices, xs.lds, Prec<T>::rho(oh, n), oh->splitShift, cap,
-			                          repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), xs.info, b->vz, nullptr, xs.plan,
-			                          false, nullptr, 0, -1, b->vzPar[0]));
-			b->vzPar[0] ^= 1;
+	// the product generates x's slices from its plan (k_csrmv_plan): no stored slices and no count read back
+	// before it; a vector of more slices than its registers hold goes on below
+	const bool fsum = oh->sumMode == 0;
+	if (oh->splitEpsMode != 2 && as.count <= 4 && !(fsum && oh->fastMode) && !(b->mixed && !fsum)) {
+		const int cap = split_cap(oh);
+		int *out = (int *)b->hPinned;
+		const uint64_t mark = wmark(oh);
+		xs.x = x;
+		xs.lds = rup(n, 32);
+		xs.slices = (double *)walloc(oh, 8ull * xs.lds * (cap + 2));
+		xs.info = (int *)walloc(oh, 16);
+		xs.plan = (VsPlan *)walloc(oh, sizeof(VsPlan));
+		if (!xs.slices || !xs.info || !xs.plan) return OZBLAS_STATUS_WORKSPACE;
+		const int64_t ldc = rup(m, 8);
+		T *Cs = nullptr;
+		if constexpr (sizeof(T) == 4)
+			if (wide_vector(oh, n)) Cs = (T *)walloc(oh, sizeof(T) * ldc * as.count * kCsrWideSlices);
+		OZ_TRY(vz_begin(oh));
+		OZ_HIP(launch_vsplit_plan(b->stream, n, x, xs.slices, xs.lds, Prec<T>::rho(oh, n), oh->splitShift, cap,
+		                          repro_slot(oh) ? 0 : 1, Prec<T>::Jsplit(b), xs.info, b->vz, nullptr, xs.plan,
+		                          false, nullptr, 0, -1, b->vzPar[0]));
+		b->vzPar[0] ^= 1;
+		if constexpr (sizeof(T) == 4)
+			launch_csrmv_plan(b->stream, m, as.slices, as.lds, as.count, colind, rowptr, xs.ref(), oh->fastMode,
+			                  fsum ? 1 : 0, alpha, beta, y, Prec<T>::Jsum(b), out, b->mixed, Cs, ldc);
+		else
 			launch_csrmv_plan(b->stream, m, as.slices, as.lds, as.count, colind, rowptr, xs.ref(), oh->fastMode,
 			                  fsum ? 1 : 0, alpha, beta, y, Prec<T>::Jsum(b), out);
-			OZ_HIP(hipGetLastError());
-			OZ_TRY(sync(oh));
-			b->vzDirty = false;
-			if (!out[1]) {
-				oh->nSplitA = (float)as.count;
-				oh->nSplitB = (float)out[0];
-				wreset(oh, base);
-				return OZBLAS_STATUS_SUCCESS;
-			}
-			xs = VecSplit();
+		OZ_HIP(hipGetLastError());
+		OZ_TRY(sync(oh));
+		b->vzDirty = false;
+		if (!out[1]) {
+			oh->nSplitA = (float)as.count;
+			oh->nSplitB = (float)out[0];
+			wreset(oh, base);
+			return OZBLAS_STATUS_SUCCESS;
 		}
+		xs = VecSplit();
+		wreset(oh, mark);
 	}
 	OZ_TRY(vec_split(oh, n, x, xs));
 	OZ_TRY(csrmv_core(oh, m, n, nnz, alpha, as, colind, rowptr, xs, beta, y));
@@ -1662,7 +1669,7 @@ static int32_t cg_host_loop(ozblasHandle_t *oh, int n, int nnz, const double *AS
 
 // Device-resident iterations; *overflow = 1 when the host path must redo them.
 // T = float: the <float,float> solve with binary32 vectors and recurrences; p's slices are capped
-// at the CSR kernel's register bound (more overflow to the synchronous path).
+// at the CSR kernel's register bound, 8 or 32 (more overflow to the synchronous path).
 template <class T>
 static int32_t cg_device_loop(ozblasHandle_t *oh, int n, int nA, const double *AS, const int *colind,
                               const int *rowptr, T *x, int maxiter, T tol, T nrmb, T dold,
@@ -1701,9 +1708,20 @@ static int32_t cg_device_loop(ozblasHandle_t *oh, int n, int nA, const double *A
 	double *part = (double *)walloc(oh, dots_part_bytes());
 	if (!vscr || !plans || !pres || !part) return OZBLAS_STATUS_WORKSPACE;
 	int maxVec = (oh->cgDeviceSlices > 0 && oh->cgDeviceSlices < cap) ? oh->cgDeviceSlices : cap;
-	if (f32 && maxVec > 8) maxVec = 8;  // the binary32 product has no per-pair row loop
 	const int64_t ldc = rup(n, 32);
-	double *Cs = (double *)walloc(oh, 8ull * ldc * nA * maxVec);  // pair sums of the general product
+	// pair sums of the general product; binary32: of a vector of more than 8 slices (kCsrWideSlices at
+	// most), for which fewer slices serve where the workspace does not hold them
+	double *Cs = nullptr;
+	bool wide = false;
+	if constexpr (f32) {
+		if (wide_vector(oh, n) && maxVec > kCsrPlanSlices) {
+			maxVec = imin(maxVec, kCsrWideSlices);
+			Cs = (double *)walloc(oh, sizeof(T) * ldc * nA * kCsrWideSlices);
+			wide = Cs != nullptr;
+		}
+		if (!wide) maxVec = imin(maxVec, kCsrPlanSlices);
+	}
+	if (!wide) Cs = (double *)walloc(oh, 8ull * ldc * nA * maxVec);
 	if (!slP || !slQ || !slR || !sm || !S || !Cs) return OZBLAS_STATUS_WORKSPACE;
 	double *vals = (double *)sm;
 	int *info = (int *)(vals + (cap + 1) * (cap + 1));  // P, Q, R: two ints each
@@ -1742,7 +1760,7 @@ static int32_t cg_device_loop(ozblasHandle_t *oh, int n, int nA, const double *A
 		                          it > 0, S, it, kClkSpmv, par));
 		if constexpr (sizeof(T) == 4)
 			launch_csrmm_sum_dev(st, n, AS, rup(b->nnzA, 32), nA, colind, rowptr, refP, fsum, v.Q, Cs, ldc, Jn, S,
-			                     it, preQ + par, b->mixed);
+			                     it, preQ + par, b->mixed, wide ? 1 : 0);
 		else
 			launch_csrmm_sum_dev(st, n, AS, rup(b->nnzA, 32), nA, colind, rowptr, refP, fsum, v.Q, Cs, ldc, Jn, S,
 			                     it, preQ + par);

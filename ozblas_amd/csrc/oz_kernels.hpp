@@ -247,7 +247,11 @@ struct VsPlan {
 // Per-vector reductions of the predicted level chain (zero between uses: the kernel that consumes
 // them clears them).  A kernel that produces the vector may accumulate maxBits / loOff / bad itself
 // (vs_stats_* in oz_level12.hip), so that the split does not read the vector for them again.
-constexpr int kVsPred = 12;     // predicted levels evaluated at most
+// predicted levels evaluated at most: a long binary32 vector has slices of one or two bits, up to the
+// split's cap of 30
+constexpr int kVsPred = 32;
+template <class TI>
+constexpr int vs_pred_levels() { return sizeof(TI) == 4 ? kVsPred : 12; }
 constexpr int kVsLoOff = 4096;  // min lo is kept as the maximum of kVsLoOff - lo
 constexpr int kVsSpread = 16;   // workgroup b reduces into slot b % kVsSpread (one cache line each)
 struct alignas(128) VsSlot {
@@ -268,11 +272,11 @@ size_t vz_bytes();
 // Splits x into slices at stride lds (cap + 2 slots) and its plan; the count goes to info[0].
 hipError_t launch_vsplit(hipStream_t st, int n, const double *x, double *slices, int64_t lds,
                          int rho, int shift, int cap, int reproMode, const uint16_t *J, int *info,
-                         void *scratch, VsPlan *plan);
+                         void *scratch, VsPlan *plan, int parity);
 // binary32 input (JF: the binary32 tau table); slices are stored as doubles
 hipError_t launch_vsplit(hipStream_t st, int n, const float *x, double *slices, int64_t lds,
                          int rho, int shift, int cap, int reproMode, const uint16_t *JF, int *info,
-                         void *scratch, VsPlan *plan);
+                         void *scratch, VsPlan *plan, int parity);
 // The plan only: consumers that take (x, plan) generate the slices themselves; the slices are
 // stored only for a plan marked bad (the reference loop in one workgroup).  pre: a pair of VsPre
 // for the vector (zero at first); this split reads pre[parity] (holding the producer's reductions
@@ -345,16 +349,21 @@ void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas,
                           double *Cs, int64_t ldc, const uint16_t *J, CgDev *S, int it, VsPre *preY);
 // y = alpha A x + beta y with x's plan (binary64; slices of A pre-split, nA <= 4): more than
 // kCsrPlanSlices slices of x leave y untouched; out (host memory): x's count, then 1 in that case
-constexpr int kCsrPlanSlices = 8;
+// (binary32: with Cs, pair sums of a row at pitch ldc, up to kCsrWideSlices; mixed = 1: binary64 chains)
+constexpr int kCsrPlanSlices = 8, kCsrWideSlices = 32;
+void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
+                       const int *rowptr, VsRef X, int fastMode, int fsum, float alpha, float beta, float *y,
+                       const uint16_t *JF2, int *out, int mixed, float *Cs, int64_t ldc);
 void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
                        const int *rowptr, VsRef X, int fastMode, int fsum, double alpha, double beta, double *y,
                        const uint16_t *J, int *out);
-// binary32 p and q (JF2: the binary32 NearSum table); p's slices capped at 8 by maxVecSlices;
+// binary32 p and q (JF2: the binary32 NearSum table); p's slices capped at 8, or 32 with wide, by
+// maxVecSlices (the caller's choice by the slices a vector of its length takes);
 // mixed = 1: binary64 pair chains (<float,double>)
 void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA,
                           const int *colind, const int *rowptr, VsRef X, int fsum, float *y,
                           double *Cs, int64_t ldc, const uint16_t *JF2, CgDev *S, int it, VsPre *preY,
-                          int mixed = 0);
+                          int mixed = 0, int wide = 0);
 // part: dots_part_bytes() of scratch for the per-workgroup pair partials (no initial value)
 size_t dots_part_bytes();
 // DOT of two split vectors (binary32 inputs with f32), completed by `mode` (0: C[0] = the DOT, and the

@@ -552,7 +552,7 @@ __device__ inline void vs_predict(double M0, int minLo, int rho, int cap, const 
 	d = SplitRule<TI>::kPrec - rho + 1;
 	L = (d > 0 && k0 >= minLo) ? (k0 - minLo) / d + 2 : 1;
 	if (L > cap) L = cap;
-	if (L > kVsPred) L = kVsPred;
+	if (L > vs_pred_levels<TI>()) L = vs_pred_levels<TI>();
 }
 
 constexpr int kVsLevBlocks = 1024;  // workgroups of the reduction kernels at most
@@ -591,7 +591,7 @@ __device__ int vs_verify(unsigned long long mb, int lof, int bad, const unsigned
 	if (bad || M0 == 0.0 || rho < 3 || rho > SplitRule<TI>::kPrec || cap > kVsMaxLevels) return 1;
 	int k0, d, L;
 	vs_predict<TI>(M0, kVsLoOff - lof, rho, cap, J, k0, d, L);
-	int ks[kVsPred];
+	int ks[vs_pred_levels<TI>()];
 	double M = M0;
 	int s = 0;
 	bool zero = false;
@@ -618,7 +618,7 @@ __device__ int vs_verify(unsigned long long mb, int lof, int bad, const unsigned
 		count = cap;
 	if (reproMode == 0) count++;
 	const int last = zero ? s : cap - 1;
-	for (int q = 0; q <= last && q < kVsPred; q++) plan->k[q] = ks[q];
+	for (int q = 0; q <= last && q < vs_pred_levels<TI>(); q++) plan->k[q] = ks[q];
 	plan->needScan = 0;
 	plan->bad = 0;
 	plan->count = count;
@@ -669,9 +669,10 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 		// The residues by the split's own recurrence over the predicted units (remainder after level q
 		// = cmod(x, 2^(k0 - d q)), as in VsGen): four instructions a level.  A sigma outside the normal
 		// range makes the levels from there on meaningless; the walk rejects the chain at that level.
-		TI sig[kVsPred], Fm[kVsPred];
+		constexpr int NP = vs_pred_levels<TI>();
+		TI sig[NP], Fm[NP];
 #pragma unroll
-		for (int q = 0; q < kVsPred; q++) {
+		for (int q = 0; q < NP; q++) {
 			sig[q] = vs_sigma<TI>(k0 - d * q);
 			Fm[q] = 0;
 		}
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 				v[e] = ie < n ? xl : (TI)0;
 			}
 #pragma unroll
-			for (int q = 0; q < kVsPred; q++)
+			for (int q = 0; q < NP; q++)
 				if (q < L) {
 #pragma unroll
 					for (int e = 0; e < 4; e++) {
@@ -698,7 +699,7 @@ __global__ __launch_bounds__(BS) void k_vsplit_levels(int n, const TI *x, VsPre 
 		// one round for all levels: the waves' maxima through LDS, then a lane per level raises its counter
 		const int w = threadIdx.x / 64;
 #pragma unroll
-		for (int q = 0; q < kVsPred; q++)
+		for (int q = 0; q < NP; q++)
 			if (q < L) {  // L is uniform
 				const double f = wave_max_nonneg_f64((double)Fm[q]);
 				if (threadIdx.x % 64 == 0) red[w][q] = f;
@@ -895,9 +896,9 @@ static hipError_t vsplit_plan(hipStream_t st, int n, const TI *x, double *slices
 template <class TI>
 static hipError_t vsplit(hipStream_t st, int n, const TI *x, double *slices, int64_t lds, int rho,
                          int shift, int cap, int reproMode, const uint16_t *J, int *info, void *scratch,
-                         VsPlan *plan) {
+                         VsPlan *plan, int parity) {
 	const hipError_t e = vsplit_plan(st, n, x, slices, lds, rho, shift, cap, reproMode, J, info, scratch,
-	                                 nullptr, plan, false, nullptr, 0, kClkNone, 0, 0);
+	                                 nullptr, plan, false, nullptr, 0, kClkNone, 0, parity);
 	if (e != hipSuccess) return e;
 	int gw = (int)std::min<int64_t>(2048, ((int64_t)n + 255) / 256);
 	if (gw < 1) gw = 1;
@@ -908,14 +909,14 @@ static hipError_t vsplit(hipStream_t st, int n, const TI *x, double *slices, int
 
 hipError_t launch_vsplit(hipStream_t st, int n, const double *x, double *slices, int64_t lds, int rho,
                          int shift, int cap, int reproMode, const uint16_t *J, int *info, void *scratch,
-                         VsPlan *plan) {
-	return vsplit(st, n, x, slices, lds, rho, shift, cap, reproMode, J, info, scratch, plan);
+                         VsPlan *plan, int parity) {
+	return vsplit(st, n, x, slices, lds, rho, shift, cap, reproMode, J, info, scratch, plan, parity);
 }
 
 hipError_t launch_vsplit(hipStream_t st, int n, const float *x, double *slices, int64_t lds, int rho,
                          int shift, int cap, int reproMode, const uint16_t *JF, int *info, void *scratch,
-                         VsPlan *plan) {
-	return vsplit(st, n, x, slices, lds, rho, shift, cap, reproMode, JF, info, scratch, plan);
+                         VsPlan *plan, int parity) {
+	return vsplit(st, n, x, slices, lds, rho, shift, cap, reproMode, JF, info, scratch, plan, parity);
 }
 
 template <class TI>
@@ -964,6 +965,7 @@ constexpr int kDotChunk = 16;
 constexpr int kDotPairs = 64;    // pair slots per workgroup partial of k_dots_reg
 constexpr int kDotMaxWG = 512;  // workgroups of k_dots_reg at most (two waves per SIMD)
 constexpr int kDotFinBS = 1024;  // threads of the completion
+constexpr int kDotWide = 32;     // slices a side of the matrix-unit products
 
 template <int BS>
 __global__ __launch_bounds__(BS) void k_slice_dots(int n, const double *xs, int64_t ldx, int nA,
@@ -1194,10 +1196,11 @@ void launch_nearsum_small(hipStream_t st, int nvals, double *vals, double alpha,
 	                   maxlevel, fsum, J);
 }
 
-// the sum over a row's pair products (NearSum, or Fsum in level order) with ia + ib <= maxlevel
+// the sum over a row's pair products (NearSum, or Fsum in level order) with ia + ib <= maxlevel; an instance
+// of more than 32 of them takes scratch for NearSum's unsettled sums: value q of row r at Cs[q ldc + r]
 template <int NAM, int NBM, class T, class V>
 __device__ __forceinline__ T csr_pairs_sum(RegVec<NAM * NBM, V> &v, int nA, int nB, int maxlevel, int fsum,
-                                           const uint16_t *J) {
+                                           const uint16_t *J, T *Cs = nullptr, int64_t ldc = 0, int r = 0) {
 	// a pair sum as a term of the sum in T (the binary64 chain of <float,double> rounds as the
 	// reference's (float) of the scaled product)
 	auto term = [](V p) -> T {
@@ -1218,17 +1221,32 @@ __device__ __forceinline__ T csr_pairs_sum(RegVec<NAM * NBM, V> &v, int nA, int 
 			}
 	} else {
 		// NearSum over the products (its result does not depend on the order of the terms): the
-		// clear-cut case first (binary64), largest levels first
+		// clear-cut case first, largest levels first
+		SumCert c;
+#pragma unroll
+		for (int ik = 0; ik < NAM + NBM - 1; ik++)
+#pragma unroll
+			for (int ia = 0; ia < NAM; ia++) {
+				const int ib = ik - ia;
+				if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) c.add((double)term(v[ia * NBM + ib]));
+			}
 		if constexpr (sizeof(T) == 8) {
-			SumCert c;
-#pragma unroll
-			for (int ik = 0; ik < NAM + NBM - 1; ik++)
-#pragma unroll
-				for (int ia = 0; ia < NAM; ia++) {
-					const int ib = ik - ia;
-					if (ib >= 0 && ib < NBM && ia < nA && ib < nB && ik <= maxlevel) c.add(v[ia * NBM + ib]);
-				}
 			if (c.done(NAM * NBM, t)) return t;
+		} else {
+			if (c.done_f(NAM * NBM, &t)) return t;
+		}
+		if constexpr (NAM * NBM > 32) {  // through memory
+			int n = 0;
+#pragma unroll
+			for (int ia = 0; ia < NAM; ia++)
+#pragma unroll
+				for (int ib = 0; ib < NBM; ib++)
+					if (ia < nA && ib < nB && ia + ib <= maxlevel) Cs[(int64_t)(n++) * ldc + r] = term(v[ia * NBM + ib]);
+			StridedVecT<T> m{Cs + r, ldc};
+			if constexpr (sizeof(T) == 4)
+				return nearsum_f(n, m, J);
+			else
+				return nearsum(n, m, J);
 		}
 		// else compact the valid ones to the front of a register array
 		RegVec<NAM * NBM, T> u;
@@ -1344,11 +1362,11 @@ __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas
 // eighth of the rows, so that an L2 holds the part of x its rows gather.
 // ---------------------------------------------------------------------------------------------
 constexpr int kCsrRows = 256;
-template <int NAM>
+template <int NAM, class T>
 struct CsrStage {
 	static constexpr int kCap = NAM <= 2 ? 2048 : 1280;  // nonzeros: 48 KB and 50 KB, three workgroups a CU
 	double a[NAM][kCap];
-	double x[kCap];
+	T x[kCap];
 };
 
 __device__ inline int csr_block(int nb) {
@@ -1357,14 +1375,15 @@ __device__ inline int csr_block(int nb) {
 }
 
 // loads the block's nonzeros [base, base + cnt) when they fit; false (uniform) otherwise
-template <int NAM>
-__device__ __forceinline__ bool csr_stage_load(CsrStage<NAM> &st, int base, int cnt, const double *As,
-                                               int64_t ldas, int nA, const int *colind, const double *X) {
-	if (cnt > CsrStage<NAM>::kCap) return false;
-	constexpr int U = CsrStage<NAM>::kCap / kCsrRows;  // the whole stage in one round of loads
+template <int NAM, class T>
+__device__ __forceinline__ bool csr_stage_load(CsrStage<NAM, T> &st, int base, int cnt, const double *As,
+                                               int64_t ldas, int nA, const int *colind, const T *X) {
+	if (cnt > CsrStage<NAM, T>::kCap) return false;
+	constexpr int U = CsrStage<NAM, T>::kCap / kCsrRows;  // the whole stage in one round of loads
 	for (int i0 = threadIdx.x; i0 < cnt; i0 += U * kCsrRows) {
 		int c[U];
-		double a[U][NAM], x[U];
+		double a[U][NAM];
+		T x[U];
 #pragma unroll
 		for (int u = 0; u < U; u++) {  // unconditional loads at clamped indices, all in flight
 			const int i = base + min(i0 + u * kCsrRows, cnt - 1);
@@ -1388,81 +1407,152 @@ __device__ __forceinline__ bool csr_stage_load(CsrStage<NAM> &st, int base, int 
 	return true;
 }
 
-// the row with staged nonzeros [b, e): nA x nB pair sums in row order, then their sum
-template <int NAM, int NBM>
-__device__ __forceinline__ double csr_stage_row(const CsrStage<NAM> &st, int b, int e, int nA, int nB, int maxlevel,
-                                                int fsum, const uint16_t *J, const VsPlan *plan) {
-	double sig[NBM];
+// the row with staged nonzeros [b, e): nA x nB pair sums in row order (the chains of csrmm_row_sum), then
+// their sum
+template <int NAM, int NBM, class T, class V>
+__device__ __forceinline__ T csr_stage_row(const CsrStage<NAM, T> &st, int b, int e, int nA, int nB, int maxlevel,
+                                           int fsum, const uint16_t *J, const VsPlan *plan, T *Cs, int64_t ldc,
+                                           int row) {
+	T sig[NBM];
 	const int last = plan->last;
 #pragma unroll
-	for (int q = 0; q < NBM; q++) sig[q] = (q <= last) ? vs_sigma<double>(plan->k[q]) : 0.0;
-	RegVec<NAM * NBM, double> v;
+	for (int q = 0; q < NBM; q++) sig[q] = (q <= last) ? vs_sigma<T>(plan->k[q]) : (T)0;
+	RegVec<NAM * NBM, V> v;
 #pragma unroll
-	for (int q = 0; q < NAM * NBM; q++) v[q] = 0.0;
+	for (int q = 0; q < NAM * NBM; q++) v[q] = (V)0;
 	for (int j = b; j < e; j++) {
-		double r = st.x[j], a[NAM];
+		T r = st.x[j];
+		double a[NAM];
 #pragma unroll
 		for (int ia = 0; ia < NAM; ia++) a[ia] = st.a[ia][j];
 #pragma unroll
 		for (int ib = 0; ib < NBM; ib++)
 			if (ib < nB) {  // uniform
-				const double x = (r + sig[ib]) - sig[ib];  // VsGen's step
+				const T x = (r + sig[ib]) - sig[ib];  // VsGen's step
 				r = r - x;
 #pragma unroll
-				for (int ia = 0; ia < NAM; ia++) v[ia * NBM + ib] = fma(a[ia], x, v[ia * NBM + ib]);
+				for (int ia = 0; ia < NAM; ia++)
+					v[ia * NBM + ib] = (V)fma(a[ia], (double)x, (double)v[ia * NBM + ib]);
 			}
 	}
-	return csr_pairs_sum<NAM, NBM, double, double>(v, nA, nB, maxlevel, fsum, J);
+	return csr_pairs_sum<NAM, NBM, T, V>(v, nA, nB, maxlevel, fsum, J, Cs, ldc, row);
+}
+
+// a row in memory, one pair at a time: each pair sum runs over the row's nonzeros in order, then NearSum over
+// the pairs through Cs[q ldc + r], or Fsum in (level, ia) order computed on the fly -- for the rows and
+// vectors the register kernels do not take (stored slices, long rows, more slices than registers)
+template <class T, class V>
+__device__ inline T csr_big_row(int r, const double *As, int64_t ldas, int nA, const int *colind,
+                                const int *rowptr, const VsRef &X, int nB, int maxlevel, int fsum, T *Cs, int64_t ldc,
+                                const uint16_t *J) {
+	const bool stored = X.plan->bad;
+	const T *Xv = (const T *)X.x;
+	const int b = rowptr[r], e = rowptr[r + 1];
+	auto pair = [&](int ia, int ib) {
+		V acc = (V)0;
+		for (int j = b; j < e; j++) {
+			const double xv = stored ? X.slices[(int64_t)ib * X.lds + colind[j]] : vs_slot<T>(Xv[colind[j]], X.plan, ib);
+			acc = (V)fma(As[(int64_t)ia * ldas + j], xv, (double)acc);
+		}
+		if constexpr (sizeof(V) == sizeof(T))
+			return acc;
+		else
+			return sum_term<T>(acc);
+	};
+	if (fsum) {
+		T t = (T)0;
+		for (int ik = 0; ik <= maxlevel; ik++)
+			for (int ia = 0; ia < nA; ia++) {
+				const int ib = ik - ia;
+				if (ib >= 0 && ib < nB) t = t + pair(ia, ib);
+			}
+		return t;
+	}
+	int cnt = 0;
+	for (int ia = 0; ia < nA; ia++)
+		for (int ib = 0; ib < nB; ib++)
+			if (ia + ib <= maxlevel) Cs[(int64_t)(cnt++) * ldc + r] = pair(ia, ib);
+	StridedVecT<T> v{Cs + r, ldc};
+	if constexpr (sizeof(T) == 4)
+		return nearsum_f(cnt, v, J);
+	else
+		return nearsum(cnt, v, J);
 }
 
 // y = alpha A x + beta y from the slices of A and x's plan (ozblasRcsrmv).  out (host memory): x's slice
 // count, and 1 in out[1] when it exceeds the register bound NBM -- then y is untouched and the caller
 // takes the stored slices.
-template <int NAM, int NBM>
+template <int NAM, int NBM, class T, class V>
 __global__ __launch_bounds__(kCsrRows) void k_csrmv_plan(int m, const double *As, int64_t ldas, int nA,
                                                         const int *colind, const int *rowptr, VsRef X,
-                                                        int fastMode, int fsum, double alpha, double beta,
-                                                        double *y, const uint16_t *J, int *out) {
+                                                        int fastMode, int fsum, T alpha, T beta, T *y, T *Cs,
+                                                        int64_t ldc, const uint16_t *J, int *out) {
 	const int nB = X.info[0];
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		out[0] = nB;
 		out[1] = nB > NBM ? 1 : 0;
 	}
 	if (nB > NBM) return;
-	__shared__ CsrStage<NAM> st;
+	__shared__ CsrStage<NAM, T> st;
 	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
 	if (r0 >= m) return;
 	const int rows = min(kCsrRows, m - r0);
 	const int base = rowptr[r0], cnt = rowptr[r0 + rows] - base;
 	const int maxlevel = max((nA - 1) + (nB - 1) - fastMode, min(nA - 1, nB - 1));
-	const bool staged = !X.plan->bad && csr_stage_load<NAM>(st, base, cnt, As, ldas, nA, colind, (const double *)X.x);
+	const bool staged = !X.plan->bad && csr_stage_load<NAM, T>(st, base, cnt, As, ldas, nA, colind, (const T *)X.x);
 	const int r = r0 + (int)threadIdx.x;
 	if (r >= m) return;
-	double t;
+	T t;
 	if (staged) {
-		t = csr_stage_row<NAM, NBM>(st, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J, X.plan);
+		t = csr_stage_row<NAM, NBM, T, V>(st, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J, X.plan,
+		                                  Cs, ldc, r);
+	} else if constexpr (NBM > kCsrPlanSlices) {
+		t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Cs, ldc, J);
 	} else if (X.plan->bad) {
-		t = csrmm_row_sum<NAM, NBM>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel, fsum, J);
+		t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel,
+		                                                 fsum, J);
 	} else {
-		VsGen<double, NBM> g;
+		VsGen<T, NBM> g;
 		g.init(X.plan);
-		t = csrmm_row_sum<NAM, NBM, double, double, true>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel,
-		                                                  fsum, J, (const double *)X.x, &g);
+		t = csrmm_row_sum<NAM, NBM, T, T, true, V>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel, fsum, J,
+		                                           (const T *)X.x, &g);
 	}
-	y[r] = fma(alpha, t, beta * y[r]);
+	y[r] = fma1_t(alpha, t, beta * y[r]);
+}
+
+template <int NBM, class T, class V>
+static void csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
+                       const int *rowptr, VsRef X, int fastMode, int fsum, T alpha, T beta, T *y, T *Cs, int64_t ldc,
+                       const uint16_t *J, int *out) {
+	const int nb = (m + kCsrRows - 1) / kCsrRows;
+	const dim3 g(8 * ((nb + 7) / 8));
+	if (nA <= 2)
+		hipLaunchKernelGGL((k_csrmv_plan<2, NBM, T, V>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr, X,
+		                   fastMode, fsum, alpha, beta, y, Cs, ldc, J, out);
+	else
+		hipLaunchKernelGGL((k_csrmv_plan<4, NBM, T, V>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr, X,
+		                   fastMode, fsum, alpha, beta, y, Cs, ldc, J, out);
 }
 
 void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
                        const int *rowptr, VsRef X, int fastMode, int fsum, double alpha, double beta, double *y,
                        const uint16_t *J, int *out) {
-	const int nb = (m + kCsrRows - 1) / kCsrRows;
-	const dim3 g(8 * ((nb + 7) / 8));
-	if (nA <= 2)
-		hipLaunchKernelGGL((k_csrmv_plan<2, kCsrPlanSlices>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr,
-		                   X, fastMode, fsum, alpha, beta, y, J, out);
+	csrmv_plan<kCsrPlanSlices, double, double>(st, m, As, ldas, nA, colind, rowptr, X, fastMode, fsum, alpha, beta, y,
+	                                           nullptr, 0, J, out);
+}
+
+void launch_csrmv_plan(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
+                       const int *rowptr, VsRef X, int fastMode, int fsum, float alpha, float beta, float *y,
+                       const uint16_t *JF2, int *out, int mixed, float *Cs, int64_t ldc) {
+	if (mixed)
+		csrmv_plan<kCsrPlanSlices, float, double>(st, m, As, ldas, nA, colind, rowptr, X, fastMode, fsum, alpha, beta, y,
+		                                          nullptr, 0, JF2, out);
+	else if (Cs)
+		csrmv_plan<kCsrWideSlices, float, float>(st, m, As, ldas, nA, colind, rowptr, X, fastMode, fsum, alpha, beta, y,
+		                                         Cs, ldc, JF2, out);
 	else
-		hipLaunchKernelGGL((k_csrmv_plan<4, kCsrPlanSlices>), g, dim3(kCsrRows), 0, st, m, As, ldas, nA, colind, rowptr,
-		                   X, fastMode, fsum, alpha, beta, y, J, out);
+		csrmv_plan<kCsrPlanSlices, float, float>(st, m, As, ldas, nA, colind, rowptr, X, fastMode, fsum, alpha, beta, y,
+		                                         nullptr, 0, JF2, out);
 }
 
 template <int NAM, int NBM, class T, class V = T>
@@ -2026,47 +2116,10 @@ void launch_scal_axpy(hipStream_t st, int n, float beta, const float *r, float *
 // ---------------------------------------------------------------------------------------------
 __device__ inline bool cg_skip(const CgDev *S, int it) { return S != nullptr && it >= S->stopAt; }
 
-// the row sum of the product when p has more slices than the register kernel holds: each pair
-// sum runs over the row's nonzeros in order (exact) into Cs[q * ldc + r], then NearSum over the
-// row's pairs, or Fsum in (level, ia) order computed on the fly
-__device__ inline double csrmm_big_row(int r, const double *As, int64_t ldas, int nA, const int *colind,
-                                       const int *rowptr, const VsRef &X, int nB, int fsum, double *Cs,
-                                       int64_t ldc, const uint16_t *J) {
-	const bool stored = X.plan->bad;
-	const double *Xv = (const double *)X.x;
-	const int b = rowptr[r], e = rowptr[r + 1];
-	auto pair = [&](int ia, int ib) {
-		double acc = 0.0;
-		for (int j = b; j < e; j++) {
-			const double xv = stored ? X.slices[(int64_t)ib * X.lds + colind[j]]
-			                         : vs_slot<double>(Xv[colind[j]], X.plan, ib);
-			acc = fma(As[(int64_t)ia * ldas + j], xv, acc);
-		}
-		return acc;
-	};
-	const int maxlevel = (nA - 1) + (nB - 1);
-	double t;
-	if (fsum) {
-		t = 0.;
-		for (int ik = 0; ik <= maxlevel; ik++)
-			for (int ia = 0; ia < nA; ia++) {
-				const int ib = ik - ia;
-				if (ib >= 0 && ib < nB) t = t + pair(ia, ib);
-			}
-	} else {
-		int cnt = 0;
-		for (int ia = 0; ia < nA; ia++)
-			for (int ib = 0; ib < nB; ib++) Cs[(int64_t)(cnt++) * ldc + r] = pair(ia, ib);
-		StridedVec v{Cs + r, ldc};
-		t = nearsum(cnt, v, J);
-	}
-	return t;
-}
-
 // q = A p with the pre-split matrix (nA <= NAM) and the device slice count of p; alpha = 1, beta = 0
 // as ozblasRcsrmv(..., 1., ..., 0., q) at src/cpu/ozblas_cg.cpp:82.  p's slices come from p and its
 // plan (or its stored slices when the plan is marked bad); more than NBM of them take the
-// per-pair row loop (csrmm_big_row, pair sums through Cs: m x nA x maxVecSlices doubles at pitch
+// per-pair row loop (csr_big_row, pair sums through Cs: m x nA x maxVecSlices doubles at pitch
 // ldc).  The reductions of q's split accumulate into preY.
 // T = float: the <float,float> CG -- p, q binary32, the pair sums and NearSum in float (J = JF2); the
 // host caps p's slices at NBM for it (more overflow to the synchronous path).
@@ -2088,35 +2141,34 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 	int lo = 0, bad = 0;
 	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
 	const int r = r0 + (int)threadIdx.x;
-	// binary64 with a plan: the staged rows (csr_stage_row); uniform over the workgroup
-	constexpr bool kStage = sizeof(T) == 8;
+	// a plan: the staged rows (csr_stage_row); uniform over the workgroup
 	int base = 0;
 	bool staged = false;
-	__shared__ typename std::conditional<kStage, CsrStage<NAM>, int>::type stage;
-	if constexpr (kStage) {
-		if (r0 < m && nB <= NBM && !X.plan->bad) {
-			const int rows = min(kCsrRows, m - r0);
-			base = rowptr[r0];
-			staged = csr_stage_load<NAM>(stage, base, rowptr[r0 + rows] - base, As, ldas, nA, colind, (const double *)X.x);
-		}
+	__shared__ CsrStage<NAM, T> stage;
+	if (r0 < m && nB <= NBM && !X.plan->bad) {
+		const int rows = min(kCsrRows, m - r0);
+		base = rowptr[r0];
+		staged = csr_stage_load<NAM, T>(stage, base, rowptr[r0 + rows] - base, As, ldas, nA, colind, (const T *)X.x);
 	}
 	if (r < m) {
 		const int maxlevel = (nA - 1) + (nB - 1);
 		T t = 0;
+		T *Ct = (T *)Cs;
 		if (staged) {
-			if constexpr (kStage)
-				t = csr_stage_row<NAM, NBM>(stage, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J,
-				                            X.plan);
-		} else if (nB > NBM) {
-			if constexpr (sizeof(T) == 8) t = csrmm_big_row(r, As, ldas, nA, colind, rowptr, X, nB, fsum, Cs, ldc, J);
-		} else if (X.plan->bad) {
-			t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB,
-			                                                 maxlevel, fsum, J);
-		} else {
-			VsGen<T, NBM> g;
-			g.init(X.plan);
-			t = csrmm_row_sum<NAM, NBM, T, T, true, V>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel,
-			                                           fsum, J, (const T *)X.x, &g);
+			t = csr_stage_row<NAM, NBM, T, V>(stage, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J,
+			                                  X.plan, Ct, ldc, r);
+		} else if (nB > NBM || NBM > 8) {
+			t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Ct, ldc, J);
+		} else if constexpr (NBM <= 8) {
+			if (X.plan->bad) {
+				t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB,
+				                                                 maxlevel, fsum, J);
+			} else {
+				VsGen<T, NBM> g;
+				g.init(X.plan);
+				t = csrmm_row_sum<NAM, NBM, T, T, true, V>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel, fsum,
+				                                           J, (const T *)X.x, &g);
+			}
 		}
 		const T v = fma1_t((T)1, t, (T)0 * y[r]);
 		y[r] = v;
@@ -2137,126 +2189,270 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 // The pair dots are the per-workgroup partials part[p * kDotMaxWG + w] of k_dots_reg's nwg
 // workgroups, summed here by the whole workgroup (exact in any order), or with part == nullptr
 // the sums dots_general accumulated in vals.
+// NearSum of n values by a wave (the clear-cut case, SumCert over the lanes): true when settled, *t the
+// sum rounded to T.  A float's terms are exact in binary64; its rounding is settled when both ends of the
+// interval round to it.
+template <class T>
+__device__ inline bool sum_cert_wave(int n, const double *v, T *t) {
+	SumCert c;
+	for (int i = threadIdx.x % 64; i < n; i += 64) c.add((double)sum_term<T>(v[i]));
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1) {
+		const double s2 = __shfl_xor(c.s, o, 64), e2 = __shfl_xor(c.e, o, 64), a2 = __shfl_xor(c.a, o, 64);
+		const double s = c.s + s2, bb = s - c.s;
+		c.e = (c.e + e2) + ((c.s - (s - bb)) + (s2 - bb));
+		c.s = s;
+		c.a = c.a + a2;
+	}
+	double h;
+	if constexpr (sizeof(T) == 8) {
+		const bool ok = c.done(n + 64, h);
+		*t = h;
+		return ok;
+	} else {
+		return c.done_f(n + 64, t);
+	}
+}
+
 template <int BS>
-__device__ void dots_finish(int nA, int nB, double *vals, const double *part, int nwg, const uint16_t *J,
-                            int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
-	__shared__ double psum[kDotPairs];
+__device__ void dots_finish(int nA, int nB, double *vals, const double *part, int64_t pitch, int nwg,
+                            const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32,
+                            int *counts) {
+	__shared__ double psum[kDotWide * kDotWide];
 	const int npairs = nA * nB;
 	double *src = vals;
 	if (part) {
-		// wave w sums pair w, w + waves, ...: its partials are contiguous (pair-major), kDotMaxWG / 64 loads
-		// a lane and pair, all of a wave's pairs in flight together (the partials come from memory, so a
-		// round is a full memory latency), then one wave sum a pair
-		constexpr int NW = BS / 64, PW = (kDotPairs + NW - 1) / NW, L = kDotMaxWG / 64;
+		// wave w sums pairs w, w + waves, ...: a pair's partials are contiguous, a few loads a lane and
+		// four pairs in flight together (the partials come from memory, so a round is a full memory
+		// latency), then one wave sum a pair
+		constexpr int NW = BS / 64, PW = 4, L = kDotMaxWG / 64;
 		const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-		double v[PW];
+		for (int p0 = w; p0 < npairs; p0 += PW * NW) {  // uniform over the wave
+			double v[PW];
 #pragma unroll
-		for (int q = 0; q < PW; q++) {
-			v[q] = 0.0;
-			const int p = w + q * NW;
-			if (p < npairs) {  // uniform over the wave
-				const double *row = part + (int64_t)p * kDotMaxWG + l;
+			for (int q = 0; q < PW; q++) {
+				v[q] = 0.0;
+				const int p = p0 + q * NW;
+				if (p < npairs) {
+					const double *row = part + (int64_t)p * pitch;
 #pragma unroll
-				for (int u = 0; u < L; u++) {
-					const double a = row[64 * u];  // inside the buffer; not written beyond nwg
-					v[q] += l + 64 * u < nwg ? a : 0.0;
+					for (int u = 0; u < L; u++) {
+						const double a = row[min(l + 64 * u, nwg - 1)];
+						v[q] += l + 64 * u < nwg ? a : 0.0;
+					}
 				}
 			}
-		}
 #pragma unroll
-		for (int q = 0; q < PW; q++) {
-			const int p = w + q * NW;
-			if (p < npairs) {
-				const double t = wave_sum63_f64(v[q]);
-				if (l == 63) psum[p] = t;
+			for (int q = 0; q < PW; q++) {
+				const int p = p0 + q * NW;
+				if (p < npairs) {
+					const double t = wave_sum63_f64(v[q]);
+					if (l == 63) psum[p] = t;
+				}
 			}
 		}
 		__syncthreads();
 		src = psum;
 	}
 	const int maxlevel = (nA - 1) + (nB - 1);  // DOT forces fastMode = 0 (src/cpu/ozblas_gemm.cpp:25-28)
-	double tw = 0.0;
-	bool waveDone = false;
-	if (!f32 && !fsum && npairs <= 64) {
-		// NearSum across the lanes of wave 0 when every pair dot is finite
-		if (threadIdx.x >= 64) return;
-		const double pv = ((int)threadIdx.x < npairs) ? src[threadIdx.x] : 0.0;
-		const bool finite = __all(!(fabs(pv) > 1.7976931348623157e308) && pv == pv);
-		if (finite) {
-			// the clear-cut case, the same in every lane; else across the wave
-			SumCert c;
-			for (int q = 0; q < npairs; q++) c.add(src[q]);
-			if (!c.done(npairs, tw)) tw = nearsum_wave(npairs, pv, J);
-			waveDone = true;
+	if (threadIdx.x >= 64) return;
+	const int l = threadIdx.x;
+	double t = 0.0;
+	float tf = 0.f;
+	bool known = false;
+	if (!fsum) {
+		known = f32 ? sum_cert_wave<float>(npairs, src, &tf) : sum_cert_wave<double>(npairs, src, &t);
+		if (!known && !f32 && npairs <= 64) {
+			// NearSum across the lanes when every pair dot is finite
+			const double pv = l < npairs ? src[l] : 0.0;
+			if (__all(!(fabs(pv) > 1.7976931348623157e308) && pv == pv)) {
+				t = nearsum_wave(npairs, pv, J);
+				known = true;
+			}
 		}
+	} else if (npairs <= kDotWide * kDotWide) {
+		// Fsum: the terms into (level, ia) order, then one lane adds them in turn.  Pair (ia, ib) comes
+		// after the tri(L) - tri(L - nA) - tri(L - nB) + tri(L - nA - nB) pairs of the levels below
+		// L = ia + ib and after those of its level with a smaller ia.
+		__shared__ double ord[kDotWide * kDotWide];
+		auto tri = [](int x) { return x > 0 ? x * (x + 1) / 2 : 0; };
+		for (int p = l; p < npairs; p += 64) {
+			const int ia = p % nA, ib = p / nA, lv = ia + ib;
+			const int pos = tri(lv) - tri(lv - nA) - tri(lv - nB) + tri(lv - nA - nB) + ia - max(0, lv - nB + 1);
+			ord[pos] = f32 ? (double)f32_term(src[p]) : src[p];
+		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		if (l == 0) {
+#pragma unroll 8
+			for (int p = 0; p < npairs; p++) {
+				if (f32)
+					tf = tf + (float)ord[p];
+				else
+					t = t + ord[p];
+			}
+		}
+		known = true;
 	}
-	if (threadIdx.x != 0) return;
+	if (l != 0) return;
 	if (counts) {
 		counts[0] = nA;
 		counts[1] = nB;
 	}
-	if (f32) {
-		float *fv = vals_to_float(npairs, src);
-		const float t = dot_pairs_sum_f(npairs, fv, nA, nB, maxlevel, fsum, J);
-		if (mode == 0) {
-			*(float *)C = fma1_f(1.f, t, 0.f * 0.f);
+	if (!known) {
+		if (f32) {
+			float *fv = vals_to_float(npairs, src);
+			tf = dot_pairs_sum_f(npairs, fv, nA, nB, maxlevel, fsum, J);
 		} else {
+			t = dot_pairs_sum(npairs, src, nA, nB, maxlevel, fsum, J);
+		}
+	}
+	if (f32) {
+		const float r = fma1_f(1.f, tf, 0.f * 0.f);
+		if (mode == 0) {
+			*(float *)C = r;
+		} else if (mode == 1) {
 			// the <float,float> CG's recurrences in binary32 (the CgDev fields hold binary32 values)
-			const float r = fma1_f(1.f, t, 0.f * 0.f);
-			if (mode == 1) {
-				S->tmp = r;
-				S->alpha = (float)S->dold / r;
-			} else {
-				const float dnew = r;
-				const float resi = (float)sqrt((double)dnew);
-				const float nrmb = (float)S->nrmb, tol = (float)S->tol;
-				S->dnew = dnew;
-				S->resi = resi;
-				S->beta = dnew / (float)S->dold;
-				S->dold = dnew;
-				S->numiter = it + 1;
-				if (S->verbose > 0) {
-					if (resi / nrmb < tol || S->numiter % S->verbose == 0) {
-						if (S->hist) S->hist[S->vcnt] = resi / nrmb;
-						S->vcnt = S->vcnt + 1;
-					}
+			S->tmp = r;
+			S->alpha = (float)S->dold / r;
+		} else {
+			const float dnew = r;
+			const float resi = (float)sqrt((double)dnew);
+			const float nrmb = (float)S->nrmb, tol = (float)S->tol;
+			S->dnew = dnew;
+			S->resi = resi;
+			S->beta = dnew / (float)S->dold;
+			S->dold = dnew;
+			S->numiter = it + 1;
+			if (S->verbose > 0) {
+				if (resi / nrmb < tol || S->numiter % S->verbose == 0) {
+					if (S->hist) S->hist[S->vcnt] = resi / nrmb;
+					S->vcnt = S->vcnt + 1;
 				}
-				if (resi / nrmb < tol) S->stopAt = it + 1;
 			}
+			if (resi / nrmb < tol) S->stopAt = it + 1;
 		}
-		for (int q = 0; q < npairs; q++) vals[q] = 0.0;
-		return;
-	}
-	const double t = waveDone ? tw : dot_pairs_sum(npairs, src, nA, nB, maxlevel, fsum, J);
-	const double r = fma(1.0, t, 0.0 * 0.0);
-	if (mode == 0) {
-		*(double *)C = r;
-	} else if (mode == 1) {
-		S->tmp = r;
-		S->alpha = S->dold / r;
 	} else {
-		const double dnew = r;
-		const double resi = sqrt(dnew);
-		S->dnew = dnew;
-		S->resi = resi;
-		S->beta = dnew / S->dold;
-		S->dold = dnew;
-		S->numiter = it + 1;
-		if (S->verbose > 0) {
-			if (resi / S->nrmb < S->tol || S->numiter % S->verbose == 0) {
-				if (S->hist) S->hist[S->vcnt] = resi / S->nrmb;
-				S->vcnt = S->vcnt + 1;
+		const double r = fma(1.0, t, 0.0 * 0.0);
+		if (mode == 0) {
+			*(double *)C = r;
+		} else if (mode == 1) {
+			S->tmp = r;
+			S->alpha = S->dold / r;
+		} else {
+			const double dnew = r;
+			const double resi = sqrt(dnew);
+			S->dnew = dnew;
+			S->resi = resi;
+			S->beta = dnew / S->dold;
+			S->dold = dnew;
+			S->numiter = it + 1;
+			if (S->verbose > 0) {
+				if (resi / S->nrmb < S->tol || S->numiter % S->verbose == 0) {
+					if (S->hist) S->hist[S->vcnt] = resi / S->nrmb;
+					S->vcnt = S->vcnt + 1;
+				}
 			}
+			if (resi / S->nrmb < S->tol) S->stopAt = it + 1;
 		}
-		if (resi / S->nrmb < S->tol) S->stopAt = it + 1;
 	}
-	for (int q = 0; q < npairs; q++) vals[q] = 0.0;
+	// the general path accumulates in vals: zero again for the next use
+	if (part == nullptr)
+		for (int q = 0; q < npairs; q++) vals[q] = 0.0;
 }
 
 // slot q of element i of a split vector: generated from the plan, or read from the stored slices
 template <class TI>
 __device__ inline double vs_ref_slot(const VsRef &V, bool stored, int64_t i, int q) {
 	return stored ? V.slices[(int64_t)q * V.lds + i] : vs_slot<TI>(((const TI *)V.x)[i], V.plan, q);
+}
+
+// Two split vectors of up to 32 slices whose pair products are exact: every plan in the model, no
+// inexact remainder slot counted, and units that keep the products away from the subnormals.
+__device__ inline bool dots_wide(const VsRef &X, const VsRef &Y, int nA, int nB) {
+	if (X.plan->bad || Y.plan->bad || nA > kDotWide || nB > kDotWide) return false;
+	const int lx = X.plan->last, ly = Y.plan->last;
+	if (!(X.plan->zero || nA <= lx + 1) || !(Y.plan->zero || nB <= ly + 1)) return false;
+	const int kx = X.plan->k[lx], ky = Y.plan->k[ly];
+	return kx >= -1000 && ky >= -1000 && kx + ky >= -1000;
+}
+
+// The slice dots of two such vectors as a matrix product on v_mfma_f64_16x16x4: for 32 elements at a time
+// a wave's lower lanes generate the slices of x and its upper lanes those of y, an element a lane, into
+// LDS (rows of S + 1 doubles, no bank conflicts either way), and eight steps of four elements multiply
+// the S x 32 slices of x with those of y.  The sums are exact, so their order does not matter.  One pair
+// at a time (dots_general) regenerated both slice chains for every pair: 34 ms for the 783 pairs of two
+// binary32 vectors of 2 10^6, of 27 and 29 slices.  part: pair p = ia + nA ib of workgroup b at
+// p gridDim.x + b.
+template <int BS, int S, class TI>
+__device__ __forceinline__ void dots_mfma(int n, const VsRef &X, const VsRef &Y, int nA, int nB, double *lds,
+                                          double *part) {
+	typedef double d4v __attribute__((ext_vector_type(4)));
+	constexpr int NW = BS / 64, T = S / 16, LD = S + 1;
+	const int w = threadIdx.x / 64, l = threadIdx.x % 64, h = l / 32;
+	double *buf = lds + w * (64 * LD), *mine = buf + l * LD;
+	const TI *src = (const TI *)(h ? Y.x : X.x);
+	const VsPlan *pl = h ? Y.plan : X.plan;
+	const int cnt = h ? nB : nA, last = pl->last, most = max(nA, nB);
+	TI sig[S];
+#pragma unroll
+	for (int q = 0; q < S; q++) {
+		sig[q] = (q <= last) ? vs_sigma<TI>(pl->k[q]) : (TI)0;
+		mine[q] = 0.0;
+	}
+	d4v acc[T][T];
+#pragma unroll
+	for (int a = 0; a < T; a++)
+#pragma unroll
+		for (int b = 0; b < T; b++) acc[a][b] = d4v{0.0, 0.0, 0.0, 0.0};
+	const int64_t step = (int64_t)gridDim.x * NW * 32;
+	for (int64_t c = ((int64_t)blockIdx.x * NW + w) * 32; c < n; c += step) {
+		const int64_t i = c + l % 32;
+		TI r = src[min(i, (int64_t)n - 1)];
+		r = i < n ? r : (TI)0;
+#pragma unroll
+		for (int q = 0; q < S; q++)
+			if (q < most) {  // uniform
+				const TI a = (r + sig[q]) - sig[q];
+				mine[q] = q < cnt ? (double)a : 0.0;
+				r = r - a;
+			}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's LDS writes before its reads
+#pragma unroll
+		for (int kk = 0; kk < 8; kk++) {
+			double xa[T], yb[T];
+			const double *row = buf + (4 * kk + l / 16) * LD + l % 16;
+#pragma unroll
+			for (int t = 0; t < T; t++) {
+				xa[t] = row[16 * t];
+				yb[t] = row[32 * LD + 16 * t];
+			}
+#pragma unroll
+			for (int a = 0; a < T; a++)
+#pragma unroll
+				for (int b = 0; b < T; b++)
+					acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[a], yb[b], acc[a][b], 0, 0, 0);
+		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	}
+	// lane l, register r of a tile: slice 4 r + l / 16 of x, l % 16 of y (as in k_gemm_f64)
+	__syncthreads();
+	double *sums = lds + w * S * S;
+#pragma unroll
+	for (int a = 0; a < T; a++)
+#pragma unroll
+		for (int b = 0; b < T; b++)
+#pragma unroll
+			for (int r = 0; r < 4; r++) sums[(16 * a + 4 * r + l / 16) * S + 16 * b + l % 16] = acc[a][b][r];
+	__syncthreads();
+	for (int q = threadIdx.x; q < S * S; q += BS) {
+		const int a = q / S, b = q % S;
+		if (a < nA && b < nB) {
+			double v = lds[q];
+#pragma unroll
+			for (int k = 1; k < NW; k++) v += lds[k * S * S + q];
+			part[(int64_t)(a + nA * b) * gridDim.x + blockIdx.x] = v;
+		}
+	}
 }
 
 // The same for any slice counts (pairs in chunks of kDotChunk, exact partials added atomically to
@@ -2468,7 +2664,14 @@ __global__ __launch_bounds__(BS, 2) void k_dots_reg(int n, VsRef X, VsRef Y, dou
 	if (cg_skip(S, it)) return;
 	const int nA = X.info[0], nB = Y.info[0];
 	if (nA > NAM || nB > NBM) {
-		dots_general<BS, TI>(n, nA, nB, X, Y, vals);
+		// (the wide partials take the place of x's stored slices, which a plan in the model does not have)
+		__shared__ double lds[BS / 64 * 64 * (kDotWide + 1)];
+		if (!dots_wide(X, Y, nA, nB))
+			dots_general<BS, TI>(n, nA, nB, X, Y, vals);
+		else if (max(nA, nB) <= 16)
+			dots_mfma<BS, 16, TI>(n, X, Y, nA, nB, lds, const_cast<double *>(X.slices));
+		else
+			dots_mfma<BS, kDotWide, TI>(n, X, Y, nA, nB, lds, const_cast<double *>(X.slices));
 		return;
 	}
 	const bool storedX = X.plan->bad, storedY = Y.plan->bad;
@@ -2503,14 +2706,18 @@ __global__ __launch_bounds__(BS, 2) void k_dots_reg(int n, VsRef X, VsRef Y, dou
 // The completion of k_dots_reg in one workgroup (its nwg workgroups' partials, or the pair sums
 // the general path accumulated in vals)
 template <int BS, int NAM, int NBM>
-__global__ __launch_bounds__(BS) void k_dots_fin(int nwg, const int *infoX, const int *infoY,
-                                                 double *vals, const double *part, const uint16_t *J,
-                                                 int fsum, CgDev *S, int it, int mode, void *C, int f32,
-                                                 int *counts) {
+__global__ __launch_bounds__(BS) void k_dots_fin(int nwg, VsRef X, VsRef Y, double *vals, const double *part,
+                                                 const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C,
+                                                 int f32, int *counts) {
 	if (cg_skip(S, it)) return;
-	const int nA = infoX[0], nB = infoY[0];
-	const bool reg = nA <= NAM && nB <= NBM;
-	dots_finish<BS>(nA, nB, vals, reg ? part : nullptr, nwg, J, fsum, S, it, mode, C, f32, counts);
+	const int nA = X.info[0], nB = Y.info[0];
+	int64_t pitch = kDotMaxWG;
+	if (nA > NAM || nB > NBM) {
+		const bool wide = dots_wide(X, Y, nA, nB);
+		part = wide ? X.slices : nullptr;
+		pitch = nwg;
+	}
+	dots_finish<BS>(nA, nB, vals, part, pitch, nwg, J, fsum, S, it, mode, C, f32, counts);
 }
 
 // x = fma(alpha, p, x); r = fma(-alpha, q, r)   (src/cpu/ozblas_cg.cpp:87-88, ozblas_axpy.cpp),
@@ -2564,11 +2771,10 @@ __global__ __launch_bounds__(256) void k_scal_axpy_dev(int n, CgDev *S, int it, 
 	vs_stats_flush<256>(mx, lo, bad, preP);
 }
 
-template <class T, class V = T>
+template <int kNbReg, class T, class V = T>
 static void csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA, const int *colind,
                           const int *rowptr, VsRef X, int fsum, T *y, double *Cs, int64_t ldc, const uint16_t *J,
                           CgDev *S, int it, VsPre *preY) {
-	constexpr int kNbReg = 8;
 	const dim3 g(8 * (((m + kCsrRows - 1) / kCsrRows + 7) / 8));  // csr_block
 	if (nA <= 2)  // the matrix's count is known here; p's count only on the device
 		hipLaunchKernelGGL((k_csrmm_sum_dev<2, kNbReg, T, V>), g, dim3(kCsrRows), 0, st, m, As,
@@ -2581,17 +2787,20 @@ static void csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas,
 void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA,
                           const int *colind, const int *rowptr, VsRef X, int fsum, double *y,
                           double *Cs, int64_t ldc, const uint16_t *J, CgDev *S, int it, VsPre *preY) {
-	csrmm_sum_dev(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, J, S, it, preY);
+	csrmm_sum_dev<kCsrPlanSlices, double>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, J, S, it, preY);
 }
 
 void launch_csrmm_sum_dev(hipStream_t st, int m, const double *As, int64_t ldas, int nA,
                           const int *colind, const int *rowptr, VsRef X, int fsum, float *y,
                           double *Cs, int64_t ldc, const uint16_t *JF2, CgDev *S, int it, VsPre *preY,
-                          int mixed) {
+                          int mixed, int wide) {
 	if (mixed)
-		csrmm_sum_dev<float, double>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, JF2, S, it, preY);
+		csrmm_sum_dev<kCsrPlanSlices, float, double>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, JF2, S,
+		                                             it, preY);
+	else if (wide)
+		csrmm_sum_dev<kCsrWideSlices, float>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, JF2, S, it, preY);
 	else
-		csrmm_sum_dev<float>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, JF2, S, it, preY);
+		csrmm_sum_dev<kCsrPlanSlices, float>(st, m, As, ldas, nA, colind, rowptr, X, fsum, y, Cs, ldc, JF2, S, it, preY);
 }
 
 size_t dots_part_bytes() { return sizeof(double) * kDotPairs * kDotMaxWG; }
@@ -2599,7 +2808,7 @@ size_t dots_part_bytes() { return sizeof(double) * kDotPairs * kDotMaxWG; }
 void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, double *part,
                      const uint16_t *J, int fsum, CgDev *S, int it, int mode, void *C, int f32, int *counts) {
 	constexpr int kRA = 8, kRB = 8;
-	int gx = (n + 256 * kDotStep - 1) / (256 * kDotStep);
+	int gx = (n + 511) / 512;
 	if (gx > kDotMaxWG) gx = kDotMaxWG;
 	if (gx < 1) gx = 1;
 	if (f32)
@@ -2608,7 +2817,7 @@ void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, doub
 	else
 		hipLaunchKernelGGL((k_dots_reg<256, kRA, kRB, double>), dim3(gx), dim3(256), 0, st, n, X, Y, vals,
 		                   part, (const CgDev *)S, it);
-	hipLaunchKernelGGL((k_dots_fin<kDotFinBS, kRA, kRB>), dim3(1), dim3(kDotFinBS), 0, st, gx, X.info, Y.info, vals,
+	hipLaunchKernelGGL((k_dots_fin<kDotFinBS, kRA, kRB>), dim3(1), dim3(kDotFinBS), 0, st, gx, X, Y, vals,
 	                   (const double *)part, J, fsum, S, it, mode, C, f32, counts);
 }
 
@@ -2743,7 +2952,7 @@ __global__ __launch_bounds__(BS) void k_dot_small(int n, const TI *x, const TI *
 	}
 	__syncthreads();
 	if (threadIdx.x == 0) out[2] = 0;
-	dots_finish<BS>(cnt[0], cnt[1], vals, nullptr, 0, Jn, fsum, nullptr, 0, 0, out + 4, sizeof(TI) == 4 ? 1 : 0, out);
+	dots_finish<BS>(cnt[0], cnt[1], vals, nullptr, 0, 0, Jn, fsum, nullptr, 0, 0, out + 4, sizeof(TI) == 4 ? 1 : 0, out);
 }
 
 template <class TI>

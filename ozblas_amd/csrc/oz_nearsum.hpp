@@ -150,6 +150,15 @@ struct SumCert {
 		const bool ok = E > 123 && Ea < 1893 && (hb << 12) != 0;
 		return ok && fabs(l) + 2.0 * n * n * 0x1p-106 * a < half * (1.0 - 0x1p-20);
 	}
+	// binary32: the sum of binary32 values rounded to float, settled when an interval around h that
+	// contains it (2^-50 |h| covers l and the bound) rounds to one float inside the normal range
+	__host__ __device__ inline bool done_f(int n, float *f) const {
+		const double h = s + e;
+		const double r = fabs(h) * 0x1p-50;
+		*f = (float)h;
+		return fabs(h) > 0x1p-100 && a < 0x1p100 && n * n * 0x1p-104 * a < r * 0.25 && (float)(h - r) == *f &&
+		       (float)(h + r) == *f;
+	}
 };
 
 // ---------------------------------------------------------------------------------------------
