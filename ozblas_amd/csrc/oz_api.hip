@@ -1109,7 +1109,7 @@ static int32_t csr_split(ozblasHandle_t *oh, int m, int nnz, const T *val, const
 		if (!cs.slices) return OZBLAS_STATUS_WORKSPACE;
 	}
 	OZ_HIP(hipMemsetAsync(b->dCounters, 0, sizeof(int), b->stream));
-	launch_split_csr(b->stream, m, val, rowptr, work, cs.slices, cs.lds, oh->splitShift, cap,
+	launch_split_csr(b->stream, m, nnz, val, rowptr, work, cs.slices, cs.lds, oh->splitShift, cap,
 	                 Prec<T>::Jsplit(b), zrow, b->dCounters, oh->splitEpsMode, b->mixed);
 	OZ_HIP(hipMemcpyAsync(b->hPinned, b->dCounters, sizeof(int), hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));

@@ -1283,59 +1283,32 @@ __device__ __forceinline__ T csr_pairs_sum(RegVec<NAM * NBM, V> &v, int nA, int 
 // (float)fma(a, x, (double)v) of csrmm_n<float> (<float,float>), with V = double the binary64 chain
 // of csrmm_n<double> (<float,double>), whose sum then enters the float sum as f32_term; then
 // NearSum<float> (J = JF2) or Fsum in float.
-// With OTF the slices of x are generated from x and its plan (gen) instead of read from Xs.
-template <int NAM, int NBM, class T = double, class TI = double, bool OTF = false, class V = T>
+template <int NAM, int NBM, class T = double, class TI = double, class V = T>
 __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas, int nA,
                                            const int *colind, const int *rowptr, const double *Xs,
                                            int64_t ldxs, int nB, int maxlevel, int fsum,
-                                           const uint16_t *J, const TI *X = nullptr,
-                                           const VsGen<TI, NBM> *gen = nullptr) {
+                                           const uint16_t *J) {
 	const int b = rowptr[r], e = rowptr[r + 1];
 	RegVec<NAM * NBM, V> v;
 #pragma unroll
 	for (int q = 0; q < NAM * NBM; q++) v[q] = (V)0;
-	// nonzeros in chunks of CH: the chunk's column indices, then its A and x loads, all in flight
-	// together, then the fma chains in row order (the products of one pair stay in sequence).  With
-	// OTF every load is unconditional, at an index clamped into the row and the slice counts, and the
-	// unused values are selected away afterwards: a conditional load becomes a branch with a full
-	// memory wait behind it, which serialises the chunk.
+	// nonzeros in chunks of CH: the chunk's column indices, then its A and x loads, then the fma chains in
+	// row order (the products of one pair stay in sequence)
 	constexpr int CH = (NAM * NBM <= 16) ? 4 : 2;
 	for (int j0 = b; j0 < e; j0 += CH) {
 		int c[CH];
 		double a[CH][NAM], x[CH][NBM];
-		if constexpr (OTF) {
 #pragma unroll
-			for (int q = 0; q < CH; q++) c[q] = colind[min(j0 + q, e - 1)];
+		for (int q = 0; q < CH; q++) c[q] = (j0 + q < e) ? colind[j0 + q] : 0;
 #pragma unroll
-			for (int q = 0; q < CH; q++) {
-				const bool in = j0 + q < e;
-				const int jj = min(j0 + q, e - 1);
+		for (int q = 0; q < CH; q++) {
+			const bool in = j0 + q < e;
 #pragma unroll
-				for (int ia = 0; ia < NAM; ia++) {
-					const double av = As[(int64_t)min(ia, nA - 1) * ldas + jj];
-					a[q][ia] = (in && ia < nA) ? av : 0.0;
-				}
-				const TI xv = X[c[q]];
-				gen->gen(in ? xv : (TI)0, x[q]);
+			for (int ia = 0; ia < NAM; ia++)
+				a[q][ia] = (in && ia < nA) ? As[(int64_t)ia * ldas + j0 + q] : 0.0;
 #pragma unroll
-				for (int ib = 0; ib < NBM; ib++)
-					if (ib >= nB) x[q][ib] = 0.0;
-			}
-		} else {
-			// (the stored slices: the compiler sinks such loads into their branches whatever the
-			// source form, and this one measured fastest)
-#pragma unroll
-			for (int q = 0; q < CH; q++) c[q] = (j0 + q < e) ? colind[j0 + q] : 0;
-#pragma unroll
-			for (int q = 0; q < CH; q++) {
-				const bool in = j0 + q < e;
-#pragma unroll
-				for (int ia = 0; ia < NAM; ia++)
-					a[q][ia] = (in && ia < nA) ? As[(int64_t)ia * ldas + j0 + q] : 0.0;
-#pragma unroll
-				for (int ib = 0; ib < NBM; ib++)
-					x[q][ib] = (in && ib < nB) ? Xs[(int64_t)ib * ldxs + c[q]] : 0.0;
-			}
+			for (int ib = 0; ib < NBM; ib++)
+				x[q][ib] = (in && ib < nB) ? Xs[(int64_t)ib * ldxs + c[q]] : 0.0;
 		}
 #pragma unroll
 		for (int q = 0; q < CH; q++) {
@@ -1357,8 +1330,7 @@ __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas
 // from the plan.  Read row by row from memory, neighbouring lanes are a row apart (7 nonzeros of a
 // stencil), so every cache line was fetched by seven instructions, and each row's chain of column index
 // and gather was a memory latency of its own: 59 us for the 100^3 Laplacian with 2 slices of A and 4 of x
-// at 426 VALU instructions a wave.  A block with more nonzeros than the stage holds takes the row walk
-// in memory.  Workgroups of one XCD (consecutive ones go to the 8 XCDs in turn) take one contiguous
+// at 426 VALU instructions a wave.  A longer range passes through the stage in parts.  Workgroups of one XCD (consecutive ones go to the 8 XCDs in turn) take one contiguous
 // eighth of the rows, so that an L2 holds the part of x its rows gather.
 // ---------------------------------------------------------------------------------------------
 constexpr int kCsrRows = 256;
@@ -1374,45 +1346,45 @@ __device__ inline int csr_block(int nb) {
 	return ((int)blockIdx.x % 8) * chunk + (int)blockIdx.x / 8;  // may be nb or more (grid 8 chunk)
 }
 
-// loads the block's nonzeros [base, base + cnt) when they fit; false (uniform) otherwise
+// nonzeros [c0, c1) of the workgroup's range into the stage (c1 - c0 <= kCap)
 template <int NAM, class T>
-__device__ __forceinline__ bool csr_stage_load(CsrStage<NAM, T> &st, int base, int cnt, const double *As,
-                                               int64_t ldas, int nA, const int *colind, const T *X) {
-	if (cnt > CsrStage<NAM, T>::kCap) return false;
+__device__ __forceinline__ void csr_stage_load(CsrStage<NAM, T> &st, int c0, int c1, const double *As, int64_t ldas,
+                                               int nA, const int *colind, const T *X) {
 	constexpr int U = CsrStage<NAM, T>::kCap / kCsrRows;  // the whole stage in one round of loads
-	for (int i0 = threadIdx.x; i0 < cnt; i0 += U * kCsrRows) {
-		int c[U];
-		double a[U][NAM];
-		T x[U];
+	int c[U];
+	double a[U][NAM];
+	T x[U];
+	const int t = threadIdx.x;
 #pragma unroll
-		for (int u = 0; u < U; u++) {  // unconditional loads at clamped indices, all in flight
-			const int i = base + min(i0 + u * kCsrRows, cnt - 1);
-			c[u] = colind[i];
+	for (int u = 0; u < U; u++) {  // unconditional loads at clamped indices, all in flight
+		const int i = min(c0 + t + u * kCsrRows, c1 - 1);
+		c[u] = colind[i];
 #pragma unroll
-			for (int q = 0; q < NAM; q++) a[u][q] = As[(int64_t)min(q, nA - 1) * ldas + i];
-		}
+		for (int q = 0; q < NAM; q++) a[u][q] = As[(int64_t)min(q, nA - 1) * ldas + i];
+	}
 #pragma unroll
-		for (int u = 0; u < U; u++) x[u] = X[c[u]];
+	for (int u = 0; u < U; u++) x[u] = X[c[u]];
 #pragma unroll
-		for (int u = 0; u < U; u++) {
-			const int i = i0 + u * kCsrRows;
-			if (i < cnt) {
+	for (int u = 0; u < U; u++) {
+		const int i = t + u * kCsrRows;
+		if (c0 + i < c1) {
 #pragma unroll
-				for (int q = 0; q < NAM; q++) st.a[q][i] = q < nA ? a[u][q] : 0.0;
-				st.x[i] = x[u];
-			}
+			for (int q = 0; q < NAM; q++) st.a[q][i] = q < nA ? a[u][q] : 0.0;
+			st.x[i] = x[u];
 		}
 	}
-	__syncthreads();
-	return true;
 }
 
-// the row with staged nonzeros [b, e): nA x nB pair sums in row order (the chains of csrmm_row_sum), then
-// their sum
+// The sum of row r (r0 + thread; none beyond m) over its staged nonzeros: nA x nB pair sums in row order (the
+// chains of csrmm_row_sum), the range passing through the stage kCap nonzeros at a time, then their sum.
+// Called by the whole workgroup.
 template <int NAM, int NBM, class T, class V>
-__device__ __forceinline__ T csr_stage_row(const CsrStage<NAM, T> &st, int b, int e, int nA, int nB, int maxlevel,
-                                           int fsum, const uint16_t *J, const VsPlan *plan, T *Cs, int64_t ldc,
-                                           int row) {
+__device__ __forceinline__ T csr_stage_row(CsrStage<NAM, T> &st, int r0, int m, const double *As, int64_t ldas, int nA,
+                                           const int *colind, const int *rowptr, const T *X, int nB, int maxlevel,
+                                           int fsum, const uint16_t *J, const VsPlan *plan, T *Cs, int64_t ldc) {
+	const int r = r0 + (int)threadIdx.x;
+	const int c0 = rowptr[r0], c1 = rowptr[min(r0 + kCsrRows, m)];
+	const int b = r < m ? rowptr[r] : 0, e = r < m ? rowptr[r + 1] : 0;
 	T sig[NBM];
 	const int last = plan->last;
 #pragma unroll
@@ -1420,22 +1392,30 @@ __device__ __forceinline__ T csr_stage_row(const CsrStage<NAM, T> &st, int b, in
 	RegVec<NAM * NBM, V> v;
 #pragma unroll
 	for (int q = 0; q < NAM * NBM; q++) v[q] = (V)0;
-	for (int j = b; j < e; j++) {
-		T r = st.x[j];
-		double a[NAM];
+	for (int c = c0; c < c1; c += CsrStage<NAM, T>::kCap) {
+		const int ce = min(c + CsrStage<NAM, T>::kCap, c1);
+		if (c > c0) __syncthreads();  // the rows are done with the previous part
+		csr_stage_load<NAM, T>(st, c, ce, As, ldas, nA, colind, X);
+		__syncthreads();
+		const int je = min(e, ce) - c;
+		for (int j = max(b, c) - c; j < je; j++) {
+			T w = st.x[j];
+			double a[NAM];
 #pragma unroll
-		for (int ia = 0; ia < NAM; ia++) a[ia] = st.a[ia][j];
+			for (int ia = 0; ia < NAM; ia++) a[ia] = st.a[ia][j];
 #pragma unroll
-		for (int ib = 0; ib < NBM; ib++)
-			if (ib < nB) {  // uniform
-				const T x = (r + sig[ib]) - sig[ib];  // VsGen's step
-				r = r - x;
+			for (int ib = 0; ib < NBM; ib++)
+				if (ib < nB) {  // uniform
+					const T x = (w + sig[ib]) - sig[ib];  // VsGen's step
+					w = w - x;
 #pragma unroll
-				for (int ia = 0; ia < NAM; ia++)
-					v[ia * NBM + ib] = (V)fma(a[ia], (double)x, (double)v[ia * NBM + ib]);
-			}
+					for (int ia = 0; ia < NAM; ia++)
+						v[ia * NBM + ib] = (V)fma(a[ia], (double)x, (double)v[ia * NBM + ib]);
+				}
+		}
 	}
-	return csr_pairs_sum<NAM, NBM, T, V>(v, nA, nB, maxlevel, fsum, J, Cs, ldc, row);
+	if (r >= m) return (T)0;
+	return csr_pairs_sum<NAM, NBM, T, V>(v, nA, nB, maxlevel, fsum, J, Cs, ldc, r);
 }
 
 // a row in memory, one pair at a time: each pair sum runs over the row's nonzeros in order, then NearSum over
@@ -1496,26 +1476,20 @@ __global__ __launch_bounds__(kCsrRows) void k_csrmv_plan(int m, const double *As
 	__shared__ CsrStage<NAM, T> st;
 	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
 	if (r0 >= m) return;
-	const int rows = min(kCsrRows, m - r0);
-	const int base = rowptr[r0], cnt = rowptr[r0 + rows] - base;
 	const int maxlevel = max((nA - 1) + (nB - 1) - fastMode, min(nA - 1, nB - 1));
-	const bool staged = !X.plan->bad && csr_stage_load<NAM, T>(st, base, cnt, As, ldas, nA, colind, (const T *)X.x);
 	const int r = r0 + (int)threadIdx.x;
-	if (r >= m) return;
-	T t;
-	if (staged) {
-		t = csr_stage_row<NAM, NBM, T, V>(st, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J, X.plan,
-		                                  Cs, ldc, r);
-	} else if constexpr (NBM > kCsrPlanSlices) {
-		t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Cs, ldc, J);
-	} else if (X.plan->bad) {
-		t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel,
-		                                                 fsum, J);
+	T t = (T)0;
+	if (!X.plan->bad) {  // uniform
+		t = csr_stage_row<NAM, NBM, T, V>(st, r0, m, As, ldas, nA, colind, rowptr, (const T *)X.x, nB, maxlevel, fsum, J,
+		                                  X.plan, Cs, ldc);
+		if (r >= m) return;
 	} else {
-		VsGen<T, NBM> g;
-		g.init(X.plan);
-		t = csrmm_row_sum<NAM, NBM, T, T, true, V>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel, fsum, J,
-		                                           (const T *)X.x, &g);
+		if (r >= m) return;
+		if constexpr (NBM > kCsrPlanSlices)
+			t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Cs, ldc, J);
+		else
+			t = csrmm_row_sum<NAM, NBM, T, double, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel, fsum,
+			                                          J);
 	}
 	y[r] = fma1_t(alpha, t, beta * y[r]);
 }
@@ -1563,7 +1537,7 @@ __global__ __launch_bounds__(256) void k_csrmm_sum(int m, const double *As, int6
                                                    const uint16_t *J) {
 	const int r = blockIdx.x * blockDim.x + threadIdx.x;
 	if (r >= m) return;
-	const T t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, Xs, ldxs,
+	const T t = csrmm_row_sum<NAM, NBM, T, double, V>(r, As, ldas, nA, colind, rowptr, Xs, ldxs,
 	                                                         nB, maxlevel, fsum, J);
 	y[r] = fma1_t(alpha, t, beta * y[r]);
 }
@@ -2142,33 +2116,21 @@ __global__ __launch_bounds__(256) void k_csrmm_sum_dev(int m, const double *As, 
 	const int r0 = csr_block((m + kCsrRows - 1) / kCsrRows) * kCsrRows;
 	const int r = r0 + (int)threadIdx.x;
 	// a plan: the staged rows (csr_stage_row); uniform over the workgroup
-	int base = 0;
-	bool staged = false;
 	__shared__ CsrStage<NAM, T> stage;
-	if (r0 < m && nB <= NBM && !X.plan->bad) {
-		const int rows = min(kCsrRows, m - r0);
-		base = rowptr[r0];
-		staged = csr_stage_load<NAM, T>(stage, base, rowptr[r0 + rows] - base, As, ldas, nA, colind, (const T *)X.x);
-	}
+	const int maxlevel = (nA - 1) + (nB - 1);
+	T t = 0;
+	T *Ct = (T *)Cs;
+	const bool staged = r0 < m && nB <= NBM && !X.plan->bad;
+	if (staged)
+		t = csr_stage_row<NAM, NBM, T, V>(stage, r0, m, As, ldas, nA, colind, rowptr, (const T *)X.x, nB, maxlevel, fsum, J,
+		                                  X.plan, Ct, ldc);
 	if (r < m) {
-		const int maxlevel = (nA - 1) + (nB - 1);
-		T t = 0;
-		T *Ct = (T *)Cs;
-		if (staged) {
-			t = csr_stage_row<NAM, NBM, T, V>(stage, rowptr[r] - base, rowptr[r + 1] - base, nA, nB, maxlevel, fsum, J,
-			                                  X.plan, Ct, ldc, r);
-		} else if (nB > NBM || NBM > 8) {
-			t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Ct, ldc, J);
-		} else if constexpr (NBM <= 8) {
-			if (X.plan->bad) {
-				t = csrmm_row_sum<NAM, NBM, T, double, false, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB,
-				                                                 maxlevel, fsum, J);
-			} else {
-				VsGen<T, NBM> g;
-				g.init(X.plan);
-				t = csrmm_row_sum<NAM, NBM, T, T, true, V>(r, As, ldas, nA, colind, rowptr, nullptr, 0, nB, maxlevel, fsum,
-				                                           J, (const T *)X.x, &g);
-			}
+		if (!staged) {
+			if (nB > NBM || NBM > kCsrPlanSlices)
+				t = csr_big_row<T, V>(r, As, ldas, nA, colind, rowptr, X, nB, maxlevel, fsum, Ct, ldc, J);
+			else if constexpr (NBM <= kCsrPlanSlices)
+				t = csrmm_row_sum<NAM, NBM, T, double, V>(r, As, ldas, nA, colind, rowptr, X.slices, X.lds, nB, maxlevel,
+				                                          fsum, J);
 		}
 		const T v = fma1_t((T)1, t, (T)0 * y[r]);
 		y[r] = v;

@@ -268,8 +268,8 @@ __device__ void split_csr_row(int r, const TI *val, const int *rowptr, TI *work,
 // the current slice are rows in LDS, each slice leaves as one contiguous store of the range, and the
 // remainders never touch memory (row by row in memory: 0.34 ms for the 100^3 Laplacian, 2 slices, most
 // of it partial cache lines).  A longer range takes split_csr_row.
-constexpr int kCsrSplitCap = 2048;
-template <class TI>
+// CAP: nonzeros of the stage, 32 or 64 KB of it by the mean row length (eight nonzeros fill the smaller one).
+template <class TI, int CAP>
 __global__ __launch_bounds__(256) void k_split_csr_staged(int m, const TI *val, const int *rowptr, TI *work,
                                                           double *split, int64_t lds, int shift, int cap,
                                                           const uint16_t *J, int *zrow, int *zmax, int epsMode,
@@ -277,12 +277,12 @@ __global__ __launch_bounds__(256) void k_split_csr_staged(int m, const TI *val, 
 	const int r0 = blockIdx.x * 256, rows = min(256, m - r0);
 	const int base = rowptr[r0], cnt = rowptr[r0 + rows] - base;
 	const int r = r0 + (int)threadIdx.x;
-	if (cnt > kCsrSplitCap) {
+	if (cnt > CAP) {
 		if (r < m) split_csr_row(r, val, rowptr, work, split, lds, shift, cap, J, zrow, zmax, epsMode, mixed);
 		return;
 	}
-	__shared__ TI rem[kCsrSplitCap];
-	__shared__ double sl[kCsrSplitCap];
+	__shared__ TI rem[CAP];
+	__shared__ double sl[CAP];
 	for (int i = threadIdx.x; i < cnt; i += 256) rem[i] = val[base + i];
 	__syncthreads();
 	int b = 0, e = 0, rho = 0;
@@ -495,18 +495,29 @@ void launch_copy(hipStream_t st, const double *src, double *dst, int64_t n) {
 	hipLaunchKernelGGL(k_copy, dim3((unsigned)g), dim3(256), 0, st, src, dst, n);
 }
 
-void launch_split_csr(hipStream_t st, int m, const double *val, const int *rowptr, double *work,
-                      double *split, int64_t lds, int shift, int cap, const uint16_t *J, int *zrow,
-                      int *zmax, int epsMode, int mixed) {
-	hipLaunchKernelGGL(k_split_csr_staged<double>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
-	                   work, split, lds, shift, cap, J, zrow, zmax, epsMode, mixed);
+template <class TI>
+static void split_csr(hipStream_t st, int m, int nnz, const TI *val, const int *rowptr, TI *work, double *split,
+                      int64_t lds, int shift, int cap, const uint16_t *J, int *zrow, int *zmax, int epsMode,
+                      int mixed) {
+	const dim3 g((m + 255) / 256);
+	if (nnz <= (int64_t)m * 8)
+		hipLaunchKernelGGL((k_split_csr_staged<TI, 2048>), g, dim3(256), 0, st, m, val, rowptr, work, split, lds, shift,
+		                   cap, J, zrow, zmax, epsMode, mixed);
+	else
+		hipLaunchKernelGGL((k_split_csr_staged<TI, 4096>), g, dim3(256), 0, st, m, val, rowptr, work, split, lds, shift,
+		                   cap, J, zrow, zmax, epsMode, mixed);
 }
 
-void launch_split_csr(hipStream_t st, int m, const float *val, const int *rowptr, float *work,
+void launch_split_csr(hipStream_t st, int m, int nnz, const double *val, const int *rowptr, double *work,
+                      double *split, int64_t lds, int shift, int cap, const uint16_t *J, int *zrow,
+                      int *zmax, int epsMode, int mixed) {
+	split_csr(st, m, nnz, val, rowptr, work, split, lds, shift, cap, J, zrow, zmax, epsMode, mixed);
+}
+
+void launch_split_csr(hipStream_t st, int m, int nnz, const float *val, const int *rowptr, float *work,
                       double *split, int64_t lds, int shift, int cap, const uint16_t *JF, int *zrow,
                       int *zmax, int epsMode, int mixed) {
-	hipLaunchKernelGGL(k_split_csr_staged<float>, dim3((m + 255) / 256), dim3(256), 0, st, m, val, rowptr,
-	                   work, split, lds, shift, cap, JF, zrow, zmax, epsMode, mixed);
+	split_csr(st, m, nnz, val, rowptr, work, split, lds, shift, cap, JF, zrow, zmax, epsMode, mixed);
 }
 
 void launch_zero_slots_csr(hipStream_t st, int m, const int *rowptr, double *split, int64_t lds,

@@ -64,7 +64,7 @@ CASES = {
     "block": [7] * 256,
     "block_plus_one": [7] * 257,
     "stage_full": [8] * 256 + [3] * 40,         # 2048 nonzeros in the first block
-    "stage_over": [9] * 256 + [2] * 300,        # the first block walks its rows in memory
+    "stage_over": [9] * 256 + [2] * 300,        # the first block passes through the stage in parts
     "empty_rows": [0, 3] * 300,
     "all_empty": [0] * 300,
     "long_row": [2] * 100 + [3000] + [1] * 500,
