@@ -358,6 +358,43 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		wreset(oh, base);
 		return OZBLAS_STATUS_SUCCESS;
 	}
+	// binary64 GEMV: the split of op(A) is fused into the slice products (the matrix is read once, its slices
+	// never stored, no counting pass); more slices than the kernel holds go on below
+	if constexpr (std::is_same<T, double>::value) {
+		if (!dotPath && n == 1 && fastMode == 0 && !b->mixed && split_gemv_fits(k)) {
+			const int cap = split_cap(oh), rho = Prec<T>::rho(oh, k), rem = repro_slot(oh) ? 1 : 0;
+			constexpr int kSlots = 5;  // slots of x that are valid after its split (the kernel reads 4)
+			double *Xs = (double *)walloc(oh, 8ull * ldk * (cap + 2 > kSlots ? cap + 2 : kSlots));
+			double *Pv = (double *)walloc(oh, split_gemv_pairs_bytes(m));
+			int *zcol = (int *)walloc(oh, 256);
+			if (Xs && Pv && zcol) {
+				int *out = (int *)b->hPinned;
+				OZ_HIP(hipMemsetAsync(b->dCounters, 0, 2 * sizeof(int), st));
+				launch_split_cols(st, k, 1, bin, ldbi, (T *)nullptr, ldk, Xs, ldk, ldk, rho, oh->splitShift, cap,
+				                  Prec<T>::Jsplit(b), zcol, b->dCounters, kSlots);
+				OZ_HIP(hipEventRecord(b->ev[3], st));
+				launch_split_gemv(st, k, m, ain, ldai, rho, oh->splitShift, cap, Prec<T>::Jsplit(b), rem, Xs, ldk,
+				                  b->dCounters, fsum ? 1 : 0, alpha, beta, C, Prec<T>::Jsum(b), Pv, out);
+				OZ_HIP(hipEventRecord(b->ev[4], st));
+				OZ_HIP(hipGetLastError());
+				OZ_TRY(sync(oh));
+				if (!out[2]) {
+					oh->mbk = m;
+					oh->nbk = n;
+					oh->nSplitA = (float)out[0];
+					oh->nSplitB = (float)out[1];
+					oh->nSplitC = (float)out[0] * (float)out[1];
+					oh->t_comp = ev_sec(b->ev[3], b->ev[4]);
+					oh->t_sum = 0.f;
+					oh->t_total = tt.sec();
+					oh->n_comp = (float)(2.0 * m * n * (double)k * oh->nSplitC);
+					wreset(oh, base);
+					return OZBLAS_STATUS_SUCCESS;
+				}
+			}
+			wreset(oh, base2);
+		}
+	}
 	// blocking: slice counts of the whole operands bound those of any block, so halving the
 	// larger side (as src/cpu/ozblas_gemm.cpp:91-96) until the exact need fits is safe
 	int nAf = 0, nBf = 0, zAf = -1, zBf = -1;
@@ -390,34 +427,6 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 			wreset(oh, base2);
 			T *rem = (T *)walloc(oh, sizeof(T) * ldk * std::max(mbk_, nbk_));
 			if (!rem) return OZBLAS_STATUS_WORKSPACE;
-			// binary64 GEMV over the whole matrix: the split of op(A) is fused into the slice
-			// products (the matrix is read once, its slices never stored); x is split as usual
-			if constexpr (std::is_same<T, double>::value) {
-				if (!dotPath && n == 1 && fastMode == 0 && nbk_ == 1 && mbk == m && !b->mixed &&
-				    split_gemv_fits(k, nAf, nBf)) {
-					DenseSplit dx;
-					OZ_TRY(dense_split(oh, k, nbk_, bin + (int64_t)in * nbk * ldbi, ldbi, rem, ldk, dx,
-					                   nbk == n ? zBf : -1));
-					T *Cblk = C + (int64_t)ldc * ((int64_t)in * nbk) + (int64_t)im * mbk;
-					double *P = (double *)walloc(oh, split_gemv_pairs_bytes(mbk_));
-					if (!P) return OZBLAS_STATUS_WORKSPACE;
-					OZ_HIP(hipEventRecord(b->ev[3], st));
-					if (launch_split_gemv(st, k, mbk_, ain + (int64_t)im * mbk * ldai, ldai, Prec<T>::rho(oh, k),
-					                      oh->splitShift, split_cap(oh), Prec<T>::Jsplit(b), nAf, dx.slices,
-					                      dx.sstride, dx.count, fsum ? 1 : 0, alpha, beta, Cblk,
-					                      Prec<T>::Jsum(b), P)) {
-						OZ_HIP(hipEventRecord(b->ev[4], st));
-						OZ_HIP(hipGetLastError());
-						OZ_TRY(sync(oh));
-						tcomp += ev_sec(b->ev[3], b->ev[4]);
-						sA += nAf;
-						sB += dx.count;
-						sC += (double)nAf * dx.count;
-						blocks++;
-						continue;
-					}
-				}
-			}
 			DenseSplit da, db;
 			// a block that is the whole operand reuses the first-zero level of count_cols
 			OZ_TRY(dense_split(oh, k, mbk_, ain + (int64_t)im * mbk * ldai, ldai, rem, ldk, da,

@@ -222,14 +222,15 @@ void launch_csrmm_store(hipStream_t st, int m, const double *As, int64_t ldas, i
 // GEMV of the plain form on k-contiguous slices (slice s of A column i at As + s*sA + i*ldk, of x
 // at Xs + s*sX), fused with the sum (Fsum in level order or NearSum) and the epilogue into y;
 // false when the slice counts exceed its register bound (8 x 8)
-// GEMV with the split of op(A) fused (binary64; rows of op(A) k-contiguous in `in`): false when the
-// sizes or slice counts are outside the kernel's (then nothing was launched; split_gemv_fits tells)
-// P: split_gemv_pairs_bytes(M) of scratch for the pair values of every row
-bool split_gemv_fits(int K, int nA, int nB);
+// GEMV with the split of op(A) fused (binary64; rows of op(A) k-contiguous in `in`), for K that
+// split_gemv_fits: no count is known before.  x's slices (at least 4 valid, zero beyond its count) at Xs; z:
+// x's first-zero level, then the maximum of A's (zero before).  P: split_gemv_pairs_bytes(M) of scratch.
+// out (host memory): the slice counts, and out[2] = 1 when they exceed 8 x 4 -- then y is untouched.
+bool split_gemv_fits(int K);
 size_t split_gemv_pairs_bytes(int M);
-bool launch_split_gemv(hipStream_t st, int K, int M, const double *in, int64_t ldi, int rho, int shift,
-                       int cap, const uint16_t *Js, int nA, const double *Xs, int64_t sX, int nB,
-                       int fsum, double alpha, double beta, double *y, const uint16_t *J, double *P);
+void launch_split_gemv(hipStream_t st, int K, int M, const double *in, int64_t ldi, int rho, int shift, int cap,
+                       const uint16_t *Js, int remSlot, const double *Xs, int64_t sX, int *z, int fsum,
+                       double alpha, double beta, double *y, const uint16_t *J, double *P, int *out);
 bool launch_gemv_slices(hipStream_t st, int M, int K, const double *As, int64_t ldk, int64_t sA, int nA,
                         const double *Xs, int64_t sX, int nB, int fsum, double alpha, double beta,
                         double *y, const uint16_t *J);

@@ -33,6 +33,28 @@ __device__ inline double block_sum_d(double v, double *red) {
 	return r;
 }
 
+// halving lane exchanges: the sums of a over the lane pairs (l, l + 32) in the lower half of the result
+// and of b in the upper half; the same for neighbouring rows of 16 lanes, a in the even rows, b in the odd
+__device__ __forceinline__ double swap_add32(double a, double b) {
+	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+	const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+	const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+	const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+	const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+
+// slice count of a split whose first all-zero remainder is after level z (cap: none), as split_count
+__device__ inline int sg_count(int z, int cap, int remSlot) {
+	return (cap <= 1 ? 1 : z < cap ? max(z, 1) + 1 : cap) + (remSlot ? 1 : 0);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Vector split without grid barriers.
 //
@@ -1799,159 +1821,216 @@ bool launch_gemv_slices(hipStream_t st, int M, int K, const double *As, int64_t 
 }
 
 // ---------------------------------------------------------------------------------------------
-// GEMV with the split of op(A) fused (binary64): one 512-thread workgroup per row of op(A), which
-// is a k-contiguous column of `in` (K <= 512 R; up to 8 slices of A and 4 of x).  The row is split in registers level by level
-// with the rule of k_split_cols_reg (slot s: the part of level s; then the remainder slot and zero
-// slots up to nA), and each slot is multiplied at once by the x slices, which every thread keeps
-// in registers for its R indices: the pair dots sum_k As_s[k] Xs_b[k] are exact, so the workgroup
-// sums them in any order (one LDS round per level carries the nB pair sums and the next level's
-// remainder maximum).  The nA x nB pair values of row i go to P[i * kSgPairs + a * NBM + b]; the
-// slices of A are never stored, the matrix is read once.  k_pairs_sum then sums each row's values
-// as k_gemv_slices does (Fsum in (level, ia) order, or NearSum) and writes y_i.
+// GEMV with the split of op(A) fused (binary64): a workgroup per row of op(A), a k-contiguous column of
+// `in` (K <= BS R).  The row is split in registers level by level with the rule of k_split_cols_reg, and
+// each slice is multiplied at once by the x slices, which every thread keeps in registers for its R
+// indices over all the rows it takes.  The pair dots sum_k As_s[k] Xs_b[k] are exact, so their order does
+// not matter: each wave reduces its four sums of a level by two halving lane exchanges and leaves them in
+// LDS, and only the next level's remainder maximum goes through a workgroup barrier.  The next row's
+// elements load while this one is split.  The slices of A are never stored, the matrix is read once.  Slots
+// not reached are zero.  P[(i kSgNAM + slot) NBM + b]: the pair values of row i.
+// One workgroup of 512 with 16 elements a thread whatever K, all five values of a level reduced by
+// shuffles: 400 us for 8192 x 8192 (1.3 TB/s); with four sums by lane exchanges and the next row loading meanwhile: 240 us (2.2 TB/s, bound by FP64 arithmetic and the barrier of each level), and no count pass before it (130 us).
 // ---------------------------------------------------------------------------------------------
-constexpr int kSgBS = 512, kSgNAM = 8, kSgPairs = 64;
-template <int R, int NBM>
-__global__ __launch_bounds__(kSgBS) void k_split_gemv(int K, int M, const double *in, int64_t ldi,
-                                                      int rho, int shift, int cap, const uint16_t *Js,
-                                                      int nA, const double *Xs, int64_t sX, int nB,
-                                                      double *P) {
-	constexpr int BS = kSgBS, NW = BS / 64, NV = NBM + 1;  // per round: NBM sums and a maximum
-	__shared__ double red[2][NW][NV];
-	const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
-	double xr[NBM][R];
+constexpr int kSgNAM = 8, kSgNBM = 4;
+template <int BS, int R>
+__global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *in, int64_t ldi, int rho, int shift,
+                                                   int cap, const uint16_t *Js, int remSlot, const double *Xs,
+                                                   int64_t sX, const int *zx, double *P, int *zmax) {
+	constexpr int NW = BS / 64, NB = kSgNBM;
+	__shared__ double red[2][NW];
+	__shared__ double sums[2][kSgNAM][NW][NB];
+	const int l = threadIdx.x % 64, w = threadIdx.x / 64;
+	const int nB = sg_count(*zx, cap, remSlot);
+	if (nB > NB) return;
+	double xr[NB][R];
 #pragma unroll
-	for (int b = 0; b < NBM; b++)
+	for (int b = 0; b < NB; b++)
 #pragma unroll
 		for (int q = 0; q < R; q++) {
 			const int i = threadIdx.x + BS * q;
 			xr[b][q] = (b < nB && i < K) ? Xs[(int64_t)b * sX + i] : 0.0;
 		}
-	int round = 0;
-	// one reduction round over the workgroup: val[0..NBM) summed, val[NBM] maximised; every
-	// thread gets the totals (double-buffered by round parity: one barrier per round)
-	auto reduce = [&](double (&val)[NV]) {
-#pragma unroll
-		for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-			for (int b = 0; b < NBM; b++) val[b] += __shfl_xor(val[b], o, 64);
-			val[NBM] = std_max(val[NBM], __shfl_xor(val[NBM], o, 64));
-		}
-		const int buf = round & 1;
-		if (lane == 0) {
-#pragma unroll
-			for (int c = 0; c < NV; c++) red[buf][w][c] = val[c];
-		}
-		__syncthreads();
-#pragma unroll
-		for (int c = 0; c < NV; c++) val[c] = red[buf][0][c];
-		for (int u = 1; u < NW; u++) {
-#pragma unroll
-			for (int b = 0; b < NBM; b++) val[b] += red[buf][u][b];
-			val[NBM] = std_max(val[NBM], red[buf][u][NBM]);
-		}
-		round++;
+	int par = 0, z = 0;
+	// this wave's sums of slot s (uniform) into the buffer of the row's parity
+	auto reduce4 = [&](const double (&v)[NB], int rowPar, int s) {
+		// lane rows 0 .. 3 end with values 0, 1, 2, 3 (wave_reduce_pairs for four)
+		double t = swap_add16(swap_add32(v[0], v[2]), swap_add32(v[1], v[3]));
+		t += dpp_f64<0xB1>(t);
+		t += dpp_f64<0x4E>(t);
+		t += dpp_f64<0x141>(t);
+		t += dpp_f64<0x140>(t);
+		if (l % 16 == 0) sums[rowPar][s][w][(l / 16) % 2 + 2 * (l / 32)] = t;
 	};
-	for (int j = blockIdx.x; j < M; j += gridDim.x) {
-		const double *x = in + (int64_t)j * ldi;
-		double *Pj = P + (int64_t)j * kSgPairs;
-		double v[R];
-		double val[NV];
-#pragma unroll
-		for (int c = 0; c < NV; c++) val[c] = 0.0;
+	double nx[R];
+	auto load = [&](int j) {
+		// a buffer of the row's K elements: offsets beyond it load 0.  The empty statement keeps the R offsets
+		// from being held in registers over the loop, which spilled.
+		const auto x = __builtin_amdgcn_make_buffer_rsrc((void *)(in + (int64_t)j * ldi), 0, K * 8, 0x00027000);
+		int off = threadIdx.x * 8;
+		asm volatile("" : "+v"(off));
 #pragma unroll
 		for (int q = 0; q < R; q++) {
-			const int i = threadIdx.x + BS * q;
-			v[q] = (i < K) ? x[i] : 0.0;
-			val[NBM] = std_max(val[NBM], fabs(v[q]));
+			const auto t = __builtin_amdgcn_raw_buffer_load_b64(x, off + BS * 8 * q, 0, 0);
+			nx[q] = __builtin_bit_cast(double, t);
 		}
-		reduce(val);
-		double mx = val[NBM];
+	};
+	int prev = -1, prevSlots = 0;
+	// the sums of a finished row over the waves; called after a barrier that follows its products
+	auto store = [&](int rowPar) {
+		for (int q = threadIdx.x; q < kSgNAM * NB; q += BS) {
+			const int s = q / NB, b = q % NB;
+			double t = 0.0;
+			if (s < prevSlots) {
+				t = sums[rowPar][s][0][b];
+#pragma unroll
+				for (int u = 1; u < NW; u++) t += sums[rowPar][s][u][b];
+			}
+			P[(int64_t)prev * (kSgNAM * NB) + q] = t;
+		}
+	};
+	int rowPar = 0;
+	if ((int)blockIdx.x < M) load(blockIdx.x);
+	for (int j = blockIdx.x; j < M; j += gridDim.x) {
+		double v[R], lm = 0.0;
+#pragma unroll
+		for (int q = 0; q < R; q++) {
+			v[q] = nx[q];
+			lm = max_abs(lm, v[q]);
+		}
+		if (j + (int)gridDim.x < M) load(j + gridDim.x);
+		auto reduce = [&](double a) {  // one barrier: two buffers
+			a = wave_max_nonneg_f64(a);
+			if (l == 0) red[par][w] = a;
+			__syncthreads();
+			a = red[par][0];
+#pragma unroll
+			for (int u = 1; u < NW; u++) a = std_max(a, red[par][u]);
+			par ^= 1;
+			return a;
+		};
+		double mx = reduce(lm);
+		if (prev >= 0) store(rowPar ^ 1);
 		int s = 0;
 		bool zero = false;
 		for (s = 0; s < cap; s++) {
-			const int tau = SplitRule<double>::tau(mx, Js);
-			const double sigma = SplitRule<double>::sigma(rho, tau, shift);
-#pragma unroll
-			for (int c = 0; c < NV; c++) val[c] = 0.0;
+			const double sigma = SplitRule<double>::sigma(rho, SplitRule<double>::tau(mx, Js), shift);
+			double acc[NB] = {};
+			lm = 0.0;
 #pragma unroll
 			for (int q = 0; q < R; q++) {
 				const double part = (v[q] + sigma) - sigma;
-				const double rr = v[q] - part;
-				v[q] = rr;
+				v[q] = v[q] - part;
+				lm = max_abs(lm, v[q]);
 #pragma unroll
-				for (int b = 0; b < NBM; b++) val[b] = fma(part, xr[b][q], val[b]);
-				val[NBM] = std_max(val[NBM], fabs(rr));
+				for (int b = 0; b < NB; b++) acc[b] = fma(part, xr[b][q], acc[b]);
 			}
-			reduce(val);
-			if (threadIdx.x < NBM && s < kSgNAM) Pj[s * NBM + threadIdx.x] = val[threadIdx.x];
-			mx = val[NBM];
+			if (s < kSgNAM) reduce4(acc, rowPar, s);
+			mx = reduce(lm);
 			if (mx == 0.0) {
 				zero = true;
 				break;
 			}
 		}
-		const int last = zero ? s : cap - 1;
-		if (!zero && last + 1 < nA) {  // the remainder slot
-#pragma unroll
-			for (int c = 0; c < NV; c++) val[c] = 0.0;
+		const int zr = zero ? s : cap;
+		int slots = zero ? s + 1 : cap;
+		if (!zero && remSlot && cap < kSgNAM) {  // the remainder slot of reproMode 0
+			double acc[NB] = {};
 #pragma unroll
 			for (int q = 0; q < R; q++)
 #pragma unroll
-				for (int b = 0; b < NBM; b++) val[b] = fma(v[q], xr[b][q], val[b]);
-			reduce(val);
-			if (threadIdx.x < NBM && last + 1 < kSgNAM) Pj[(last + 1) * NBM + threadIdx.x] = val[threadIdx.x];
+				for (int b = 0; b < NB; b++) acc[b] = fma(v[q], xr[b][q], acc[b]);
+			reduce4(acc, rowPar, cap);
+			slots = cap + 1;
+			__syncthreads();
 		}
-		// zero slots
-		const int z0 = zero ? last + 1 : last + 2;
-		for (int t = z0 + (int)threadIdx.x / NBM; t < nA && t < kSgNAM; t += BS / NBM)
-			Pj[t * NBM + threadIdx.x % NBM] = 0.0;
+		z = max(z, zr);
+		prev = j;
+		prevSlots = slots;
+		rowPar ^= 1;
 	}
+	__syncthreads();
+	if (prev >= 0) store(rowPar ^ 1);
+	if (threadIdx.x == 0 && z > 0 && __hip_atomic_load(zmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < z)
+		atomicMax(zmax, z);
 }
 
-// y_i = fma(alpha, sum of row i's pair values, beta * y_i); one thread per row
-template <int NBM>
-__global__ __launch_bounds__(256) void k_pairs_sum(int M, double *P, int nA, int nB, int fsum,
-                                                   double alpha, double beta, double *y,
-                                                   const uint16_t *J) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= M) return;
-	const double *Pi = P + (int64_t)i * kSgPairs;
-	double t;
-	if (fsum) {
-		t = 0.0;
-		for (int ik = 0; ik < kSgNAM + NBM - 1; ik++)
+// y_i = fma(alpha, sum of row i's pair values, beta * y_i): 16 threads a row, the clear-cut case of NearSum
+// over their values, then one thread for the rest.  The counts come from the split kernels' first-zero
+// levels; with more slices than the kernels hold y stays untouched and out[2] = 1.  out (host memory):
+// slice counts of A and x, the flag.
+__global__ __launch_bounds__(256) void k_pairs_sum(int M, double *P, const int *z, int cap, int remSlot, int fsum,
+                                                   double alpha, double beta, double *y, const uint16_t *J, int *out) {
+	constexpr int NB = kSgNBM;
+	const int nA = sg_count(z[1], cap, remSlot), nB = sg_count(z[0], cap, remSlot);
+	const bool over = nA > kSgNAM || nB > NB;
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		out[0] = nA;
+		out[1] = nB;
+		out[2] = over ? 1 : 0;
+	}
+	if (over) return;
+	const int i = blockIdx.x * 16 + threadIdx.x / 16, t = threadIdx.x % 16;
+	double *Pi = P + (int64_t)min(i, M - 1) * (kSgNAM * NB);
+	double s = 0.0;
+	if (!fsum) {
+		// threads 0 .. 15 hold values t and t + 16 of the row (absent pairs are zero)
+		SumCert c;
+		c.add(Pi[t]);
+		c.add(Pi[t + 16]);
+#pragma unroll
+		for (int o = 1; o < 16; o <<= 1) {
+			const double s2 = __shfl_xor(c.s, o, 64), e2 = __shfl_xor(c.e, o, 64), a2 = __shfl_xor(c.a, o, 64);
+			const double u = c.s + s2, bb = u - c.s;
+			c.e = (c.e + e2) + ((c.s - (u - bb)) + (s2 - bb));
+			c.s = u;
+			c.a = c.a + a2;
+		}
+		if (t != 0 || i >= M) return;
+		if (!c.done(kSgNAM * NB + 16, s)) {
+			// the values in (a, b) order, compacted in place (scratch), then NearSum over them
+			int cnt = 0;
+			for (int a = 0; a < nA; a++)
+				for (int b = 0; b < nB; b++) Pi[cnt++] = Pi[a * NB + b];
+			StridedVec u{Pi, 1};
+			s = nearsum(cnt, u, J);
+		}
+	} else {
+		if (t != 0 || i >= M) return;
+		double v[kSgNAM * NB];
+#pragma unroll
+		for (int q = 0; q < kSgNAM * NB; q++) v[q] = Pi[q];
+#pragma unroll
+		for (int ik = 0; ik < kSgNAM + NB - 1; ik++)
+#pragma unroll
 			for (int a = 0; a < kSgNAM; a++) {
 				const int b = ik - a;
-				if (b >= 0 && b < NBM && a < nA && b < nB) t = t + Pi[a * NBM + b];
+				if (b >= 0 && b < NB && a < nA && b < nB) s = s + v[a * NB + b];
 			}
-	} else {
-		// the values in (a, b) order, compacted in place (scratch), then NearSum over them
-		double *Pw = P + (int64_t)i * kSgPairs;
-		int cnt = 0;
-		for (int a = 0; a < nA; a++)
-			for (int b = 0; b < nB; b++) Pw[cnt++] = Pw[a * NBM + b];
-		StridedVec u{Pw, 1};
-		t = nearsum(cnt, u, J);
 	}
-	y[i] = fma(alpha, t, beta * y[i]);
+	y[i] = fma(alpha, s, beta * y[i]);
 }
 
-size_t split_gemv_pairs_bytes(int M) { return sizeof(double) * kSgPairs * (size_t)(M > 0 ? M : 1); }
+size_t split_gemv_pairs_bytes(int M) { return sizeof(double) * kSgNAM * kSgNBM * (size_t)(M > 0 ? M : 1); }
 
-bool split_gemv_fits(int K, int nA, int nB) {
-	return nA >= 1 && nA <= kSgNAM && nB >= 1 && nB <= 4 && K >= 1 && K <= 16 * kSgBS;
-}
+bool split_gemv_fits(int K) { return K >= 1 && K <= 8192; }
 
-bool launch_split_gemv(hipStream_t st, int K, int M, const double *in, int64_t ldi, int rho, int shift,
-                       int cap, const uint16_t *Js, int nA, const double *Xs, int64_t sX, int nB,
-                       int fsum, double alpha, double beta, double *y, const uint16_t *J, double *P) {
-	if (!split_gemv_fits(K, nA, nB) || M < 1) return false;
-	const int grid = M < 1024 ? M : 1024;
-	const int gs = (M + 255) / 256;
-	hipLaunchKernelGGL((k_split_gemv<16, 4>), dim3(grid), dim3(kSgBS), 0, st, K, M, in, ldi, rho, shift, cap,
-	                   Js, nA, Xs, sX, nB, P);
-	hipLaunchKernelGGL((k_pairs_sum<4>), dim3(gs), dim3(256), 0, st, M, P, nA, nB, fsum, alpha, beta, y, J);
-	return true;
+void launch_split_gemv(hipStream_t st, int K, int M, const double *in, int64_t ldi, int rho, int shift, int cap,
+                       const uint16_t *Js, int remSlot, const double *Xs, int64_t sX, int *z, int fsum,
+                       double alpha, double beta, double *y, const uint16_t *J, double *P, int *out) {
+#define OZ_SPLIT_GEMV(BS, R, PER)                                                                           \
+	hipLaunchKernelGGL((k_split_gemv<BS, R>), dim3(M < 256 * PER ? M : 256 * PER), dim3(BS), 0, st, K, M, in, ldi, \
+	                   rho, shift, cap, Js, remSlot, Xs, sX, (const int *)z, P, z + 1)
+	// workgroups resident on 256 CUs, each over its share of the rows
+	if (K <= 256 * 2)
+		OZ_SPLIT_GEMV(256, 2, 8);
+	else if (K <= 256 * 8)
+		OZ_SPLIT_GEMV(256, 8, 4);
+	else
+		OZ_SPLIT_GEMV(512, 16, 1);
+#undef OZ_SPLIT_GEMV
+	hipLaunchKernelGGL(k_pairs_sum, dim3((M + 15) / 16), dim3(256), 0, st, M, P, (const int *)z, cap, remSlot, fsum,
+	                   alpha, beta, y, J, out);
 }
 
 // general case: store the products where blasRcsrmm puts them (column ic of CSplit, ld ldcs);
@@ -2477,20 +2556,6 @@ __device__ __forceinline__ void vs_gen_masked(const VsGen<TI, NS> &g, TI v, int 
 // leaves lane half h with value q + h NV / 2, swapping neighbouring rows of 16 lanes the same way with
 // NV / 4 values a lane; those are summed over the rows on the DPP network.  For 64 values 336
 // instructions, against 1152 for 64 full wave sums.
-__device__ __forceinline__ double swap_add32(double a, double b) {
-	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
-	const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
-	const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
-	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
-	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
-}
-__device__ __forceinline__ double swap_add16(double a, double b) {
-	const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
-	const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
-	const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
-	return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
-	       __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
-}
 template <int NV>
 __device__ __forceinline__ void wave_reduce_pairs(double (&v)[NV], double *out) {
 	static_assert(NV % 4 == 0, "two halvings");
