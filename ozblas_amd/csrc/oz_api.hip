@@ -146,29 +146,39 @@ static int32_t dense_split(ozblasHandle_t *oh, int k, int cols, const T *in, int
 }
 
 // ---------------------------------------------------------------------------------------------
-// slice count of a k-contiguous operand without storing slices (for the blocking decision)
+// slice counts of two k-contiguous operands without storing slices (for the blocking decision), with one
+// synchronisation for both: counts and first-zero levels
 // ---------------------------------------------------------------------------------------------
 template <class T>
-static int32_t count_cols(ozblasHandle_t *oh, int k, int cols, const T *in, int64_t ldi,
-                          int *count, int *zmaxOut = nullptr) {
+static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const T *const (&in)[2],
+                          const int64_t (&ldi)[2], int (&count)[2], int (&z)[2]) {
 	Backend *b = be(oh);
 	const uint64_t mark = wmark(oh);
 	const int64_t ldk = rup(k, 16);
-	T *rem = (T *)walloc(oh, sizeof(T) * ldk * cols);
-	double *scratch = (double *)walloc(oh, 8ull * ldk * cols);
-	int *zcol = (int *)walloc(oh, sizeof(int) * (size_t)cols);
+	const int most = imax(cols[0], cols[1]);
+	T *rem = (T *)walloc(oh, sizeof(T) * ldk * most);
+	double *scratch = (double *)walloc(oh, 8ull * ldk * most);
+	int *zcol = (int *)walloc(oh, sizeof(int) * (size_t)most);
 	if (!rem || !scratch || !zcol) return OZBLAS_STATUS_WORKSPACE;
-	OZ_HIP(hipMemsetAsync(b->dCounters, 0, sizeof(int), b->stream));
-	launch_split_cols(b->stream, k, cols, in, ldi, rem, ldk, scratch, ldk, 0,
-	                  Prec<T>::rho(oh, k), oh->splitShift, split_cap(oh),
-	                  Prec<T>::Jsplit(b), zcol, b->dCounters);
-	OZ_HIP(hipMemcpyAsync(b->hPinned, b->dCounters, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+	OZ_HIP(hipMemsetAsync(b->dCounters, 0, 2 * sizeof(int), b->stream));
+	for (int q = 0; q < 2; q++)
+		launch_split_cols(b->stream, k, cols[q], in[q], ldi[q], rem, ldk, scratch, ldk, 0, Prec<T>::rho(oh, k),
+		                  oh->splitShift, split_cap(oh), Prec<T>::Jsplit(b), zcol, b->dCounters + q);
+	OZ_HIP(hipMemcpyAsync(b->hPinned, b->dCounters, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
-	*count = split_count(oh, ((int32_t *)b->hPinned)[0]);
-	if (zmaxOut) *zmaxOut = ((int32_t *)b->hPinned)[0];
+	for (int q = 0; q < 2; q++) {
+		z[q] = ((int32_t *)b->hPinned)[q];
+		count[q] = split_count(oh, z[q]);
+	}
 	wreset(oh, mark);
 	return OZBLAS_STATUS_SUCCESS;
 }
+
+// Work (slice pairs times m n k) from which the residue form is the faster way to NearSum's bits.  Its
+// statistics, uploads and one more synchronisation cost what the FP64 products take below the line: 256^3, 16
+// pairs (2.7e8), 140 us by FP64 slices and 170 us by residues; 384^3 (9e8) 166 and 150; 128 x 128 x 2500
+// (6.6e8) 494 and 171; 2500 x 128 x 128, 12 pairs (4.9e8) 175 and 159; 2500 x 2301 x 2700 8,480 and 770.
+constexpr double kPlainResidueWork = 5e8;
 
 // slice pairs of a GEMM in the reference's level order (src/cpu/ozblas_gemm.cpp:163-164,237-264)
 static std::vector<int2> pair_list(int nA, int nB, int fastMode) {
@@ -314,6 +324,50 @@ static int32_t gemm_narrow(ozblasHandle_t *oh, int m, int n, int k, T alpha, con
 	return OZBLAS_STATUS_SUCCESS;
 }
 
+static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int k, double alpha, const double *ain,
+                                 int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
+                                 int maxE, bool *handled);
+
+// ---------------------------------------------------------------------------------------------
+// GEMM, plain form with NearSum, at the bits of the residue form (binary64).  Where the split is complete
+// and no slice product can round, NearSum's result is RN of the exact inner product whatever the slices, and
+// the residue form computes that number from INT8 products.  *handled = false, with nothing written, where that
+// does not hold or the workspace does not hold the residue planes:
+//   - slices dropped (fastMode, nSplitMax) or other units (splitEpsMode, splitShift);
+//   - what fast_valid excludes (infinities, NaN, spans the split cap truncates, products near the ends of the
+//     exponent range), or a sigma near the upper end of it (maxE);
+//   - m = 1 or n = 1: the sum over the GEMV and DOT maps.
+// ---------------------------------------------------------------------------------------------
+static int32_t gemm_plain_residue(ozblasHandle_t *oh, int m, int n, int k, double alpha, const double *ain,
+                                  int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
+                                  int nA, int nB, bool *handled) {
+	Backend *b = be(oh);
+	*handled = false;
+	if (oh->fastMode != 0 || oh->splitEpsMode != 0 || oh->sumMode != 1 || b->mixed || m < 2 || n < 2)
+		return OZBLAS_STATUS_SUCCESS;
+	if ((double)nA * nB * m * n * (double)k < kPlainResidueWork) return OZBLAS_STATUS_SUCCESS;
+	const uint64_t base = wmark(oh);
+	const int tiles = oh->fallbackTiles, bins = oh->nLevelBins, scheme = oh->schemeUsed;
+	const float tA = oh->t_SplitA, tB = oh->t_SplitB;
+	OZ_HIP(hipEventRecord(b->ev[0], b->stream));
+	const int32_t s = gemm_residue_core(oh, 1, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, 900, handled);
+	wreset(oh, base);
+	if (s != OZBLAS_STATUS_SUCCESS) *handled = false;
+	oh->fallbackTiles = tiles;
+	oh->nLevelBins = bins;
+	oh->schemeUsed = scheme;
+	oh->t_SplitA = tA;
+	oh->t_SplitB = tB;
+	if (!*handled) return s == OZBLAS_STATUS_WORKSPACE ? OZBLAS_STATUS_SUCCESS : s;
+	oh->mbk = m;
+	oh->nbk = n;
+	oh->nSplitA = (float)nA;
+	oh->nSplitB = (float)nB;
+	oh->nSplitC = (float)nA * (float)nB;
+	oh->n_comp = (float)(2.0 * m * n * (double)k * oh->nSplitC);
+	return OZBLAS_STATUS_SUCCESS;
+}
+
 // ---------------------------------------------------------------------------------------------
 // GEMM, plain form (src/cpu/ozblas_gemm.cpp:3-315)
 // ---------------------------------------------------------------------------------------------
@@ -397,9 +451,9 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 	}
 	// blocking: slice counts of the whole operands bound those of any block, so halving the
 	// larger side (as src/cpu/ozblas_gemm.cpp:91-96) until the exact need fits is safe
-	int nAf = 0, nBf = 0, zAf = -1, zBf = -1;
-	OZ_TRY(count_cols(oh, k, m, ain, ldai, &nAf, &zAf));
-	OZ_TRY(count_cols(oh, k, n, bin, ldbi, &nBf, &zBf));
+	int nf[2], zf[2];
+	OZ_TRY(count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf));
+	const int nAf = nf[0], nBf = nf[1], zAf = zf[0], zBf = zf[1];
 	auto need = [&](int64_t mb, int64_t nb) -> uint64_t {
 		uint64_t bytes = 8ull * ldk * std::max(mb, nb) * 2;            // remainder + count scratch
 		bytes += 8ull * ldk * (mb * (nAf + 1) + nb * (nBf + 1));        // slices (+ remainder slot)
@@ -415,6 +469,17 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 			mbk = (mbk + 1) / 2;
 		else
 			nbk = (nbk + 1) / 2;
+	}
+	if constexpr (std::is_same<T, double>::value) {
+		if (mbk == m && nbk == n) {
+			bool handled = false;
+			OZ_TRY(gemm_plain_residue(oh, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, nAf, nBf, &handled));
+			if (handled) {
+				oh->t_total = tt.sec();
+				wreset(oh, base);
+				return OZBLAS_STATUS_SUCCESS;
+			}
+		}
 	}
 	oh->mbk = mbk;
 	oh->nbk = nbk;
@@ -767,33 +832,16 @@ static int32_t res_stats(ozblasHandle_t *oh, int k, int cols, const double *in, 
 	return OZBLAS_STATUS_SUCCESS;
 }
 
-static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m, int n, int k,
-                            double alpha, const double *A, int lda, const double *B, int ldb,
-                            double beta, double *C, int ldc, bool *handled) {
+// elem: the element of the residue planes (1 INT8, 2 FP16, 3 BF16); ain, bin: k-contiguous op(A), op(B)
+// (event 0 recorded before their transposition); not handled with elements of 2^maxE or more
+static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int k, double alpha, const double *ain,
+                                 int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
+                                 int maxE, bool *handled) {
 	Backend *b = be(oh);
 	hipStream_t st = b->stream;
 	*handled = false;
-	const int elem = (oh->sliceType == OZBLAS_SLICE_INT8) ? 1 : (oh->sliceType == OZBLAS_SLICE_FP16 ? 2 : 3);
 	const uint64_t base = wmark(oh);
 	WallTimer tt;
-	const int64_t ldk = rup(k, 16);
-	const double *ain = A, *bin = B;
-	int64_t ldai = lda, ldbi = ldb;
-	OZ_HIP(hipEventRecord(b->ev[0], st));
-	if (is_n(transA)) {
-		double *tA = (double *)walloc(oh, 8ull * ldk * m);
-		if (!tA) return OZBLAS_STATUS_WORKSPACE;
-		launch_transpose(st, m, k, A, lda, tA, ldk);
-		ain = tA;
-		ldai = ldk;
-	}
-	if (!is_n(transB)) {
-		double *tB = (double *)walloc(oh, 8ull * ldk * n);
-		if (!tB) return OZBLAS_STATUS_WORKSPACE;
-		launch_transpose(st, n, k, B, ldb, tB, ldk);
-		bin = tB;
-		ldbi = ldk;
-	}
 	ResOperand ra, rb;
 	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, 2 * kStatBytes);
 	if (!dst) return OZBLAS_STATUS_WORKSPACE;
@@ -808,7 +856,7 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 		wreset(oh, base);
 		return OZBLAS_STATUS_SUCCESS;
 	};
-	if (!fast_valid(oh, ra.st, rb.st, k)) return give_up();
+	if (!fast_valid(oh, ra.st, rb.st, k) || ra.st.maxE > maxE || rb.st.maxE > maxE) return give_up();
 	if (ra.st.maxS == 0 || rb.st.maxS == 0) {  // an all-zero operand: C = fma(alpha, +0, beta C)
 		*handled = true;
 		int *lv = (int *)walloc(oh, sizeof(int));
@@ -918,6 +966,39 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 	oh->nbk = n;
 	oh->t_total = tt.sec();
 	oh->n_comp = (float)(2.0 * m * n * (double)k * nmod);
+	wreset(oh, base);
+	return OZBLAS_STATUS_SUCCESS;
+}
+
+static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m, int n, int k,
+                            double alpha, const double *A, int lda, const double *B, int ldb,
+                            double beta, double *C, int ldc, bool *handled) {
+	Backend *b = be(oh);
+	hipStream_t st = b->stream;
+	*handled = false;
+	const int elem = (oh->sliceType == OZBLAS_SLICE_INT8) ? 1 : (oh->sliceType == OZBLAS_SLICE_FP16 ? 2 : 3);
+	const uint64_t base = wmark(oh);
+	WallTimer tt;
+	const int64_t ldk = rup(k, 16);
+	const double *ain = A, *bin = B;
+	int64_t ldai = lda, ldbi = ldb;
+	OZ_HIP(hipEventRecord(b->ev[0], st));
+	if (is_n(transA)) {
+		double *tA = (double *)walloc(oh, 8ull * ldk * m);
+		if (!tA) return OZBLAS_STATUS_WORKSPACE;
+		launch_transpose(st, m, k, A, lda, tA, ldk);
+		ain = tA;
+		ldai = ldk;
+	}
+	if (!is_n(transB)) {
+		double *tB = (double *)walloc(oh, 8ull * ldk * n);
+		if (!tB) return OZBLAS_STATUS_WORKSPACE;
+		launch_transpose(st, n, k, B, ldb, tB, ldk);
+		bin = tB;
+		ldbi = ldk;
+	}
+	OZ_TRY(gemm_residue_core(oh, elem, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, INT32_MAX, handled));
+	if (*handled) oh->t_total = tt.sec();
 	wreset(oh, base);
 	return OZBLAS_STATUS_SUCCESS;
 }
