@@ -56,7 +56,7 @@ def ozaki_mm(A: torch.Tensor, B: torch.Tensor, form: str = "int8", transA=False,
     k2, n = (B.shape[1], B.shape[0]) if transB else (B.shape[0], B.shape[1])
     if k != k2:
         raise ValueError(f"inner dimensions differ: {k} vs {k2}")
-    C = torch.empty((m, n), dtype=torch.float64, device=A.device)
+    C = torch.zeros((m, n), dtype=torch.float64, device=A.device)  # 0 C enters the result: NaN if C is
     h = _handle(form, _work_bytes(m, n, k))
     # column-major view: C^T (n x m) = op(B)^T (n x k) * op(A)^T (k x m)
     # a row-major R x S buffer is the column-major S x R matrix with ld = S

@@ -43,3 +43,16 @@ def test_residue_reconstruction_exact(oz, m, n, k, bits, shift):
     H.dgemm("N", "N", m, n, k, 2.0, dev(flat(A, m, k)), m, dev(flat(B, k, n)), k, -0.5, dC, m)
     assert H.schemeUsed == 2
     assert bits_equal(host(dC), want), first_diff(host(dC), want)
+
+
+def test_matmul_result_memory_is_not_an_input():
+    """beta = 0 multiplies C rather than dropping it (as the reference does), so the product must not start from
+    recycled memory: NaN left in it came out in the result."""
+    torch = torch_cuda()
+    from ozblas_amd.autograd import ozaki_mm
+    A, B = torch.ones((7, 5), dtype=torch.float64).cuda(), torch.ones((5, 6), dtype=torch.float64).cuda()
+    for form in ("int8", "fp16"):
+        for _ in range(3):
+            left = torch.full((7, 6), float("nan"), dtype=torch.float64, device="cuda")
+            del left  # back to the allocator, which hands it out for the next 7 x 6
+            assert bool((ozaki_mm(A, B, form) == 5.0).all())
