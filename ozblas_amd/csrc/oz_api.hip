@@ -164,21 +164,28 @@ static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const
 	for (int q = 0; q < 2; q++)
 		launch_split_cols(b->stream, k, cols[q], in[q], ldi[q], rem, ldk, scratch, ldk, 0, Prec<T>::rho(oh, k),
 		                  oh->splitShift, split_cap(oh), Prec<T>::Jsplit(b), zcol, b->dCounters + q);
-	OZ_HIP(hipMemcpyAsync(b->hPinned, b->dCounters, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
+	// behind the statistics of the residue form, which may be on their way too
+	int32_t *h = (int32_t *)((char *)b->hPinned + 2 * kStatBytes);
+	OZ_HIP(hipMemcpyAsync(h, b->dCounters, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
 	for (int q = 0; q < 2; q++) {
-		z[q] = ((int32_t *)b->hPinned)[q];
+		z[q] = h[q];
 		count[q] = split_count(oh, z[q]);
 	}
 	wreset(oh, mark);
 	return OZBLAS_STATUS_SUCCESS;
 }
 
-// Work (slice pairs times m n k) from which the residue form is the faster way to NearSum's bits.  Its
-// statistics, uploads and one more synchronisation cost what the FP64 products take below the line: 256^3, 16
-// pairs (2.7e8), 140 us by FP64 slices and 170 us by residues; 384^3 (9e8) 166 and 150; 128 x 128 x 2500
-// (6.6e8) 494 and 171; 2500 x 128 x 128, 12 pairs (4.9e8) 175 and 159; 2500 x 2301 x 2700 8,480 and 770.
-constexpr double kPlainResidueWork = 5e8;
+// Whether the residue form is the faster way to NearSum's bits: its statistics, writers and reconstruction cost
+// about 45 us more than splitting and summing a small product, while the FP64 kernel takes 0.17 us per element of k
+// for the 16 pairs of full mantissas until it fills the chip, 55 TFLOP/s from there on.  Measured by FP64 slices
+// and by residues: 128^3 88 and 108 us, 1024 x 64 x 128 110 and 118, 256^3 118 and 115, 2500 x 128 x 128 156 and
+// 136, 64 x 64 x 2500 515 and 146, 2500 x 2301 x 2700 8,480 and 730.
+static bool plain_residue_pays(double m, double n, double k, double pairs) {
+	return k >= 256 ? pairs >= 9 : pairs * m * n * k >= 4e8;
+}
+// slice pairs of full mantissas, by which that is judged before the slices are counted
+constexpr double kFullPairs = 16;
 
 // slice pairs of a GEMM in the reference's level order (src/cpu/ozblas_gemm.cpp:163-164,237-264)
 static std::vector<int2> pair_list(int nA, int nB, int fastMode) {
@@ -324,9 +331,18 @@ static int32_t gemm_narrow(ozblasHandle_t *oh, int m, int n, int k, T alpha, con
 	return OZBLAS_STATUS_SUCCESS;
 }
 
+struct ResOperand {
+	int *colE = nullptr, *colLo = nullptr;
+	ExpStatsH st{};
+	void *planes = nullptr;
+	int64_t ldp = 0, pstride = 0;
+};
+static int32_t res_stats(ozblasHandle_t *oh, int m, int n, int k, const double *ain, int64_t ldai, const double *bin,
+                         int64_t ldbi, ResOperand &ra, ResOperand &rb);
+static void res_stats_read(ozblasHandle_t *oh, ResOperand &ra, ResOperand &rb);
 static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int k, double alpha, const double *ain,
                                  int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
-                                 int maxE, bool *handled);
+                                 ResOperand &ra, ResOperand &rb, bool *handled);
 
 // ---------------------------------------------------------------------------------------------
 // GEMM, plain form with NearSum, at the bits of the residue form (binary64).  Where the split is complete
@@ -340,17 +356,15 @@ static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int
 // ---------------------------------------------------------------------------------------------
 static int32_t gemm_plain_residue(ozblasHandle_t *oh, int m, int n, int k, double alpha, const double *ain,
                                   int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
-                                  int nA, int nB, bool *handled) {
+                                  int nA, int nB, ResOperand &ra, ResOperand &rb, bool *handled) {
 	Backend *b = be(oh);
 	*handled = false;
-	if (oh->fastMode != 0 || oh->splitEpsMode != 0 || oh->sumMode != 1 || b->mixed || m < 2 || n < 2)
+	if (!plain_residue_pays(m, n, k, (double)nA * nB) || ra.st.maxE > 900 || rb.st.maxE > 900)
 		return OZBLAS_STATUS_SUCCESS;
-	if ((double)nA * nB * m * n * (double)k < kPlainResidueWork) return OZBLAS_STATUS_SUCCESS;
 	const uint64_t base = wmark(oh);
 	const int tiles = oh->fallbackTiles, bins = oh->nLevelBins, scheme = oh->schemeUsed;
 	const float tA = oh->t_SplitA, tB = oh->t_SplitB;
-	OZ_HIP(hipEventRecord(b->ev[0], b->stream));
-	const int32_t s = gemm_residue_core(oh, 1, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, 900, handled);
+	const int32_t s = gemm_residue_core(oh, 1, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, ra, rb, handled);
 	wreset(oh, base);
 	if (s != OZBLAS_STATUS_SUCCESS) *handled = false;
 	oh->fallbackTiles = tiles;
@@ -452,7 +466,20 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 	// blocking: slice counts of the whole operands bound those of any block, so halving the
 	// larger side (as src/cpu/ozblas_gemm.cpp:91-96) until the exact need fits is safe
 	int nf[2], zf[2];
+	ResOperand ra, rb;
+	bool residue = false;  // whether the residue form may be taken: its statistics come with the counts
+	if constexpr (std::is_same<T, double>::value) {
+		residue = fastMode == 0 && oh->splitEpsMode == 0 && !fsum && !b->mixed && m > 1 && n > 1 &&
+		          oh->nSplitMax == 0 && plain_residue_pays(m, n, k, kFullPairs);
+		if (residue) {
+			OZ_HIP(hipEventRecord(b->ev[0], st));
+			const int32_t s = res_stats(oh, m, n, k, ain, ldai, bin, ldbi, ra, rb);
+			if (s == OZBLAS_STATUS_WORKSPACE) residue = false;
+			else OZ_TRY(s);
+		}
+	}
 	OZ_TRY(count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf));
+	if (residue) res_stats_read(oh, ra, rb);
 	const int nAf = nf[0], nBf = nf[1], zAf = zf[0], zBf = zf[1];
 	auto need = [&](int64_t mb, int64_t nb) -> uint64_t {
 		uint64_t bytes = 8ull * ldk * std::max(mb, nb) * 2;            // remainder + count scratch
@@ -471,9 +498,10 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 			nbk = (nbk + 1) / 2;
 	}
 	if constexpr (std::is_same<T, double>::value) {
-		if (mbk == m && nbk == n) {
+		if (residue && mbk == m && nbk == n) {
 			bool handled = false;
-			OZ_TRY(gemm_plain_residue(oh, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, nAf, nBf, &handled));
+			OZ_TRY(gemm_plain_residue(oh, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, nAf, nBf, ra, rb,
+			                          &handled));
 			if (handled) {
 				oh->t_total = tt.sec();
 				wreset(oh, base);
@@ -576,13 +604,6 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 // ---------------------------------------------------------------------------------------------
 // GEMM, fast forms: exact digit planes (no reference counterpart; same bits as NearSum)
 // ---------------------------------------------------------------------------------------------
-// the empty statistics of two operands (the residue form reduces both in one block)
-static const ExpStatsSlot *stats_init() {
-	static const std::vector<ExpStatsSlot> init(
-	    2 * kStatSlots, ExpStatsSlot{ExpStatsH{0, INT32_MAX, INT32_MIN, 0, INT32_MIN, INT32_MIN, {0, 0}}});
-	return init.data();
-}
-
 struct DigitOperand {
 	void *planes = nullptr;
 	int64_t ldp = 0, pstride = 0;  // in elements
@@ -597,7 +618,7 @@ static int32_t digit_split(ozblasHandle_t *oh, int elem, int k, int cols, const 
 	d.colE = (int *)walloc(oh, sizeof(int) * (size_t)cols * 2);
 	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, kStatBytes);
 	if (!d.colE || !dst) return OZBLAS_STATUS_WORKSPACE;
-	OZ_HIP(hipMemcpyAsync(dst, stats_init(), kStatBytes, hipMemcpyHostToDevice, b->stream));
+	launch_stats_init(b->stream, dst, kStatSlots);
 	launch_digit_stats(b->stream, k, cols, in, ldi, d.colE, d.colE + cols, dst);
 	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, kStatBytes, hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
@@ -815,48 +836,72 @@ static int32_t gemm_fast(ozblasHandle_t *oh, char transA, char transB, int m, in
 // (oz_residue.hip).  Returns with *handled = false when the moduli cannot cover the product (the
 // caller then takes the digit form or the plain form).
 // ---------------------------------------------------------------------------------------------
-struct ResOperand {
-	int *colE = nullptr, *colLo = nullptr;
-	ExpStatsH st{};
-	void *planes = nullptr;
-	int64_t ldp = 0, pstride = 0;
-};
+// statistics of op(A) and op(B), k-contiguous, on their way to the host; res_stats_read once the stream has
+// been waited for (the one host round trip: they decide the number of moduli)
+static int32_t res_stats(ozblasHandle_t *oh, int m, int n, int k, const double *ain, int64_t ldai, const double *bin,
+                         int64_t ldbi, ResOperand &ra, ResOperand &rb) {
+	Backend *b = be(oh);
+	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, 2 * kStatBytes);
+	ra.colE = (int *)walloc(oh, sizeof(int) * (size_t)m * 3);
+	rb.colE = (int *)walloc(oh, sizeof(int) * (size_t)n * 3);
+	if (!dst || !ra.colE || !rb.colE) return OZBLAS_STATUS_WORKSPACE;
+	ra.colLo = ra.colE + 2 * (size_t)m;
+	rb.colLo = rb.colE + 2 * (size_t)n;
+	launch_stats_init(b->stream, dst, 2 * kStatSlots);
+	launch_digit_stats(b->stream, k, m, ain, ldai, ra.colE, ra.colE + m, dst, ra.colLo);
+	launch_digit_stats(b->stream, k, n, bin, ldbi, rb.colE, rb.colE + n, dst + kStatSlots, rb.colLo);
+	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, 2 * kStatBytes, hipMemcpyDeviceToHost, b->stream));
+	return OZBLAS_STATUS_SUCCESS;
+}
+static void res_stats_read(ozblasHandle_t *oh, ResOperand &ra, ResOperand &rb) {
+	ra.st = merge_stats((const ExpStatsSlot *)be(oh)->hPinned);
+	rb.st = merge_stats((const ExpStatsSlot *)be(oh)->hPinned + kStatSlots);
+}
 
-// dst: the operand's kStatSlots statistics slots, initialised by the caller
-static int32_t res_stats(ozblasHandle_t *oh, int k, int cols, const double *in, int64_t ldi,
-                         ResOperand &r, ExpStatsSlot *dst) {
-	r.colE = (int *)walloc(oh, sizeof(int) * (size_t)cols * 3);
-	if (!r.colE) return OZBLAS_STATUS_WORKSPACE;
-	r.colLo = r.colE + 2 * (size_t)cols;
-	launch_digit_stats(be(oh)->stream, k, cols, in, ldi, r.colE, r.colE + cols, dst, r.colLo);
+// The device copies of res_const_host(nmod) and res_tab_host(nmod) (nullptr beyond kResTabMod), kept by the
+// handle from the first product of so many moduli on: at most kResMaxMod pairs of 95 KB.  Uploaded on each
+// call they cost two staged copies, 35 us of a small product.
+static int32_t res_device_consts(ozblasHandle_t *oh, int nmod, const ResConst **rc, const ResTab **tab) {
+	Backend *b = be(oh);
+	const uint64_t off = (sizeof(ResConst) + 255) & ~uint64_t(255);
+	const bool withTab = nmod <= kResTabMod;
+	char *p = b->resConst[nmod];
+	if (!p) {
+		const uint64_t bytes = off + (withTab ? sizeof(ResTab) : 0);
+		bool kept = true;
+		if (hipMalloc((void **)&p, bytes) != hipSuccess) {  // no device memory left: in the workspace, this call's
+			(void)hipGetLastError();
+			kept = false;
+			if (!(p = (char *)walloc(oh, bytes))) return OZBLAS_STATUS_WORKSPACE;
+		}
+		// on the product's stream, in order with the kernels that read them
+		hipError_t err = hipMemcpyAsync(p, &res_const_host(nmod), sizeof(ResConst), hipMemcpyHostToDevice, b->stream);
+		if (err == hipSuccess && withTab)
+			err = hipMemcpyAsync(p + off, &res_tab_host(nmod), sizeof(ResTab), hipMemcpyHostToDevice, b->stream);
+		if (kept && err == hipSuccess) b->resConst[nmod] = p;
+		if (kept && err != hipSuccess) (void)hipFree(p);
+		OZ_HIP(err);
+	}
+	*rc = (const ResConst *)p;
+	*tab = withTab ? (const ResTab *)(p + off) : nullptr;
 	return OZBLAS_STATUS_SUCCESS;
 }
 
 // elem: the element of the residue planes (1 INT8, 2 FP16, 3 BF16); ain, bin: k-contiguous op(A), op(B)
-// (event 0 recorded before their transposition); not handled with elements of 2^maxE or more
+// (event 0 recorded before their transposition); ra, rb: their statistics
 static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int k, double alpha, const double *ain,
                                  int64_t ldai, const double *bin, int64_t ldbi, double beta, double *C, int ldc,
-                                 int maxE, bool *handled) {
+                                 ResOperand &ra, ResOperand &rb, bool *handled) {
 	Backend *b = be(oh);
 	hipStream_t st = b->stream;
 	*handled = false;
 	const uint64_t base = wmark(oh);
 	WallTimer tt;
-	ResOperand ra, rb;
-	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, 2 * kStatBytes);
-	if (!dst) return OZBLAS_STATUS_WORKSPACE;
-	OZ_HIP(hipMemcpyAsync(dst, stats_init(), 2 * kStatBytes, hipMemcpyHostToDevice, st));
-	OZ_TRY(res_stats(oh, k, m, ain, ldai, ra, dst));
-	OZ_TRY(res_stats(oh, k, n, bin, ldbi, rb, dst + kStatSlots));
-	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, 2 * kStatBytes, hipMemcpyDeviceToHost, st));
-	OZ_TRY(sync(oh));  // the one host round trip: the statistics decide the number of moduli
-	ra.st = merge_stats((const ExpStatsSlot *)b->hPinned);
-	rb.st = merge_stats((const ExpStatsSlot *)b->hPinned + kStatSlots);
 	auto give_up = [&]() {
 		wreset(oh, base);
 		return OZBLAS_STATUS_SUCCESS;
 	};
-	if (!fast_valid(oh, ra.st, rb.st, k) || ra.st.maxE > maxE || rb.st.maxE > maxE) return give_up();
+	if (!fast_valid(oh, ra.st, rb.st, k)) return give_up();
 	if (ra.st.maxS == 0 || rb.st.maxS == 0) {  // an all-zero operand: C = fma(alpha, +0, beta C)
 		*handled = true;
 		int *lv = (int *)walloc(oh, sizeof(int));
@@ -879,9 +924,6 @@ static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int
 	while (nmod <= kResMaxMod && res_log2_product(nmod) < need + 1e-6) nmod++;
 	if (nmod > kResMaxMod) return give_up();
 	const ResConst &rc = res_const_host(nmod);
-	ResConst *dRc = (ResConst *)walloc(oh, sizeof(ResConst));
-	ResTab *dTab = nullptr;
-	if (nmod <= kResTabMod && !(dTab = (ResTab *)walloc(oh, sizeof(ResTab)))) return give_up();
 	if (elem == 1) {
 		ra.ldp = rb.ldp = rup(k, 128);
 		ra.pstride = ra.ldp * rup(m, 256);
@@ -906,39 +948,38 @@ static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int
 	// registers leave no room to flush inside the loop
 	if (elem != 1 || tile == 256) ngroups = nmod;
 	const int G = (nmod + ngroups - 1) / ngroups;
-	std::vector<int2> pairs(nmod);
-	std::vector<LevelBin> bins;
-	for (int t = 0; t < nmod; t++) pairs[t] = make_int2(t, t);
-	for (int c = 0; c < nchunk; c++)
-		for (int t0 = 0; t0 < nmod; t0 += G) {
-			LevelBin bn;
+	// pairs, bins and their order in one block, one upload
+	const int nbins = nchunk * ((nmod + G - 1) / G);
+	const size_t binsAt = sizeof(int2) * (size_t)nmod, orderAt = binsAt + sizeof(LevelBin) * (size_t)nbins;
+	std::vector<char> items(orderAt + sizeof(int) * (size_t)nbins);
+	for (int t = 0; t < nmod; t++) ((int2 *)items.data())[t] = make_int2(t, t);
+	for (int c = 0, q = 0; c < nchunk; c++)
+		for (int t0 = 0; t0 < nmod; t0 += G, q++) {
+			LevelBin &bn = ((LevelBin *)(items.data() + binsAt))[q];
 			bn.level = t0;
 			bn.pair0 = t0;
 			bn.npairs = std::min(G, nmod - t0);
 			bn.k0 = c * kc;
 			bn.k1 = std::min(Kpad, (c + 1) * kc);
-			bins.push_back(bn);
+			((int *)(items.data() + orderAt))[q] = q;
 		}
-	const int nbins = (int)bins.size();
-	std::vector<int> order(nbins);
-	for (int q = 0; q < nbins; q++) order[q] = q;
 	// product residues: whole INT8 tiles, or (FP16/BF16) every 4-column word of the m x n product
 	const int64_t ldt = (elem == 1) ? rup(m, 256) : rup(m, 64);
 	const int64_t tstride = ldt * ((elem == 1) ? rup(n, 256) : rup(n, 4));
-	int2 *dPairs = (int2 *)walloc(oh, sizeof(int2) * pairs.size());
-	LevelBin *dBins = (LevelBin *)walloc(oh, sizeof(LevelBin) * bins.size());
-	int *dOrder = (int *)walloc(oh, sizeof(int) * order.size());
+	char *dItems = (char *)walloc(oh, items.size());
 	uint8_t *Rp = (uint8_t *)walloc(oh, (size_t)tstride * nmod * nchunk);
-	if (!dRc || !ra.planes || !rb.planes || !dPairs || !dBins || !dOrder || !Rp) {
+	if (!ra.planes || !rb.planes || !dItems || !Rp) {
 		wreset(oh, base);
 		return OZBLAS_STATUS_WORKSPACE;
 	}
+	const ResConst *dRc;
+	const ResTab *dTab;
+	OZ_TRY(res_device_consts(oh, nmod, &dRc, &dTab));
 	*handled = true;
-	OZ_HIP(hipMemcpyAsync(dRc, &rc, sizeof(ResConst), hipMemcpyHostToDevice, st));
-	if (dTab) OZ_HIP(hipMemcpyAsync(dTab, &res_tab_host(nmod), sizeof(ResTab), hipMemcpyHostToDevice, st));
-	OZ_HIP(hipMemcpyAsync(dPairs, pairs.data(), sizeof(int2) * pairs.size(), hipMemcpyHostToDevice, st));
-	OZ_HIP(hipMemcpyAsync(dBins, bins.data(), sizeof(LevelBin) * bins.size(), hipMemcpyHostToDevice, st));
-	OZ_HIP(hipMemcpyAsync(dOrder, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice, st));
+	OZ_HIP(hipMemcpyAsync(dItems, items.data(), items.size(), hipMemcpyHostToDevice, st));
+	const int2 *dPairs = (const int2 *)dItems;
+	const LevelBin *dBins = (const LevelBin *)(dItems + binsAt);
+	const int *dOrder = (const int *)(dItems + orderAt);
 	OZ_HIP(hipEventRecord(b->ev[1], st));
 	launch_res_write(st, elem, k, m, ain, ldai, ra.colLo, dRc, nmod, ra.st.maxSpan, 1, ra.planes, ra.ldp, ra.pstride);
 	OZ_HIP(hipEventRecord(b->ev[2], st));
@@ -997,7 +1038,11 @@ static int32_t gemm_residue(ozblasHandle_t *oh, char transA, char transB, int m,
 		bin = tB;
 		ldbi = ldk;
 	}
-	OZ_TRY(gemm_residue_core(oh, elem, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, INT32_MAX, handled));
+	ResOperand ra, rb;
+	OZ_TRY(res_stats(oh, m, n, k, ain, ldai, bin, ldbi, ra, rb));
+	OZ_TRY(sync(oh));
+	res_stats_read(oh, ra, rb);
+	OZ_TRY(gemm_residue_core(oh, elem, m, n, k, alpha, ain, ldai, bin, ldbi, beta, C, ldc, ra, rb, handled));
 	if (*handled) oh->t_total = tt.sec();
 	wreset(oh, base);
 	return OZBLAS_STATUS_SUCCESS;

@@ -215,6 +215,7 @@ extern "C" int32_t ozblasDestroy(ozblasHandle_t *oh) {
 	(void)hipFree(b->dTauF2);
 	(void)hipFree(b->dCounters);
 	(void)hipFree(b->vz);
+	for (char *p : b->resConst) (void)hipFree(p);
 	(void)hipHostFree(b->hPinned);
 	delete b;
 	oh->backend = nullptr;

@@ -61,6 +61,7 @@ struct Backend {
 	char *vz = nullptr;
 	int vzPar[2] = {0, 0};
 	bool vzDirty = true;
+	char *resConst[64] = {};  // per number of moduli: the residue form's constants on the device
 	char *scratch = nullptr;  // this device's copy of the static scratch array (ozblasDdotNoAlloc)
 };
 
@@ -401,7 +402,7 @@ struct alignas(64) ExpStatsSlot {
 	ExpStatsH s;
 };
 constexpr uint64_t kStatBytes = kStatSlots * sizeof(ExpStatsSlot);
-static_assert(2 * kStatBytes <= kPinnedBytes);
+static_assert(2 * kStatBytes + 64 <= kPinnedBytes);
 inline ExpStatsH merge_stats(const ExpStatsSlot *p) {
 	ExpStatsH r = p[0].s;
 	for (int q = 1; q < kStatSlots; q++) {

@@ -37,6 +37,7 @@ void launch_split_csr(hipStream_t st, int m, int nnz, const float *val, const in
                       int *zmax, int epsMode, int mixed = 0);
 void launch_zero_slots_csr(hipStream_t st, int m, const int *rowptr, double *split, int64_t lds,
                            const int *zrow, int count);
+void launch_stats_init(hipStream_t st, ExpStatsSlot *slots, int count);  // the empty statistics
 void launch_digit_stats(hipStream_t st, int m, int n, const double *in, int64_t ldi, int *colE,
                         int *colS, void *stats, int *colLo = nullptr);
 void launch_digit_write(hipStream_t st, int elem, int m, int n, const double *in, int64_t ldi,

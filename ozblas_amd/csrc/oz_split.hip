@@ -527,6 +527,15 @@ void launch_zero_slots_csr(hipStream_t st, int m, const int *rowptr, double *spl
 	                   lds, zrow, count);
 }
 
+__global__ __launch_bounds__(64) void k_stats_init(ExpStatsSlot *slots, int count) {
+	for (int q = threadIdx.x; q < count; q += 64)
+		slots[q].s = ExpStatsH{0, INT32_MAX, INT32_MIN, 0, INT32_MIN, INT32_MIN, {0, 0}};
+}
+
+void launch_stats_init(hipStream_t st, ExpStatsSlot *slots, int count) {
+	hipLaunchKernelGGL(k_stats_init, dim3(1), dim3(64), 0, st, slots, count);
+}
+
 void launch_digit_stats(hipStream_t st, int m, int n, const double *in, int64_t ldi, int *colE,
                         int *colS, void *stats, int *colLo) {
 	const int grid = n < 2048 ? n : 2048;  // columns per workgroup share its few counter atomics
