@@ -427,15 +427,27 @@ struct I8Tile {
 	const ResConst *rc;
 };
 
-// v mod p in [0, p) for |v| <= 2^30 and 3 <= p <= 256, in binary64 without a correction step:
-// q = floor(fma(v, RN(1/p), 2^-10)) is floor(v / p) exactly -- the fma's error, below
-// |v/p| 2^-53 + 2^-23 < 2^-22, and the offset 2^-10 stay inside the gap of at least 1/p >= 2^-8 that
-// separates a non-integer v/p from the integer above it, and the offset lifts an integer v/p off the
-// one below -- so r = v - q p, exact in one fma, is the canonical residue.
-__device__ __forceinline__ int mod_f64(int v, double p, double invp) {
-	const double vd = (double)v;
-	const double q = floor(fma(vd, invp, 0x1p-10));
-	return (int)fma(-q, p, vd);
+// The low byte of the canonical residue v mod p, for a sum v of products of balanced residues modulo p <= 256
+// over up to 65536 k (|v| <= p^2 / 4 2^16, so |v / p| <= 2^22 p / 256), negp = -p.  The fma leaves v / p + 2^-9
+// in units of 2^-9 in the low word of its result, off by at most 2^-10 (and 2^-31 from RN(1/p)); offset and error
+// together stay above 0 and below 1/p >= 2^-8, the gap between a non-integer v/p and the integer above it.  So the
+// word without its 9 fraction bits is q = floor(v / p), and r = v - q p takes one 24-bit multiply-add.  The word
+// overflows for p = 256 and v = 2^30 alone, where r's low byte is v's whatever q.
+// In binary64 throughout (floor, a second fma, conversion back) the 2500 x 2301 x 2700 product of 22 moduli took
+// 381 us, with this 351; 8192^3 with 23 moduli 10.2 and 9.8 ms.
+__host__ __device__ __forceinline__ int mod_residue(int v, double invp, int negp) {
+	const double t = fma((double)v, invp, 0x1.8p43 + 0x1p-9);
+	const int q = (int)(uint32_t)__builtin_bit_cast(uint64_t, t) >> 9;
+#ifdef __HIP_DEVICE_COMPILE__
+	return v + __mul24(q, negp);
+#else
+	return v + q * negp;
+#endif
+}
+// the low bytes of four residues as one word
+__device__ __forceinline__ uint32_t pack_low_bytes(int r0, int r1, int r2, int r3) {
+	return __builtin_amdgcn_perm((uint32_t)r1, (uint32_t)r0, 0x0c0c0400) |
+	       __builtin_amdgcn_perm((uint32_t)r3, (uint32_t)r2, 0x04000c0c);
 }
 
 // Product residues of the residue form: one byte per element, four consecutive columns of a row
@@ -591,7 +603,7 @@ __device__ __forceinline__ void i8_tile(const I8Tile &g, char *stage0, char *sta
 			if (--left > 0) return;
 			left = kst;
 			const int t = g.s0 + mq++;
-			const double p = (double)g.rc->p[t];
+			const int negp = -g.rc->p[t];
 			const double invp = g.rc->invpd[t];
 			uint8_t *Rb = g.R + (int64_t)t * g.rstride;
 			// |acc| <= 2^14 k <= 2^30 (chunks of at most 65536 k)
@@ -603,13 +615,13 @@ __device__ __forceinline__ void i8_tile(const I8Tile &g, char *stage0, char *sta
 					for (int r4 = 0; r4 < 4; r4++) {
 						const int i = i0 + wm + 32 * mi + l % 32;
 						const int j = j0 + wn + 32 * nj + 8 * r4 + 4 * (l / 32);
-						uint32_t w = 0;
+						int r[4];
 #pragma unroll
 						for (int c = 0; c < 4; c++) {
-							w |= (uint32_t)mod_f64(acc[mi][nj][4 * r4 + c], p, invp) << (8 * c);
+							r[c] = mod_residue(acc[mi][nj][4 * r4 + c], invp, negp);
 							acc[mi][nj][4 * r4 + c] = 0;
 						}
-						*(uint32_t *)(Rb + res_word_offset(i, j, g.ldt)) = w;
+						*(uint32_t *)(Rb + res_word_offset(i, j, g.ldt)) = pack_low_bytes(r[0], r[1], r[2], r[3]);
 					}
 		}
 	};

@@ -410,3 +410,9 @@ extern "C" int32_t ozblas_internal_res_const(int32_t nmod, void *out, uint64_t b
 }
 
 extern "C" double ozblas_internal_res_log2(int32_t nmod) { return oz::res_log2_product(nmod); }
+
+// test hook: the low bytes of v[i] mod p as the product kernels form them
+extern "C" void ozblas_internal_mod_residue(int32_t n, const int32_t *v, int32_t p, uint8_t *out) {
+	const double invp = 1.0 / (double)p;
+	for (int32_t i = 0; i < n; i++) out[i] = (uint8_t)oz::mod_residue(v[i], invp, -p);
+}

@@ -123,10 +123,8 @@ __device__ inline void res_write_tile_i8(int m, int n, const double *in, int64_t
 				uint32_t r[4];
 #pragma unroll
 				for (int u = 0; u < 4; u++) r[u] = res_member_byte(rf[u], ri[u], mp.x, negp);
-				// the four low bytes as one word
-				const uint32_t lo = __builtin_amdgcn_perm(r[1], r[0], 0x0c0c0400);
-				const uint32_t hi = __builtin_amdgcn_perm(r[3], r[2], 0x04000c0c);
-				*(uint32_t *)(dst + (int64_t)s * pstride) = lo | hi;
+				*(uint32_t *)(dst + (int64_t)s * pstride) =
+				    pack_low_bytes((int)r[0], (int)r[1], (int)r[2], (int)r[3]);
 			}
 		}
 	}
