@@ -76,3 +76,23 @@ def test_non_finite(oz, oracle, bad):
     assert np.array_equal(np.isfinite(got), np.isfinite(want))
     ok = np.isfinite(want)
     assert bits_equal(got[ok], want[ok])
+
+
+@pytest.mark.parametrize("form", ["fp16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(3, 5, 700), (70, 33, 129), (130, 260, 500)])
+@pytest.mark.parametrize("work", [1 << 30, 4 << 20])
+def test_half_forms_residues(oz, oracle, form, m, n, k, work):
+    """FP16 and BF16 residues: INT8 planes, or planes of their own where a tight workspace does not hold those."""
+    rng = np.random.default_rng(m)
+    A, B = rng.standard_normal(m * k), rng.standard_normal(k * n)
+    want = oracle.exact_gemm_rn("N", "N", m, n, k, A, m, B, k).ravel(order="F")  # m x n to column-major
+    H = oz.Handle(work, sumMode=1, sliceType=form, digitScheme=2)
+    C = dev(np.zeros(m * n))
+    say(f"half form {form} {m}x{n}x{k} work={work}")
+    try:
+        H.dgemm("N", "N", m, n, k, 1.0, dev(A), m, dev(B), k, 0.0, C, m)
+    except Exception as e:  # 130 x 260 x 500 needs more than 4 MB in either layout
+        assert work == 4 << 20 and m == 130, e
+        return
+    assert H.schemeUsed == 2
+    assert bits_equal(host(C), want), first_diff(host(C), want)
