@@ -740,7 +740,7 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 				w.scaleU = side == 0 ? 1 : 0;
 				w.rcw = (const ResConst *)(M2 + rcOff[h.nmod]);
 				writeStart.push_back(wb);
-				wb += (int)(rup64(w.n, 256) / 16);
+				wb += (w.n + 15) / 16;
 				hWrite.push_back(w);
 			}
 			for (int c = 0; c < 2; c++) {

@@ -290,7 +290,7 @@ void launch_res_write(hipStream_t st, int elem, int m, int n, const double *in, 
 	if (elem == 1) {  // tiled layout; ldp % 128 == 0 and pstride = ldp * (n rounded up to 256)
 		const int ktiles = (int)(ldp / 64);
 		const int gx = ktiles < 16 ? ktiles : 16;
-		hipLaunchKernelGGL(k_res_write_i8t, dim3((unsigned)gx, (unsigned)(pstride / ldp / 16)), dim3(256),
+		hipLaunchKernelGGL(k_res_write_i8t, dim3((unsigned)gx, (unsigned)((n + 15) / 16)), dim3(256),
 		                   res_lds_bytes(nmod, shLimit), st, m, n, in, ldi, colLo, rc, nmod, shLimit, scaleU,
 		                   (int8_t *)planes, ldp, pstride);
 		return;

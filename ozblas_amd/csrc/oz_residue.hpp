@@ -84,12 +84,13 @@ __device__ inline void res_lds_load(ResLds &T, const ResConst *rc, int nmod, int
 }
 
 // One 256-thread workgroup: residues of the 16 columns x 64 k-bytes tile (kt, jb) of every modulus
-// plane in the INT8 tiled layout (4 bytes per thread).
+// plane in the INT8 tiled layout (4 bytes per thread).  The blocks of 16 columns beyond n, up to the tile size of the
+// product, are not written: what they hold only enters product elements outside the m x n result.
 __device__ inline void res_write_tile_i8(int m, int n, const double *in, int64_t ldi, const int *colLo,
                                          int nmod, const ResLds &T, int8_t *planes, int64_t ldp,
                                          int64_t pstride, int kt, int jb) {
 	const int t = threadIdx.x;
-	if (jb * 16 >= n || kt * 64 >= m) {  // a tile of padding only: zero residues, nothing to compute
+	if (kt * 64 >= m) {  // a tile of k padding only: zero residues, nothing to compute
 		int8_t *dst = planes + (int64_t)jb * 16 * ldp + (int64_t)kt * 1024 + 4 * t;
 		for (int s = 0; s < nmod; s++) *(uint32_t *)(dst + (int64_t)s * pstride) = 0u;
 		return;
