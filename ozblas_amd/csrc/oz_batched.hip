@@ -64,12 +64,10 @@ struct GProb {  // one problem of the grouped MFMA launch
 	int64_t apstride, bpstride, ldp;
 	uint8_t *R;  // residue planes of the products, one per (modulus, k chunk)
 	int64_t ldt, tstride;
-	const LevelBin *bins;
-	const int2 *pairs;
 	int tilesM, nmod;
 };
 struct GItem {
-	int prob, bin, tile, pad;
+	int prob, mod, chunk, tile;  // first modulus (256 x 256 tiles: the only one; 128 x 128: of all), k chunk
 };
 struct GRec {  // Chinese-remainder reconstruction + epilogue of one problem
 	const uint8_t *R;
@@ -210,8 +208,13 @@ __global__ __launch_bounds__(256) void k_write_grouped(const GWrite *g, const in
 		res_write_tile_i8(w.m, w.n, w.in, w.ldi, w.colLo, w.nmod, T, w.planes, w.ldp, w.pstride, kt, jb);
 }
 
-// Persistent grouped MFMA launch: every workgroup takes the next (problem, bin, tile) item from
-// the counter until the list is exhausted.  Items are sorted by decreasing cost.
+// Persistent grouped MFMA launch: every workgroup starts with the item of its own number and then takes the next
+// (problem, modulus, chunk, tile) item from the counter until the list is exhausted.  Items are sorted by decreasing
+// cost, and an item is two dependent scalar loads away (the list, the problem).  128 x 128 tiles run two workgroups a
+// CU (256 registers a lane) and claim the next item before the current one is computed, so the counter's latency is
+// not waited for; the 256 x 256 tile has no register left to hold the claim.  256 products of 64 to 1024: 128 x 128
+// tiles 4.45 ms with the item read through tables of bins and pairs (more registers, one workgroup a CU), now 2.35;
+// 256 x 256 tiles 2.8 before and after.
 template <int TM, int TN>
 __global__ __launch_bounds__(256, 1) void k_gemm_grouped(const GProb *P, const GItem *items,
                                                          int nitems, int *counter, const int *flag,
@@ -221,36 +224,35 @@ __global__ __launch_bounds__(256, 1) void k_gemm_grouped(const GProb *P, const G
 	__shared__ __attribute__((aligned(16))) char stage1[(TBM + TBN) * I8_BK];
 	__shared__ int next;
 	if (*flag) return;  // the plan check failed: the call will be planned again
-	for (;;) {
-		if (threadIdx.x == 0) next = atomicAdd(counter, 1);
-		__syncthreads();  // also: the previous item's LDS traffic is complete
-		// uniform across the workgroup: the item and problem tables are then read with scalar loads
-		const int it = __builtin_amdgcn_readfirstlane(next);
-		__syncthreads();
-		if (it >= nitems) break;
-		const GItem w = items[it];
-		const GProb p = P[w.prob];
-		const LevelBin bin = p.bins[w.bin];
-		const int2 st0 = p.pairs[bin.pair0];
+	// tables of the plan, not written while kernels run: the constant address space, for scalar loads
+	const auto *cItems = (const __attribute__((address_space(4))) GItem *)items;
+	const auto *cP = (const __attribute__((address_space(4))) GProb *)P;
+	int it = blockIdx.x;
+	while (it < nitems) {
+		int claimed = 0;
+		if (TM == 2 && threadIdx.x == 0) claimed = (int)gridDim.x + atomicAdd(counter, 1);
+		const int prob = cItems[it].prob, tile = cItems[it].tile, tilesM = cP[prob].tilesM, nmod = cP[prob].nmod;
 		I8Tile g;
-		g.A = p.A;
-		g.B = p.B;
-		g.apstride = p.apstride;
-		g.bpstride = p.bpstride;
-		g.ldp = p.ldp;
-		g.s0 = st0.x;
-		g.t0 = st0.y;
-		g.npairs = bin.npairs;
-		g.k0 = bin.k0;
-		g.k1 = bin.k1;
-		g.i0 = (w.tile % p.tilesM) * TBM;
-		g.j0 = (w.tile / p.tilesM) * TBN;
+		g.A = cP[prob].A;
+		g.B = cP[prob].B;
+		g.apstride = cP[prob].apstride;
+		g.bpstride = cP[prob].bpstride;
+		g.ldp = cP[prob].ldp;
+		g.s0 = g.t0 = cItems[it].mod;
+		g.npairs = TM == 4 ? 1 : nmod;
+		g.k0 = cItems[it].chunk * kResChunk;
+		g.k1 = (int)min(g.ldp, (int64_t)g.k0 + kResChunk);
+		g.i0 = (tile % tilesM) * TBM;
+		g.j0 = (tile / tilesM) * TBN;
 		g.T = nullptr;
-		g.ldt = p.ldt;
-		g.R = p.R + (int64_t)(bin.k0 / kResChunk) * p.nmod * p.tstride;  // bin: moduli over one k chunk
-		g.rstride = p.tstride;
+		g.ldt = cP[prob].ldt;
+		g.rstride = cP[prob].tstride;
+		g.R = cP[prob].R + (int64_t)cItems[it].chunk * nmod * g.rstride;
 		g.rc = rc;
 		i8_tile<TM, TN, true>(g, stage0, stage1);
+		if (threadIdx.x == 0) next = TM == 2 ? claimed : (int)gridDim.x + atomicAdd(counter, 1);
+		__syncthreads();  // also: the item's LDS traffic is complete
+		it = __builtin_amdgcn_readfirstlane(next);  // overwritten only behind the next item's barriers
 	}
 }
 
@@ -585,7 +587,6 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 		int q, nmod, nchunk, budget;
 		int64_t ldp, apstride, bpstride, ldt, tstride;
 		uint64_t planesA, planesB, R;
-		int bin0[2], nbins[2];  // per tile shape: all moduli of a chunk per bin (128), one modulus (256)
 	};
 	std::vector<ProbH> probs;
 	for (int q : live) {
@@ -620,9 +621,6 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	}
 	const int cap = split_cap(oh);
 	Layout L2;
-	std::vector<LevelBin> hBins;  // the bins of both tile shapes
-	std::vector<int2> hPairs;
-	for (int t = 0; t < kResMaxMod; t++) hPairs.push_back(make_int2(t, t));  // product t: plane t x plane t
 	std::vector<int> usedNmod;
 	for (ProbH &h : probs) {
 		const int q = h.q;
@@ -631,39 +629,11 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 		h.bpstride = h.ldp * rup64(n[q], 256);
 		h.ldt = rup64(m[q], 256);
 		h.tstride = h.ldt * rup64(n[q], 256);
-		h.nbins[0] = h.nbins[1] = 0;
-		h.bin0[0] = h.bin0[1] = (int)hBins.size();
 		h.nchunk = 1;
 		if (h.nmod > 0) {
 			h.planesA = L2.take((uint64_t)h.apstride * h.nmod);
 			h.planesB = L2.take((uint64_t)h.bpstride * h.nmod);
-			const int Kpad = (int)h.ldp;
-			const int kc = kResChunk;
-			h.nchunk = (Kpad + kc - 1) / kc;
-			// 128 x 128 tiles: one item streams every modulus of a tile and chunk through one
-			// pipeline; 256 x 256 tiles: one modulus per item
-			for (int c = 0; c < h.nchunk; c++) {
-				LevelBin bn;
-				bn.level = 0;
-				bn.pair0 = 0;
-				bn.npairs = h.nmod;
-				bn.k0 = c * kc;
-				bn.k1 = std::min(Kpad, (c + 1) * kc);
-				hBins.push_back(bn);
-			}
-			h.nbins[0] = (int)hBins.size() - h.bin0[0];
-			h.bin0[1] = (int)hBins.size();
-			for (int c = 0; c < h.nchunk; c++)
-				for (int t = 0; t < h.nmod; t++) {
-					LevelBin bn;
-					bn.level = t;
-					bn.pair0 = t;
-					bn.npairs = 1;
-					bn.k0 = c * kc;
-					bn.k1 = std::min(Kpad, (c + 1) * kc);
-					hBins.push_back(bn);
-				}
-			h.nbins[1] = (int)hBins.size() - h.bin0[1];
+			h.nchunk = (int)((h.ldp + kResChunk - 1) / kResChunk);
 			h.R = L2.take((uint64_t)h.tstride * h.nmod * h.nchunk);
 			p->totalPairs += h.nmod;
 			p->ops += 2.0 * m[q] * (double)n[q] * k[q] * h.nmod;
@@ -688,14 +658,12 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	std::vector<GProb> hProb[2];
 	std::vector<GItem> hItems[2];
 	std::vector<double> itemCost[2];
-	const uint64_t binsOff = L2.take(sizeof(LevelBin) * (hBins.size() + 1));
-	const uint64_t pairsOff = L2.take(sizeof(int2) * (hPairs.size() + 1));
 	// sizes of the remaining tables are known from probs
 	size_t nItemsMax[2] = {0, 0};
 	for (const ProbH &h : probs)
 		for (int c = 0; c < 2; c++) {
 			const int TB = c == 0 ? 128 : 256;
-			nItemsMax[c] += (size_t)h.nbins[c] * ((m[h.q] + TB - 1) / TB) * ((n[h.q] + TB - 1) / TB);
+			nItemsMax[c] += (size_t)(c == 0 ? 1 : h.nmod) * h.nchunk * ((m[h.q] + TB - 1) / TB) * ((n[h.q] + TB - 1) / TB);
 		}
 	const uint64_t writeOff = L2.take(sizeof(GWrite) * (2 * probs.size() + 1));
 	const uint64_t writeStartOff = L2.take(4 * (2 * probs.size() + 1));
@@ -709,8 +677,6 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	}
 	OZ_HIP(hipMalloc(&p->mem2, L2.top));
 	char *M2 = p->mem2;
-	const LevelBin *dBins = (const LevelBin *)(M2 + binsOff);
-	const int2 *dPairs = (const int2 *)(M2 + pairsOff);
 	p->dRcAll = (const ResConst *)(M2 + rcAllOff);
 	OZ_HIP(hipMemcpyAsync(M2 + rcAllOff, &res_const_host(kResMaxMod), sizeof(ResConst), hipMemcpyHostToDevice, st));
 	for (int nm : usedNmod) {
@@ -754,21 +720,22 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 				g.R = (uint8_t *)(M2 + h.R);
 				g.ldt = h.ldt;
 				g.tstride = h.tstride;
-				g.bins = dBins + h.bin0[c];
-				g.pairs = dPairs;
 				g.tilesM = (m[q] + TB - 1) / TB;
 				g.nmod = h.nmod;
 				const int pi = (int)hProb[c].size();
 				hProb[c].push_back(g);
 				const int tiles = g.tilesM * ((n[q] + TB - 1) / TB);
-				for (int bi = 0; bi < h.nbins[c]; bi++) {
-					const LevelBin &bn = hBins[h.bin0[c] + bi];
-					const double cost = (double)bn.npairs * (bn.k1 - bn.k0);
-					for (int t = 0; t < tiles; t++) {
-						hItems[c].push_back(GItem{pi, bi, t, 0});
-						itemCost[c].push_back(cost);
+				// 128 x 128 tiles: one item streams every modulus of a tile and chunk through one
+				// pipeline; 256 x 256 tiles: one modulus per item
+				for (int ch = 0; ch < h.nchunk; ch++)
+					for (int t = 0; t < (c == 0 ? 1 : h.nmod); t++) {
+						const double cost = (double)(c == 0 ? h.nmod : 1) *
+						                    (double)std::min<int64_t>(kResChunk, h.ldp - (int64_t)ch * kResChunk);
+						for (int i = 0; i < tiles; i++) {
+							hItems[c].push_back(GItem{pi, t, ch, i});
+							itemCost[c].push_back(cost);
+						}
 					}
-				}
 			}
 		}
 		GRec r;
@@ -848,9 +815,6 @@ static int32_t plan_build(ozblasHandle_t *oh, BatchPlan *p, int batch, const cha
 	p->dRecStart = (int *)(M2 + recStartOff);
 	p->nCheck = (int)hCheck.size();
 	p->dCheck = (GCheck *)(M2 + checkOff);
-	if (!hBins.empty())
-		OZ_HIP(hipMemcpyAsync(M2 + binsOff, hBins.data(), sizeof(LevelBin) * hBins.size(), hipMemcpyHostToDevice, st));
-	OZ_HIP(hipMemcpyAsync(M2 + pairsOff, hPairs.data(), sizeof(int2) * hPairs.size(), hipMemcpyHostToDevice, st));
 	if (p->nWrite > 0) {
 		OZ_HIP(hipMemcpyAsync(p->dWrite, hWrite.data(), sizeof(GWrite) * hWrite.size(), hipMemcpyHostToDevice, st));
 		OZ_HIP(hipMemcpyAsync(p->dWriteStart, writeStart.data(), 4 * writeStart.size(), hipMemcpyHostToDevice, st));
