@@ -296,7 +296,9 @@ def bench_batched(count, torch, oz):
            "grouped_mfma_tops": round(H.n_comp / H.t_comp / 1e12, 1) if H.t_comp > 0 else None}
     # the same problems one plain-form (FP64 slices, NearSum) ozblasDgemm at a time: the bits the
     # batch must reproduce
-    Hs = oz.Handle(8 << 30, sumMode=1, sliceType="fp64")
+    # a slice limit beyond the count keeps the products of FP64 slices (without one the plain form may take its
+    # bits from residues): an independent check
+    Hs = oz.Handle(8 << 30, sumMode=1, sliceType="fp64", nSplitMax=30)
     Cl = [torch.zeros_like(c) for c in Cs]
     for rep in range(2):
         torch.cuda.synchronize()
@@ -364,7 +366,8 @@ def main():
                                                       steps, args.warmup, torch)
         if args.fp64_steps > 0:
             dC = torch.zeros(n * n, dtype=torch.float64, device="cuda:0")
-            H64 = ozblas_amd.Handle(work, sumMode=1, reproMode=1, sliceType="fp64")
+            # products of FP64 slices, as in the batched check
+            H64 = ozblas_amd.Handle(work, sumMode=1, reproMode=1, sliceType="fp64", nSplitMax=30)
             t_64, tk_64, info_64 = timed_gemm(H64, n, dA, dB, dC, args.fp64_steps, 1, torch)
             H64.close()
             same = eq(C_fast, dC)

@@ -20,13 +20,8 @@ void launch_transpose(hipStream_t st, int rows, int cols, const double *in, int6
                       double *out, int64_t ldo);
 void launch_transpose(hipStream_t st, int rows, int cols, const float *in, int64_t ldi, float *out,
                       int64_t ldo);
-void launch_vec_max(hipStream_t st, int m, const double *x, unsigned long long *slot);
-void launch_split_vec_pass(hipStream_t st, int m, const double *src, double *rem, double *slice,
-                           int rho, int shift, const uint16_t *J, const unsigned long long *maxIn,
-                           unsigned long long *maxOut);
 void launch_fill(hipStream_t st, double *p, int64_t n, double v);
 void launch_fill(hipStream_t st, float *p, int64_t n, float v);
-void launch_copy(hipStream_t st, const double *src, double *dst, int64_t n);
 // mixed = 1: the rho of the mixed split (binary64 data into binary32 slices, or binary32 data
 // into binary64 slices)
 void launch_split_csr(hipStream_t st, int m, int nnz, const double *val, const int *rowptr, double *work,

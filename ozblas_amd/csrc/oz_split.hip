@@ -167,54 +167,11 @@ __global__ __launch_bounds__(256) void k_transpose(int rows, int cols, const T *
 	}
 }
 
-// ---------------------------------------------------------------------------------------------
-// vectors: one tau for the whole vector (ozblasSplitVecKernel, src/cpu/ozblas_split.cpp:75-104)
-// ---------------------------------------------------------------------------------------------
-__device__ inline double u2d(unsigned long long u) { return __builtin_bit_cast(double, u); }
-
-template <int BS>
-__global__ __launch_bounds__(BS) void k_vec_max(int m, const double *x, unsigned long long *slot) {
-	__shared__ double red[BS / 64];
-	double mx = 0.0;
-	for (int i = blockIdx.x * BS + threadIdx.x; i < m; i += gridDim.x * BS)
-		mx = std_max(mx, fabs(x[i]));
-	mx = block_max<BS>(mx, red);
-	if (threadIdx.x == 0) atomicMax(slot, (unsigned long long)d2u(mx));
-}
-
-template <int BS>
-__global__ __launch_bounds__(BS) void k_split_vec_pass(int m, const double *src, double *rem,
-                                                       double *slice, int rho, int shift,
-                                                       const uint16_t *J,
-                                                       const unsigned long long *maxIn,
-                                                       unsigned long long *maxOut) {
-	__shared__ double red[BS / 64];
-	const int tau = tau_of(u2d(*maxIn), J);
-	const double sigma = split_sigma(rho, tau, shift);
-	double lm = 0.0;
-	for (int i = blockIdx.x * BS + threadIdx.x; i < m; i += gridDim.x * BS) {
-		const double v = src[i];
-		const double a = (v + sigma) - sigma;
-		const double rr = v - a;
-		slice[i] = a;
-		rem[i] = rr;
-		lm = std_max(lm, fabs(rr));
-	}
-	lm = block_max<BS>(lm, red);
-	if (threadIdx.x == 0) atomicMax(maxOut, (unsigned long long)d2u(lm));
-}
-
 template <class T>
 __global__ void k_fill(T *p, int64_t n, T v) {
 	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
 	     i += (int64_t)gridDim.x * blockDim.x)
 		p[i] = v;
-}
-
-__global__ void k_copy(const double *src, double *dst, int64_t n) {
-	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-	     i += (int64_t)gridDim.x * blockDim.x)
-		dst[i] = src[i];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -457,23 +414,6 @@ void launch_transpose(hipStream_t st, int rows, int cols, const float *in, int64
 	                   rows, cols, in, ldi, out, ldo);
 }
 
-void launch_vec_max(hipStream_t st, int m, const double *x, unsigned long long *slot) {
-	int grid = (m + 255) / 256;
-	if (grid > 1024) grid = 1024;
-	if (grid < 1) grid = 1;
-	hipLaunchKernelGGL(k_vec_max<256>, dim3(grid), dim3(256), 0, st, m, x, slot);
-}
-
-void launch_split_vec_pass(hipStream_t st, int m, const double *src, double *rem, double *slice,
-                           int rho, int shift, const uint16_t *J, const unsigned long long *maxIn,
-                           unsigned long long *maxOut) {
-	int grid = (m + 255) / 256;
-	if (grid > 1024) grid = 1024;
-	if (grid < 1) grid = 1;
-	hipLaunchKernelGGL(k_split_vec_pass<256>, dim3(grid), dim3(256), 0, st, m, src, rem, slice,
-	                   rho, shift, J, maxIn, maxOut);
-}
-
 void launch_fill(hipStream_t st, double *p, int64_t n, double v) {
 	if (n <= 0) return;
 	int64_t g = (n + 255) / 256;
@@ -486,13 +426,6 @@ void launch_fill(hipStream_t st, float *p, int64_t n, float v) {
 	int64_t g = (n + 255) / 256;
 	if (g > 4096) g = 4096;
 	hipLaunchKernelGGL(k_fill<float>, dim3((unsigned)g), dim3(256), 0, st, p, n, v);
-}
-
-void launch_copy(hipStream_t st, const double *src, double *dst, int64_t n) {
-	if (n <= 0) return;
-	int64_t g = (n + 255) / 256;
-	if (g > 4096) g = 4096;
-	hipLaunchKernelGGL(k_copy, dim3((unsigned)g), dim3(256), 0, st, src, dst, n);
 }
 
 template <class TI>

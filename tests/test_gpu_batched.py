@@ -178,3 +178,26 @@ def test_batched_config4_full_size(oz, oracle):
         ex = oracle.exact_gemm_rn("N", "N", q["m"], q["n"], q["k"], q["A"], q["m"], q["B"], q["k"])
         got = host(dC[p]).reshape(q["n"], q["m"]).T
         assert bits_equal(got, ex), (p, first_diff(got, ex))
+
+
+@pytest.mark.parametrize("sizes", [
+    [(1, 1, 1), (5, 3, 127), (128, 128, 128), (129, 257, 300)],       # tile and stage remainders
+    [(24, 40, 66000), (3, 2, 65536), (16, 16, 65537)],                # several k chunks in an item list
+    [(700, 600, 513)] + [(64 + i, 200 - i, 20 + 31 * i) for i in range(12)],
+], ids=["remainders", "chunks", "mixed"])
+def test_grouped_items_equal_single_products(oz, oracle, sizes):
+    """The item list of the grouped products over moduli, chunks and tiles: bitwise each problem alone."""
+    rng = np.random.default_rng(len(sizes))
+    ms, ns, ks = (list(v) for v in zip(*sizes))
+    A = [dev(rng.standard_normal(m * k)) for m, n, k in sizes]
+    B = [dev(rng.standard_normal(k * n)) for m, n, k in sizes]
+    C = [dev(np.zeros(m * n)) for m, n, k in sizes]
+    one = len(sizes)
+    H = oz.Handle(1 << 30, sumMode=1, sliceType="int8")
+    for _ in range(2):  # planned, then replayed
+        say(f"grouped items {sizes}")
+        H.dgemm_batched(["N"] * one, ["N"] * one, ms, ns, ks, [1.0] * one, A, ms, B, ks, [0.0] * one, C, ms)
+        for q, (m, n, k) in enumerate(sizes):
+            want = dev(np.zeros(m * n))
+            oz.Handle(1 << 30, sumMode=1, sliceType="int8").dgemm("N", "N", m, n, k, 1.0, A[q], m, B[q], k, 0.0, want, m)
+            assert bits_equal(host(C[q]), host(want)), (sizes[q], first_diff(host(C[q]), host(want)))
