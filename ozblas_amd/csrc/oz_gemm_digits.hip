@@ -53,7 +53,8 @@ __device__ inline void store_stage(const Stage &s, char *sA, char *sB) {
 //   (r / 16) * 16 * ldp + (q / 64) * 1024 + (r % 16) * 64 + q % 64,
 // so the 16 rows x 64 bytes a wave loads with one instruction are one contiguous KiB.  Rows are
 // padded to a multiple of 256 and k to a multiple of 128 with zero digits: the kernel has no
-// bounds checks.
+// bounds checks.  (Residue planes hold anything in the 16-row blocks beyond the operand: those rows only enter
+// product elements that nothing reads.)
 //
 // Workgroup = 2 x 2 waves; wave tile = TM x TN MFMA tiles of 32 x 32 (block tile 64TM x 64TN).
 // A stage is 128 k-bytes (4 MFMA k-steps); two LDS stages.  Per stage: the next stage's global

@@ -1829,8 +1829,9 @@ bool launch_gemv_slices(hipStream_t st, int M, int K, const double *As, int64_t 
 // LDS, and only the next level's remainder maximum goes through a workgroup barrier.  The next row's
 // elements load while this one is split.  The slices of A are never stored, the matrix is read once.  Slots
 // not reached are zero.  P[(i kSgNAM + slot) NBM + b]: the pair values of row i.
-// One workgroup of 512 with 16 elements a thread whatever K, all five values of a level reduced by
-// shuffles: 400 us for 8192 x 8192 (1.3 TB/s); with four sums by lane exchanges and the next row loading meanwhile: 240 us (2.2 TB/s, bound by FP64 arithmetic and the barrier of each level), and no count pass before it (130 us).
+// One workgroup of 512 with 16 elements a thread whatever K, all five values of a level reduced by shuffles:
+// 400 us for 8192 x 8192 (1.3 TB/s), and 130 us of a counting pass before it.  With four sums by lane exchanges and
+// the next row loading meanwhile: 240 us (2.2 TB/s, bound by FP64 arithmetic and the barrier of each level).
 // ---------------------------------------------------------------------------------------------
 constexpr int kSgNAM = 8, kSgNBM = 4;
 template <int BS, int R>

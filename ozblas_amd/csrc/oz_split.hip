@@ -8,7 +8,7 @@
 // Because tau is per column (dense) or per row (CSR), one workgroup (dense) or one thread (CSR)
 // runs every slice of its column/row in a single launch; the global slice count (the reference
 // loops until the sum of all column maxima is zero) is max over columns, read back once.
-// Vectors share one tau across all elements, so their split is one grid-wide pass per slice.
+// Vectors share one tau across all elements; their split is in oz_level12.hip.
 //
 // Fast forms (INT8/FP16/BF16): exact balanced radix-256 digit planes, see k_digit_*.
 #include "oz_digits.hpp"
