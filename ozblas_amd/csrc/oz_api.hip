@@ -474,11 +474,23 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		if (residue) {
 			OZ_HIP(hipEventRecord(b->ev[0], st));
 			const int32_t s = res_stats(oh, m, n, k, ain, ldai, bin, ldbi, ra, rb);
-			if (s == OZBLAS_STATUS_WORKSPACE) residue = false;
-			else OZ_TRY(s);
+			if (s == OZBLAS_STATUS_WORKSPACE) {
+				residue = false;
+				wreset(oh, base2);
+			} else {
+				OZ_TRY(s);
+			}
 		}
 	}
-	OZ_TRY(count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf));
+	int32_t counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf);
+	if (counted == OZBLAS_STATUS_WORKSPACE && residue) {
+		// a workspace that holds the counts but not the statistics beside them: the blocked FP64 products need the
+		// counts alone (count_cols has launched nothing, and the stream orders what follows behind the statistics)
+		residue = false;
+		wreset(oh, base2);
+		counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf);
+	}
+	OZ_TRY(counted);
 	if (residue) res_stats_read(oh, ra, rb);
 	const int nAf = nf[0], nBf = nf[1], zAf = zf[0], zBf = zf[1];
 	auto need = [&](int64_t mb, int64_t nb) -> uint64_t {
