@@ -147,11 +147,11 @@ static int32_t dense_split(ozblasHandle_t *oh, int k, int cols, const T *in, int
 
 // ---------------------------------------------------------------------------------------------
 // slice counts of two k-contiguous operands without storing slices (for the blocking decision), with one
-// synchronisation for both: counts and first-zero levels
+// synchronisation for both: counts and first-zero levels (known1: the second operand's level when it was met before)
 // ---------------------------------------------------------------------------------------------
 template <class T>
 static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const T *const (&in)[2],
-                          const int64_t (&ldi)[2], int (&count)[2], int (&z)[2]) {
+                          const int64_t (&ldi)[2], int (&count)[2], int (&z)[2], int known1 = -1) {
 	Backend *b = be(oh);
 	const uint64_t mark = wmark(oh);
 	const int64_t ldk = rup(k, 16);
@@ -161,7 +161,7 @@ static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const
 	int *zcol = (int *)walloc(oh, sizeof(int) * (size_t)most);
 	if (!rem || !scratch || !zcol) return OZBLAS_STATUS_WORKSPACE;
 	OZ_HIP(hipMemsetAsync(b->dCounters, 0, 2 * sizeof(int), b->stream));
-	for (int q = 0; q < 2; q++)
+	for (int q = 0; q < (known1 < 0 ? 2 : 1); q++)
 		launch_split_cols(b->stream, k, cols[q], in[q], ldi[q], rem, ldk, scratch, ldk, 0, Prec<T>::rho(oh, k),
 		                  oh->splitShift, split_cap(oh), Prec<T>::Jsplit(b), zcol, b->dCounters + q);
 	// behind the statistics of the residue form, which may be on their way too
@@ -169,7 +169,7 @@ static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const
 	OZ_HIP(hipMemcpyAsync(h, b->dCounters, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
 	OZ_TRY(sync(oh));
 	for (int q = 0; q < 2; q++) {
-		z[q] = h[q];
+		z[q] = q == 1 && known1 >= 0 ? known1 : h[q];
 		count[q] = split_count(oh, z[q]);
 	}
 	wreset(oh, mark);
@@ -428,6 +428,7 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 	}
 	// binary64 GEMV: the split of op(A) is fused into the slice products (the matrix is read once, its slices
 	// never stored, no counting pass); more slices than the kernel holds go on below
+	int zx = -1;  // x's first-zero level, if it was split here
 	if constexpr (std::is_same<T, double>::value) {
 		if (!dotPath && n == 1 && fastMode == 0 && !b->mixed && split_gemv_fits(k)) {
 			const int cap = split_cap(oh), rho = Prec<T>::rho(oh, k), rem = repro_slot(oh) ? 1 : 0;
@@ -459,6 +460,7 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 					wreset(oh, base);
 					return OZBLAS_STATUS_SUCCESS;
 				}
+				zx = out[3];
 			}
 			wreset(oh, base2);
 		}
@@ -482,13 +484,13 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 			}
 		}
 	}
-	int32_t counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf);
+	int32_t counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf, zx);
 	if (counted == OZBLAS_STATUS_WORKSPACE && residue) {
 		// a workspace that holds the counts but not the statistics beside them: the blocked FP64 products need the
 		// counts alone (count_cols has launched nothing, and the stream orders what follows behind the statistics)
 		residue = false;
 		wreset(oh, base2);
-		counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf);
+		counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf, zx);
 	}
 	OZ_TRY(counted);
 	if (residue) res_stats_read(oh, ra, rb);

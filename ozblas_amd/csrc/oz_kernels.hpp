@@ -221,7 +221,8 @@ void launch_csrmm_store(hipStream_t st, int m, const double *As, int64_t ldas, i
 // GEMV with the split of op(A) fused (binary64; rows of op(A) k-contiguous in `in`), for K that
 // split_gemv_fits: no count is known before.  x's slices (at least 4 valid, zero beyond its count) at Xs; z:
 // x's first-zero level, then the maximum of A's (zero before).  P: split_gemv_pairs_bytes(M) of scratch.
-// out (host memory): the slice counts, and out[2] = 1 when they exceed 8 x 4 -- then y is untouched.
+// out (host memory): the slice counts, out[2] = 1 when they exceed 8 x 4 -- then y is untouched -- and x's first-zero
+// level.
 bool split_gemv_fits(int K);
 size_t split_gemv_pairs_bytes(int M);
 void launch_split_gemv(hipStream_t st, int K, int M, const double *in, int64_t ldi, int rho, int shift, int cap,

@@ -1832,6 +1832,9 @@ bool launch_gemv_slices(hipStream_t st, int M, int K, const double *As, int64_t 
 // One workgroup of 512 with 16 elements a thread whatever K, all five values of a level reduced by shuffles:
 // 400 us for 8192 x 8192 (1.3 TB/s), and 130 us of a counting pass before it.  With four sums by lane exchanges and
 // the next row loading meanwhile: 240 us (2.2 TB/s, bound by FP64 arithmetic and the barrier of each level).
+// A matrix of more slices is given up at once: a row stops after kSgNAM levels, a workgroup at its own such row or at
+// the first one after another's.  Run to the end, the pass was lost to such calls: 2100 x 2100 of 17 slices 1,869 us
+// with the counts first, 2,053 with a whole pass before them, 1,877 with one given up.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSgNAM = 8, kSgNBM = 4;
 template <int BS, int R>
@@ -1839,6 +1842,7 @@ __global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *i
                                                    int cap, const uint16_t *Js, int remSlot, const double *Xs,
                                                    int64_t sX, const int *zx, double *P, int *zmax) {
 	constexpr int NW = BS / 64, NB = kSgNBM;
+	__shared__ int passed[2];
 	__shared__ double red[2][NW];
 	__shared__ double sums[2][kSgNAM][NW][NB];
 	const int l = threadIdx.x % 64, w = threadIdx.x / 64;
@@ -1891,15 +1895,21 @@ __global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *i
 		}
 	};
 	int rowPar = 0;
+	// a matrix of more slices than this kernel holds: the levels stop at the last slot, and so do the workgroups, each
+	// at its own such row or once it sees in zmax that another met one (loaded a row ahead)
+	const int levels = min(cap, kSgNAM);
+	int seen = 0;
 	if ((int)blockIdx.x < M) load(blockIdx.x);
 	for (int j = blockIdx.x; j < M; j += gridDim.x) {
 		double v[R], lm = 0.0;
+		if (threadIdx.x == 0) passed[rowPar] = seen;
 #pragma unroll
 		for (int q = 0; q < R; q++) {
 			v[q] = nx[q];
 			lm = max_abs(lm, v[q]);
 		}
 		if (j + (int)gridDim.x < M) load(j + gridDim.x);
+		if (threadIdx.x == 0) seen = __hip_atomic_load(zmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		auto reduce = [&](double a) {  // one barrier: two buffers
 			a = wave_max_nonneg_f64(a);
 			if (l == 0) red[par][w] = a;
@@ -1911,10 +1921,11 @@ __global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *i
 			return a;
 		};
 		double mx = reduce(lm);
+		if (cap > kSgNAM && passed[rowPar] >= kSgNAM) return;
 		if (prev >= 0) store(rowPar ^ 1);
 		int s = 0;
 		bool zero = false;
-		for (s = 0; s < cap; s++) {
+		for (s = 0; s < levels; s++) {
 			const double sigma = SplitRule<double>::sigma(rho, SplitRule<double>::tau(mx, Js), shift);
 			double acc[NB] = {};
 			lm = 0.0;
@@ -1926,14 +1937,18 @@ __global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *i
 #pragma unroll
 				for (int b = 0; b < NB; b++) acc[b] = fma(part, xr[b][q], acc[b]);
 			}
-			if (s < kSgNAM) reduce4(acc, rowPar, s);
+			reduce4(acc, rowPar, s);
 			mx = reduce(lm);
 			if (mx == 0.0) {
 				zero = true;
 				break;
 			}
 		}
-		const int zr = zero ? s : cap;
+		const int zr = zero ? s : levels;
+		if (zr == kSgNAM && cap > kSgNAM) {  // more slices: no use in going on
+			if (threadIdx.x == 0) atomicMax(zmax, zr);
+			return;
+		}
 		int slots = zero ? s + 1 : cap;
 		if (!zero && remSlot && cap < kSgNAM) {  // the remainder slot of reproMode 0
 			double acc[NB] = {};
@@ -1959,7 +1974,7 @@ __global__ __launch_bounds__(BS) void k_split_gemv(int K, int M, const double *i
 // y_i = fma(alpha, sum of row i's pair values, beta * y_i): 16 threads a row, the clear-cut case of NearSum
 // over their values, then one thread for the rest.  The counts come from the split kernels' first-zero
 // levels; with more slices than the kernels hold y stays untouched and out[2] = 1.  out (host memory):
-// slice counts of A and x, the flag.
+// slice counts of A and x, the flag, x's first-zero level.
 __global__ __launch_bounds__(256) void k_pairs_sum(int M, double *P, const int *z, int cap, int remSlot, int fsum,
                                                    double alpha, double beta, double *y, const uint16_t *J, int *out) {
 	constexpr int NB = kSgNBM;
@@ -1969,6 +1984,7 @@ __global__ __launch_bounds__(256) void k_pairs_sum(int M, double *P, const int *
 		out[0] = nA;
 		out[1] = nB;
 		out[2] = over ? 1 : 0;
+		out[3] = z[0];
 	}
 	if (over) return;
 	const int i = blockIdx.x * 16 + threadIdx.x / 16, t = threadIdx.x % 16;
