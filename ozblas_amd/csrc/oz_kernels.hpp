@@ -291,6 +291,9 @@ hipError_t launch_vsplit_plan(hipStream_t st, int n, const float *x, double *sli
                               int rho, int shift, int cap, int reproMode, const uint16_t *JF, int *info,
                               void *scratch, VsPre *pre, VsPlan *plan, bool statsDone,
                               CgDev *S = nullptr, int it = 0, int clkCat = -1, int parity = 0);
+// the slices of a plan that launch_vsplit_plan made (one marked bad has them already), up to its count
+void launch_vsplit_store(hipStream_t st, int n, const double *x, double *slices, int64_t lds, const VsPlan *plan);
+void launch_vsplit_store(hipStream_t st, int n, const float *x, double *slices, int64_t lds, const VsPlan *plan);
 // the plans of two vectors of one length (the DOT's x and y; each with its own slices, info,
 // zeroed scratch and plan), by the same three launches; parity as in launch_vsplit_plan, per scratch
 hipError_t launch_vsplit_plan2(hipStream_t st, int n, const double *x, const double *y, int rho, int shift,

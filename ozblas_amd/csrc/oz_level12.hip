@@ -829,14 +829,15 @@ __device__ void vsplit_fallback(int n, const TI *x, double *slices, int64_t lds,
 
 
 // slices from the plan: slice_s = cmod(x, u_{s-1}) - cmod(x, u_s), remainder slot, zero slots;
-// a plan marked bad is split by workgroup 0 with the reference loop instead
+// a plan marked bad is split by workgroup 0 with the reference loop instead (fallback; otherwise the plan's
+// own launch has stored its slices)
 template <class TI>
 __global__ __launch_bounds__(256) void k_vsplit_write(int n, const TI *x, double *slices,
                                                       int64_t lds, const VsPlan *plan, int rho,
                                                       int shift, int cap, int reproMode,
-                                                      const uint16_t *J, int *info) {
+                                                      const uint16_t *J, int *info, int fallback) {
 	if (plan->bad) {
-		if (blockIdx.x == 0) vsplit_fallback<256, TI>(n, x, slices, lds, rho, shift, cap, reproMode, J, info);
+		if (fallback && blockIdx.x == 0) vsplit_fallback<256, TI>(n, x, slices, lds, rho, shift, cap, reproMode, J, info);
 		return;
 	}
 	const int last = plan->last, count = plan->count, zero = plan->zero;
@@ -914,6 +915,11 @@ static hipError_t vsplit_plan(hipStream_t st, int n, const TI *x, double *slices
 	return hipGetLastError();
 }
 
+static int vsplit_write_grid(int n) {
+	const int g = (int)std::min<int64_t>(2048, ((int64_t)n + 255) / 256);
+	return g < 1 ? 1 : g;
+}
+
 // the plan, then the slices (slice_s = cmod(x, u_{s-1}) - cmod(x, u_s), remainder, zero slots)
 template <class TI>
 static hipError_t vsplit(hipStream_t st, int n, const TI *x, double *slices, int64_t lds, int rho,
@@ -922,11 +928,19 @@ static hipError_t vsplit(hipStream_t st, int n, const TI *x, double *slices, int
 	const hipError_t e = vsplit_plan(st, n, x, slices, lds, rho, shift, cap, reproMode, J, info, scratch,
 	                                 nullptr, plan, false, nullptr, 0, kClkNone, 0, parity);
 	if (e != hipSuccess) return e;
-	int gw = (int)std::min<int64_t>(2048, ((int64_t)n + 255) / 256);
-	if (gw < 1) gw = 1;
-	hipLaunchKernelGGL(k_vsplit_write<TI>, dim3(gw), dim3(256), 0, st, n, x, slices, lds,
-	                   (const VsPlan *)plan, rho, shift, cap, reproMode, J, info);
+	hipLaunchKernelGGL(k_vsplit_write<TI>, dim3(vsplit_write_grid(n)), dim3(256), 0, st, n, x, slices, lds,
+	                   (const VsPlan *)plan, rho, shift, cap, reproMode, J, info, 1);
 	return hipGetLastError();
+}
+
+void launch_vsplit_store(hipStream_t st, int n, const double *x, double *slices, int64_t lds, const VsPlan *plan) {
+	hipLaunchKernelGGL(k_vsplit_write<double>, dim3(vsplit_write_grid(n)), dim3(256), 0, st, n, x, slices, lds, plan, 0,
+	                   1, 0, 0, nullptr, nullptr, 0);
+}
+
+void launch_vsplit_store(hipStream_t st, int n, const float *x, double *slices, int64_t lds, const VsPlan *plan) {
+	hipLaunchKernelGGL(k_vsplit_write<float>, dim3(vsplit_write_grid(n)), dim3(256), 0, st, n, x, slices, lds, plan, 0,
+	                   1, 0, 0, nullptr, nullptr, 0);
 }
 
 hipError_t launch_vsplit(hipStream_t st, int n, const double *x, double *slices, int64_t lds, int rho,
