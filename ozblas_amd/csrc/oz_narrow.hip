@@ -145,15 +145,17 @@ __global__ __launch_bounds__(64) void k_narrow_zero(int n, TO *planes, int64_t l
 
 // t = the ordered sum of np pair products (T planes of int32; pair p's term is T_p 2^(u_a + u_b)), one
 // thread per row and four columns; then C = fma(alpha, t, beta C).  carry: the running sums (m x n,
-// pitch m) between the launches of a product whose planes do not fit at once.
+// pitch m) between the launches of a product whose planes do not fit at once.  The row blocks of four columns, then
+// the next four, on grid x: grid y ends at 65536, 262144 columns.
 // STORE (binary32): the terms replace the int32 values, for the NearSum kernels.
 template <class T, bool STORE>
 __global__ __launch_bounds__(256) void k_narrow_sum(int m, int n, int32_t *P, int64_t ldt, int64_t tstride,
                                                     const int2 *pairs, int np, const int *ueA, const int *ueB,
                                                     T *carry, int first, int last, T alpha, T beta, T *C,
                                                     int64_t ldc) {
-	const int i = blockIdx.x * 256 + threadIdx.x;
-	const int j0 = 4 * blockIdx.y;
+	const int rb = (m + 255) / 256;
+	const int i = ((int)blockIdx.x % rb) * 256 + (int)threadIdx.x;
+	const int j0 = 4 * ((int)blockIdx.x / rb);
 	if (i >= m) return;
 	const int nc = min(4, n - j0);
 	T t[4];
@@ -259,11 +261,13 @@ void launch_narrow_zero(hipStream_t st, int elem, int n, void *planes, int64_t l
 		                   ue, zcol, count);
 }
 
+static dim3 narrow_sum_grid(int m, int n) { return dim3((unsigned)((m + 255) / 256) * (unsigned)((n + 3) / 4)); }
+
 template <class T>
 static void narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride, const int2 *pairs,
                        int np, const int *ueA, const int *ueB, T *carry, int first, int last, T alpha, T beta,
                        T *C, int64_t ldc) {
-	hipLaunchKernelGGL((k_narrow_sum<T, false>), dim3((m + 255) / 256, (n + 3) / 4), dim3(256), 0, st, m, n, P, ldt,
+	hipLaunchKernelGGL((k_narrow_sum<T, false>), narrow_sum_grid(m, n), dim3(256), 0, st, m, n, P, ldt,
 	                   tstride, pairs, np, ueA, ueB, carry, first, last, alpha, beta, C, ldc);
 }
 void launch_narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride, const int2 *pairs,
@@ -278,8 +282,8 @@ void launch_narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, in
 }
 void launch_narrow_terms_f(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride,
                            const int2 *pairs, int np, const int *ueA, const int *ueB) {
-	hipLaunchKernelGGL((k_narrow_sum<float, true>), dim3((m + 255) / 256, (n + 3) / 4), dim3(256), 0, st, m, n, P,
-	                   ldt, tstride, pairs, np, ueA, ueB, (float *)nullptr, 1, 1, 1.f, 0.f, (float *)nullptr, 0);
+	hipLaunchKernelGGL((k_narrow_sum<float, true>), narrow_sum_grid(m, n), dim3(256), 0, st, m, n, P, ldt,
+	                   tstride, pairs, np, ueA, ueB, (float *)nullptr, 1, 1, 1.f, 0.f, (float *)nullptr, 0);
 }
 
 }  // namespace oz

@@ -244,17 +244,18 @@ double res_log2_product(int nmod) {
 }
 
 // INT8 tiled planes (the layout of the digit planes): one 256-thread workgroup writes 16 columns x
-// 64 k-bytes of every modulus plane per step (4 bytes per thread), looping over k tiles.
+// 64 k-bytes of every modulus plane per step (4 bytes per thread), looping over k tiles.  gx workgroups a column
+// block, one after the other on grid x (2^31 - 1 workgroups; y holds 65536, a million columns).
 __global__ __launch_bounds__(256) void k_res_write_i8t(int m, int n, const double *in, int64_t ldi,
                                                        const int *colLo, const ResConst *rc, int nmod,
                                                        int shLimit, int scaleU, int8_t *planes,
-                                                       int64_t ldp, int64_t pstride) {
+                                                       int64_t ldp, int64_t pstride, int gx) {
 	__shared__ ResLds T;
 	res_lds_load(T, rc, nmod, shLimit, scaleU);
 	__syncthreads();
-	const int ktiles = (int)(ldp / 64);
-	for (int kt = blockIdx.x; kt < ktiles; kt += gridDim.x)
-		res_write_tile_i8(m, n, in, ldi, colLo, nmod, T, planes, ldp, pstride, kt, blockIdx.y);
+	const int ktiles = (int)(ldp / 64), jb = (int)blockIdx.x / gx;
+	for (int kt = (int)blockIdx.x % gx; kt < ktiles; kt += gx)
+		res_write_tile_i8(m, n, in, ldi, colLo, nmod, T, planes, ldp, pstride, kt, jb);
 }
 
 // 2-byte planes (FP16 / BF16): plane s of column j at planes + s*pstride + j*ldp, rows [m, ldp) zero;
@@ -290,9 +291,9 @@ void launch_res_write(hipStream_t st, int elem, int m, int n, const double *in, 
 	if (elem == 1) {  // tiled layout; ldp % 128 == 0 and pstride = ldp * (n rounded up to 256)
 		const int ktiles = (int)(ldp / 64);
 		const int gx = ktiles < 16 ? ktiles : 16;
-		hipLaunchKernelGGL(k_res_write_i8t, dim3((unsigned)gx, (unsigned)((n + 15) / 16)), dim3(256),
+		hipLaunchKernelGGL(k_res_write_i8t, dim3((unsigned)gx * (unsigned)((n + 15) / 16)), dim3(256),
 		                   res_lds_bytes(nmod, shLimit), st, m, n, in, ldi, colLo, rc, nmod, shLimit, scaleU,
-		                   (int8_t *)planes, ldp, pstride);
+		                   (int8_t *)planes, ldp, pstride, gx);
 		return;
 	}
 	const int g = n < 2048 ? n : 2048;
