@@ -147,7 +147,9 @@ __global__ __launch_bounds__(64) void k_narrow_zero(int n, TO *planes, int64_t l
 // thread per row and four columns; then C = fma(alpha, t, beta C).  carry: the running sums (m x n,
 // pitch m) between the launches of a product whose planes do not fit at once.  The row blocks of four columns, then
 // the next four, on grid x: grid y ends at 65536, 262144 columns.
-// STORE (binary32): the terms replace the int32 values, for the NearSum kernels.
+// STORE (binary32): the terms replace the int32 values, for the NearSum kernels; eight pairs a workgroup (grid y), as
+// nothing orders them (one workgroup for all pairs waited for memory eight at a time: 64 pairs of 16 x 16 39 us, 8 so).
+constexpr int kNarrowStep = 8;  // pairs whose loads are issued before their terms are used
 template <class T, bool STORE>
 __global__ __launch_bounds__(256) void k_narrow_sum(int m, int n, int32_t *P, int64_t ldt, int64_t tstride,
                                                     const int2 *pairs, int np, const int *ueA, const int *ueB,
@@ -162,9 +164,9 @@ __global__ __launch_bounds__(256) void k_narrow_sum(int m, int n, int32_t *P, in
 #pragma unroll
 	for (int c = 0; c < 4; c++) t[c] = (!STORE && !first && c < nc) ? carry[(int64_t)(j0 + c) * m + i] : (T)0;
 	int32_t *p0 = P + (int64_t)j0 * ldt + i;
-	// eight pairs' loads are issued before their terms enter the sums
-	constexpr int U = 8;
-	for (int pb = 0; pb < np; pb += U) {
+	constexpr int U = kNarrowStep;
+	const int p1 = STORE ? min(np, U * ((int)blockIdx.y + 1)) : np;
+	for (int pb = STORE ? U * (int)blockIdx.y : 0; pb < p1; pb += U) {
 		int32_t v[U][4];
 		int e[U][4];
 #pragma unroll
@@ -282,7 +284,9 @@ void launch_narrow_sum(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, in
 }
 void launch_narrow_terms_f(hipStream_t st, int m, int n, int32_t *P, int64_t ldt, int64_t tstride,
                            const int2 *pairs, int np, const int *ueA, const int *ueB) {
-	hipLaunchKernelGGL((k_narrow_sum<float, true>), narrow_sum_grid(m, n), dim3(256), 0, st, m, n, P, ldt,
+	dim3 g = narrow_sum_grid(m, n);
+	g.y = (np + kNarrowStep - 1) / kNarrowStep;
+	hipLaunchKernelGGL((k_narrow_sum<float, true>), g, dim3(256), 0, st, m, n, P, ldt,
 	                   tstride, pairs, np, ueA, ueB, (float *)nullptr, 1, 1, 1.f, 0.f, (float *)nullptr, 0);
 }
 
