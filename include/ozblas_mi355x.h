@@ -101,10 +101,10 @@ typedef struct ozblasHandle {
 	float nSplitC;
 	float t_SplitA;
 	float t_SplitB;
-	float t_comp;
+	float t_comp; /* seconds of the products */
 	float t_sum;
 	float t_total;
-	float n_comp;
+	float n_comp; /* operations of the products that ran in t_comp: 2 m n k of each */
 	int32_t mbk;
 	int32_t nbk;
 

@@ -378,8 +378,7 @@ static int32_t gemm_plain_residue(ozblasHandle_t *oh, int m, int n, int k, doubl
 	oh->nSplitA = (float)nA;
 	oh->nSplitB = (float)nB;
 	oh->nSplitC = (float)nA * (float)nB;
-	oh->n_comp = (float)(2.0 * m * n * (double)k * oh->nSplitC);
-	return OZBLAS_STATUS_SUCCESS;
+	return OZBLAS_STATUS_SUCCESS;  // n_comp: the operations of the products that ran, one per modulus, as t_comp
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -928,6 +927,7 @@ static int32_t gemm_residue_core(ozblasHandle_t *oh, int elem, int m, int n, int
 		OZ_HIP(hipGetLastError());
 		OZ_TRY(sync(oh));
 		oh->nSplitA = oh->nSplitB = oh->nSplitC = 0;
+		oh->t_comp = oh->t_sum = oh->n_comp = 0.f;  // no products
 		oh->schemeUsed = 2;
 		wreset(oh, base);
 		return OZBLAS_STATUS_SUCCESS;
