@@ -45,6 +45,9 @@ __device__ inline double mac_max(double a, double b) { return (a > b) ? a : b; }
 // exact and the other values are at least ~2^-31 away from an integer)
 __device__ inline int ceil_log2_int(int N) { return N <= 1 ? 0 : 32 - __builtin_clz((unsigned)(N - 1)); }
 
+// A sigma beyond the range (finite values whose maximum is within the factor 2^m of overflow) has no transform: the
+// reference's loop does not end, infinity times the shrinking factor staying infinity.  The results are NaN here, and so
+// is the sum.
 template <class V>
 __device__ inline void ns_transform(int n, V &vec, double rho, double &tau1, double &tau2,
                                     const uint16_t *J) {
@@ -65,6 +68,10 @@ __device__ inline void ns_transform(int n, V &vec, double rho, double &tau1, dou
 	// scalbn1(1., m + ceil(log2(mu))): +-inf/NaN exponents convert to INT_MIN -> sigma = 0
 	double sigma = (mu <= 1.7976931348623157e308) ? scalbn_clamped(1., (int64_t)m + ceil_log2_tab(mu, J))
 	                                              : 0.0;
+	if (sigma > 1.7976931348623157e308) {
+		tau1 = tau2 = __builtin_nan("");
+		return;
+	}
 	double t = rho;
 	const double tiny = 2.2250738585072014e-308;  // scalbn(1., emin)
 	const double fac = scalbn_clamped(1., 2 * m + 1 - 53);
@@ -188,6 +195,10 @@ __device__ inline void ns_transform_wave(int n, double &v, double rho, double &t
 	}
 	const int m = ceil_log2_int(n + 2);
 	double sigma = scalbn_clamped(1., (int64_t)m + ceil_log2_tab(mu, J));  // mu finite
+	if (sigma > 1.7976931348623157e308) {
+		tau1 = tau2 = __builtin_nan("");
+		return;
+	}
 	double t = rho;
 	const double tiny = 2.2250738585072014e-308;
 	const double fac = scalbn_clamped(1., 2 * m + 1 - 53);
@@ -266,6 +277,10 @@ __device__ inline void ns_transform_f(int n, V &vec, float rho, float &tau1, flo
 	float sigma = (mu <= 3.40282347e38f)
 	                  ? (float)scalbn_clamped(1., (int64_t)m + ceil_log2_tab_f(mu, JF2))
 	                  : 0.f;
+	if (sigma > 3.40282347e38f) {
+		tau1 = tau2 = __builtin_nanf("");
+		return;
+	}
 	float t = rho;
 	const double fac = scalbn_clamped(1., 2 * m + 1 - 24);
 	const double shrink = scalbn_clamped(1., m - 24);
