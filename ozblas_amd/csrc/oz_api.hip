@@ -176,16 +176,16 @@ static int32_t count_cols(ozblasHandle_t *oh, int k, const int (&cols)[2], const
 	return OZBLAS_STATUS_SUCCESS;
 }
 
-// Whether the residue form is the faster way to NearSum's bits: its statistics, writers and reconstruction cost
-// about 45 us more than splitting and summing a small product, while the FP64 kernel takes 0.17 us per element of k
-// for the 16 pairs of full mantissas until it fills the chip, 55 TFLOP/s from there on.  Measured by FP64 slices
-// and by residues: 128^3 88 and 108 us, 1024 x 64 x 128 110 and 118, 256^3 118 and 115, 2500 x 128 x 128 156 and
-// 136, 64 x 64 x 2500 515 and 146, 2500 x 2301 x 2700 8,480 and 730.
-static bool plain_residue_pays(double m, double n, double k, double pairs) {
-	return k >= 256 ? pairs >= 9 : pairs * m * n * k >= 4e8;
-}
-// slice pairs of full mantissas, by which that is judged before the slices are counted
-constexpr double kFullPairs = 16;
+// Whether the residue form is the faster way to NearSum's bits, before anything is known of the values: its
+// statistics, writers and reconstruction cost about 45 us more than splitting and summing a small product, while the
+// FP64 kernel takes 0.17 us per element of k for the 16 pairs of full mantissas until it fills the chip, 55 TFLOP/s
+// from there on.  Measured by FP64 slices and by residues: 128^3 88 and 108 us, 1024 x 64 x 128 104 and 118, 2 x 2 x 256
+// 112 and 97, 64^2 x 256 115 and 102, 256^3 121 and 109, 2500 x 128 x 128 (12 pairs) 115 and 132, (20 pairs) 143 and 138,
+// 700 x 700 x 60 150 and 141, 64 x 64 x 2500 515 and 146, 2500 x 2301 x 2700 8,480 and 650.
+// Once the statistics are there (30 us of a small product) the residues are taken whatever the slice counts: small
+// integers of 4 pairs, slices after the statistics and residues, 2 x 2 x 256 139 and 94 us, 256^3 133 and 96,
+// 1000^3 299 and 141.
+static bool plain_residue_pays(double m, double n, double k) { return k >= 256 || m * n * k >= 2.5e7; }
 
 // slice pairs of a GEMM in the reference's level order (src/cpu/ozblas_gemm.cpp:163-164,237-264)
 static std::vector<int2> pair_list(int nA, int nB, int fastMode) {
@@ -359,8 +359,7 @@ static int32_t gemm_plain_residue(ozblasHandle_t *oh, int m, int n, int k, doubl
                                   int nA, int nB, ResOperand &ra, ResOperand &rb, bool *handled) {
 	Backend *b = be(oh);
 	*handled = false;
-	if (!plain_residue_pays(m, n, k, (double)nA * nB) || ra.st.maxE > 900 || rb.st.maxE > 900)
-		return OZBLAS_STATUS_SUCCESS;
+	if (ra.st.maxE > 900 || rb.st.maxE > 900) return OZBLAS_STATUS_SUCCESS;
 	const uint64_t base = wmark(oh);
 	const int tiles = oh->fallbackTiles, bins = oh->nLevelBins, scheme = oh->schemeUsed;
 	const float tA = oh->t_SplitA, tB = oh->t_SplitB;
@@ -471,7 +470,7 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 	bool residue = false;  // whether the residue form may be taken: its statistics come with the counts
 	if constexpr (std::is_same<T, double>::value) {
 		residue = fastMode == 0 && oh->splitEpsMode == 0 && !fsum && !b->mixed && m > 1 && n > 1 &&
-		          oh->nSplitMax == 0 && plain_residue_pays(m, n, k, kFullPairs);
+		          oh->nSplitMax == 0 && plain_residue_pays(m, n, k);
 		if (residue) {
 			OZ_HIP(hipEventRecord(b->ev[0], st));
 			const int32_t s = res_stats(oh, m, n, k, ain, ldai, bin, ldbi, ra, rb);
