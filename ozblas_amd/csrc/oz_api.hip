@@ -268,8 +268,7 @@ static int32_t gemm_narrow(ozblasHandle_t *oh, int m, int n, int k, T alpha, con
 	if (lo < -1000 || hi > 990) return give_up();
 	const std::vector<int2> pairs = pair_list(s[0].count, s[1].count, fastMode);
 	const int np = (int)pairs.size();
-	// int32 product planes of as many pairs as fit (all of them for NearSum), at most kPlaneGroup so that
-	// a large product's planes do not take the whole workspace
+	// int32 product planes of as many pairs as the workspace holds (all of them for NearSum, or none)
 	const int64_t ldt = elem == 1 ? rup(m, 256) : rup(m, 64), tstride = ldt * (elem == 1 ? rup(n, 256) : n);
 	struct Tables {
 		LevelBin bin;

@@ -12,20 +12,7 @@ typedef int i16v __attribute__((ext_vector_type(16)));
 typedef int i4v __attribute__((ext_vector_type(4)));
 typedef long l2v __attribute__((ext_vector_type(2)));
 
-template <int BS>
-__device__ inline double block_max(double v, double *red) {
-	// wavefront max via cross-lane shuffles, then across the waves through LDS
-	for (int o = 32; o > 0; o >>= 1) v = std_max(v, __shfl_xor(v, o, 64));
-	const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-	__syncthreads();
-	if (l == 0) red[w] = v;
-	__syncthreads();
-	double r = red[0];
-	for (int i = 1; i < BS / 64; i++) r = std_max(r, red[i]);
-	return r;
-}
-
-// the same for non-negative values (never NaN), for loops of reductions whose latency counts: the wave
+// workgroup maximum of non-negative values (never NaN), for loops of reductions whose latency counts: the wave
 // part runs on the DPP network, and one barrier is enough because consecutive calls alternate between
 // the two halves of `red` (2 BS / 64 doubles; `par`, 0 at first, is the caller's)
 template <int BS>

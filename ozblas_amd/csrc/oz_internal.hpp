@@ -395,8 +395,8 @@ struct ExpStatsH {
 
 // The statistics kernel reduces into kStatSlots copies 64 bytes apart (workgroup b into slot
 // b % kStatSlots), merged on the host.  One shared copy took about 10 ns for each of its five atomics a
-// workgroup, one after the other: 120 us for 2001 columns of 3001.  With 16 copies a 2001 x 1777 x 3001 INT8 product (two such
-// operands) went from 863 to 671 us.
+// workgroup, one after the other: 120 us for 2001 columns of 3001.  With 16 copies a 2001 x 1777 x 3001 INT8 product
+// (two such operands) went from 863 to 671 us.
 constexpr int kStatSlots = 16;
 struct alignas(64) ExpStatsSlot {
 	ExpStatsH s;

@@ -473,9 +473,9 @@ __device__ void vs_walk(int nwg, unsigned long long *Fg, const int2 *range, int 
 // aside) -- the case for all but the last level of vectors of varied mantissas.  The reductions
 // max |x| and the lowest non-trivial unit exponent min lo (k_vsplit_pre, or the kernel that produced
 // x) fix k_0 and the last level that can be non-zero; k_vsplit_levels evaluates F at
-// k_s = k_0 - d s for those levels (plus the zero one), and k_vsplit_verify walks the chain with
-// the exact tau rule, keeping the plan when every k_s it meets is the predicted one.  Otherwise it
-// sets plan->needScan and the table scan (gated on it) and its walk make the plan.  The F values are
+// k_s = k_0 - d s for those levels (plus the zero one), and every workgroup of k_vsplit_scan walks the chain
+// with the exact tau rule (vs_verify), keeping the plan when every k_s it meets is the predicted one.  Otherwise
+// plan->needScan is set, and the table scan and its walk make the plan.  The F values are
 // exact maxima either way, so the plan -- and every slice -- is the same.
 
 // category clock of the device CG: the first workgroup of a category's first kernel charges the
@@ -604,8 +604,9 @@ __global__ __launch_bounds__(BS) void k_vsplit_pre(int n, const TI *x, VsPre *pr
 	vs_stats_flush<BS>(mx, lo, bad, pre);
 }
 
-// The walk over the predicted F values (the steps of vs_walk), by one thread of k_vsplit_verify.  Anything the prediction does not settle (an input outside the
-// model, a zero vector, a level off the chain) goes to the table path.
+// The walk over the predicted F values (the steps of vs_walk), by one thread of a workgroup of k_vsplit_scan.
+// Anything the prediction does not settle (an input outside the model, a zero vector, a level off the chain) goes to
+// the table path.
 template <class TI>
 __device__ int vs_verify(unsigned long long mb, int lof, int bad, const unsigned long long *Fb, int rho,
                          int cap, int reproMode, const uint16_t *J, VsPlan *plan, int *info, bool write) {
@@ -1360,14 +1361,15 @@ __device__ __forceinline__ T csrmm_row_sum(int r, const double *As, int64_t ldas
 }
 
 // ---------------------------------------------------------------------------------------------
-// The binary64 product with a row block staged in LDS: 256 consecutive rows of one workgroup own one
+// The product (binary64 and binary32) with a row block staged in LDS: 256 consecutive rows of one workgroup own one
 // contiguous range of nonzeros, which all threads load in order -- the slices of A, the column index, and
 // with it the element of x -- into LDS; a thread then walks its row there, generating the slices of x
 // from the plan.  Read row by row from memory, neighbouring lanes are a row apart (7 nonzeros of a
 // stencil), so every cache line was fetched by seven instructions, and each row's chain of column index
 // and gather was a memory latency of its own: 59 us for the 100^3 Laplacian with 2 slices of A and 4 of x
-// at 426 VALU instructions a wave.  A longer range passes through the stage in parts.  Workgroups of one XCD (consecutive ones go to the 8 XCDs in turn) take one contiguous
-// eighth of the rows, so that an L2 holds the part of x its rows gather.
+// at 426 VALU instructions a wave; staged 41 us.  A longer range passes through the stage in parts.  Workgroups of one
+// XCD (consecutive ones go to the 8 XCDs in turn) take one contiguous eighth of the rows, so that an L2 holds the part
+// of x its rows gather.
 // ---------------------------------------------------------------------------------------------
 constexpr int kCsrRows = 256;
 template <int NAM, class T>
@@ -2612,7 +2614,7 @@ __device__ __forceinline__ void wave_reduce_pairs(double (&v)[NV], double *out) 
 // in registers from the plans, and all pair products accumulate in registers.  Each workgroup
 // stores its pair partials to part[p * kDotMaxWG + blockIdx.x] -- no atomics on a few shared
 // addresses -- and k_dots_fin sums them (integer multiples of the product unit below 2^53: any
-// order is exact).  Larger counts take dots_general.
+// order is exact).  Larger counts take dots_mfma up to 32 x 32, and dots_general beyond or outside dots_wide.
 // The whole of k_dots_reg for two plans of at most N slices whose slots need no masking: the slots past
 // the count are zero by themselves, because the chain ended in zero or the remainder's slot is counted.
 // Without the masks and the per-row guards an element is 6 N + N^2 instructions; with them the compiler
@@ -2884,8 +2886,9 @@ void launch_dots_dev(hipStream_t st, int n, VsRef X, VsRef Y, double *vals, doub
 // level by level (ozblasSplitVecKernel, src/cpu/ozblas_split.cpp:75-104; x and y in one reduction round
 // a level), the slices again from the sigmas, all pair products, and the sum of dots_finish.  What
 // bounds a short DOT is launches: the general path's seven (fill, statistics, levels, scan, products,
-// completion, copy back) took 47 us at n = 1003.  Beyond kDotSmallMax elements one workgroup's
-// arithmetic costs more than the launches do.
+// completion, copy back) took 47 us at n = 1003, this 22.  Beyond kDotSmallMax elements one workgroup's
+// arithmetic costs more than the launches do.  A vector of more than 8 slices is left to the general path, at the cost
+// of this pass and its wait: binary32, 8000 elements of 12 slices 77 us and 20000 of 14, without it, 56.
 // ---------------------------------------------------------------------------------------------
 template <int BS, int E, class TI>
 __global__ __launch_bounds__(BS) void k_dot_small(int n, const TI *x, const TI *y, int rho, int shift, int cap,

@@ -50,9 +50,9 @@ __device__ inline void narrow_max(int *p, int v) {
 
 // The split of k_split_cols_reg (same operations in the same order, column in registers) with the
 // slices stored as their integers q.  NT threads take one column: a wave for columns of up to 512 (no
-// barrier), a workgroup beyond (1100 columns of 1200, one wave each: 43 us; 256
-// threads each 37 us, with the reductions on the DPP network and the maxima a cache line apart 16 us).  Each thread holds R4 groups of four consecutive elements, so a plane
-// is written in words.  ue[s cols + j] = u of slice s; a level past the column's last non-zero
+// barrier), a workgroup beyond (1100 columns of 1200, one wave each: 43 us; 256 threads each 37 us, with the
+// reductions on the DPP network and the maxima a cache line apart 16 us).  Each thread holds R4 groups of four
+// consecutive elements, so a plane is written in words.  ue[s cols + j] = u of slice s; a level past the column's last non-zero
 // remainder is not written here (k_narrow_zero).  stat: kNarrowSlots copies of four maxima from zero:
 // first zero level, 1 for a column outside the integer model, kNarrowOff - min u, kNarrowOff + max u.
 template <int NT, int R4, class TI, class TO>
