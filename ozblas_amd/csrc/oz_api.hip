@@ -627,8 +627,10 @@ static int32_t digit_split(ozblasHandle_t *oh, int elem, int k, int cols, const 
                            int64_t ldi, DigitOperand &d) {
 	Backend *b = be(oh);
 	d.colE = (int *)walloc(oh, sizeof(int) * (size_t)cols * 2);
-	ExpStatsSlot *dst = (ExpStatsSlot *)walloc(oh, kStatBytes);
-	if (!d.colE || !dst) return OZBLAS_STATUS_WORKSPACE;
+	// the statistics of one operand in the handle's counters: they take nothing from the workspace
+	static_assert(kStatBytes <= sizeof(int32_t) * kCounters);
+	ExpStatsSlot *dst = (ExpStatsSlot *)b->dCounters;
+	if (!d.colE) return OZBLAS_STATUS_WORKSPACE;
 	launch_stats_init(b->stream, dst, kStatSlots);
 	launch_digit_stats(b->stream, k, cols, in, ldi, d.colE, d.colE + cols, dst);
 	OZ_HIP(hipMemcpyAsync(b->hPinned, dst, kStatBytes, hipMemcpyDeviceToHost, b->stream));

@@ -176,7 +176,7 @@ extern "C" int32_t ozblasCreate(ozblasHandle_t *oh, uint64_t workSizeBytes) {
 	OZ_HIP(hipMemcpy(b->dTauF2, tau_table_host_f2(), sizeof(uint16_t) * kTauBinadesF,
 	                 hipMemcpyHostToDevice));
 	OZ_HIP(hipHostMalloc(&b->hPinned, kPinnedBytes, hipHostMallocDefault));
-	OZ_HIP(hipMalloc(&b->dCounters, 256 * sizeof(int32_t)));
+	OZ_HIP(hipMalloc(&b->dCounters, kCounters * sizeof(int32_t)));
 	OZ_HIP(hipMalloc((void **)&b->vz, vz_bytes()));
 	for (auto &e : b->ev) OZ_HIP(hipEventCreate(&e));
 	b->scratch = static_scratch(b->device);  // with the handle's device current

@@ -37,6 +37,7 @@ struct Status {
 	} while (0)
 
 constexpr uint64_t kPinnedBytes = 4096;
+constexpr int kCounters = 256;
 
 // Library-private state behind ozblasHandle_t::backend.
 struct Backend {
@@ -48,7 +49,7 @@ struct Backend {
 	uint64_t keep = 0;         // bytes preserved across calls (pre-split CSR matrix)
 	uint16_t *dTau = nullptr;  // device copy of the ceil(log2) table
 	int64_t *hPinned = nullptr;  // pinned host scratch (kPinnedBytes)
-	int32_t *dCounters = nullptr;  // device scratch counters (256 x 4 bytes)
+	int32_t *dCounters = nullptr;  // device scratch counters (kCounters)
 	hipEvent_t ev[8] = {};
 	void *batch = nullptr;  // cached plan of ozblasDgemmBatched (oz_batched.hip)
 	int nnzA = 0;           // nonzeros of the matrix pre-split for CG (slice pitch rup(nnz, 32))
