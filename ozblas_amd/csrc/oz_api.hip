@@ -424,13 +424,17 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		return OZBLAS_STATUS_SUCCESS;
 	}
 	// binary64 GEMV: the split of op(A) is fused into the slice products (the matrix is read once, its slices
-	// never stored, no counting pass); more slices than the kernel holds go on below
-	int zx = -1;  // x's first-zero level, if it was split here
+	// never stored, no counting pass); more slices than the kernel holds go on below, with the slices of x kept
+	// where the workspace holds them beside the rest (split again, 100 x 100 of 15 slices took 191 us, so 184)
+	int zx = -1;            // x's first-zero level, if it was split here
+	DenseSplit dx;          // and its slices
+	uint64_t base3 = base2;  // the workspace from behind them
 	if constexpr (std::is_same<T, double>::value) {
 		if (!dotPath && n == 1 && fastMode == 0 && !b->mixed && split_gemv_fits(k)) {
 			const int cap = split_cap(oh), rho = Prec<T>::rho(oh, k), rem = repro_slot(oh) ? 1 : 0;
 			constexpr int kSlots = 5;  // slots of x that are valid after its split (the kernel reads 4)
 			double *Xs = (double *)walloc(oh, 8ull * ldk * (cap + 2 > kSlots ? cap + 2 : kSlots));
+			const uint64_t behind = wmark(oh);
 			double *Pv = (double *)walloc(oh, split_gemv_pairs_bytes(m));
 			int *zcol = (int *)walloc(oh, 256);
 			if (Xs && Pv && zcol) {
@@ -458,8 +462,14 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 					return OZBLAS_STATUS_SUCCESS;
 				}
 				zx = out[3];
+				dx.slices = Xs;
+				dx.ldk = dx.sstride = ldk;
+				dx.count = split_count(oh, zx);
+				base3 = behind;
+				if (ldk > k)  // zero pad rows, as dense_split
+					OZ_HIP(hipMemset2DAsync(Xs + k, ldk * sizeof(double), 0, (ldk - k) * sizeof(double), dx.count, st));
 			}
-			wreset(oh, base2);
+			wreset(oh, base3);
 		}
 	}
 	// blocking: slice counts of the whole operands bound those of any block, so halving the
@@ -482,10 +492,12 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		}
 	}
 	int32_t counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf, zx);
-	if (counted == OZBLAS_STATUS_WORKSPACE && residue) {
-		// a workspace that holds the counts but not the statistics beside them: the blocked FP64 products need the
-		// counts alone (count_cols has launched nothing, and the stream orders what follows behind the statistics)
+	if (counted == OZBLAS_STATUS_WORKSPACE && (residue || dx.slices)) {
+		// a workspace that holds the counts but not the statistics, or x's slices, beside them: the blocked FP64
+		// products need the counts alone (count_cols has launched nothing, and the stream orders what follows)
 		residue = false;
+		dx.slices = nullptr;
+		base3 = base2;
 		wreset(oh, base2);
 		counted = count_cols<T>(oh, k, {m, n}, {ain, bin}, {ldai, ldbi}, nf, zf, zx);
 	}
@@ -501,7 +513,11 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		return bytes;
 	};
 	int mbk = m, nbk = n;
-	while (need(mbk, nbk) > b->cap - base2) {
+	if (dx.slices && need(m, n) > b->cap - base3) {
+		dx.slices = nullptr;
+		base3 = base2;
+	}
+	while (need(mbk, nbk) > b->cap - base3) {
 		if (mbk == 1 && nbk == 1) return OZBLAS_STATUS_WORKSPACE;
 		if (mbk >= nbk)
 			mbk = (mbk + 1) / 2;
@@ -528,15 +544,16 @@ static int32_t gemm_plain(ozblasHandle_t *oh, char transA, char transB, int m, i
 		const int mbk_ = imin(mbk, m - im * mbk);
 		for (int in = 0; in * nbk < n; in++) {
 			const int nbk_ = imin(nbk, n - in * nbk);
-			wreset(oh, base2);
+			wreset(oh, base3);
 			T *rem = (T *)walloc(oh, sizeof(T) * ldk * std::max(mbk_, nbk_));
 			if (!rem) return OZBLAS_STATUS_WORKSPACE;
-			DenseSplit da, db;
+			DenseSplit da, db = dx;
 			// a block that is the whole operand reuses the first-zero level of count_cols
 			OZ_TRY(dense_split(oh, k, mbk_, ain + (int64_t)im * mbk * ldai, ldai, rem, ldk, da,
 			                   mbk == m ? zAf : -1));
-			OZ_TRY(dense_split(oh, k, nbk_, bin + (int64_t)in * nbk * ldbi, ldbi, rem, ldk, db,
-			                   nbk == n ? zBf : -1));
+			if (!db.slices)
+				OZ_TRY(dense_split(oh, k, nbk_, bin + (int64_t)in * nbk * ldbi, ldbi, rem, ldk, db,
+				                   nbk == n ? zBf : -1));
 			const int nA = da.count, nB = db.count;
 			// ---- pairs (src/cpu/ozblas_gemm.cpp:163-164,237-264)
 			const int maxlevel = imax((nA - 1) + (nB - 1) - fastMode, imin(nA - 1, nB - 1));
